@@ -62,7 +62,7 @@ float float_le(double c) {
 }
 
 void derive(const fd2_params& p, GeomDev& g) {
-  std::memset(&g, 0, sizeof g);
+  g = GeomDev{};
   g.xdet = (float)p.detx;
   g.ydet = (float)p.dety;
   g.H = (float)p.detheight;
@@ -70,7 +70,6 @@ void derive(const fd2_params& p, GeomDev& g) {
   g.n1 = (float)p.detnC;
   g.n2 = (float)p.detnIC;
   g.top_absfrac = (float)p.dettop;
-  g.bulk = (float)p.detbulk;
   g.beta = (float)p.detbeta;
   g.d_min = (float)p.detdmin;
   g.d_max = (float)p.detdmax;
@@ -80,19 +79,31 @@ void derive(const fd2_params& p, GeomDev& g) {
   g.uby = (float)p.detuboundy;
   g.sensor_refl = (float)p.detsensorRefl;
   g.half_h = g.H / 2.0f;
-  g.depth20 = g.H * 0.2f;
-  g.neg_inv_bulk = g.bulk > 0.0f ? -1.0f / g.bulk : 0.0f;
+  const float bulk = (float)p.detbulk;
+  g.neg_inv_bulk = bulk > 0.0f ? -1.0f / bulk : 0.0f;
   g.ratio12 = g.n1 / g.n2;
   g.ratio21 = g.n2 / g.n1;
   g.gap_fresnel = (g.ratio12 < 1.57f) ? 0 : 1;
   g.dspan = g.d_max - g.d_min;
-  // exact float thresholds for the reference's double comparisons
-  const double eps = 8.1929093e-6;
-  g.eps_lt = float_ge(eps);
-  g.eps_gt = float_le(eps);
-  g.norm_lo = float_ge(1.0 - eps);
-  g.norm_hi = float_le(1.0 + eps);
-  g.r_nudge = float_le((double)g.R - 1e-5);
+  g.r_sq = g.R * g.R;
+  g.top20 = g.half_h - g.H * 0.2f;
+  g.den_up = 2.0f * g.top20;
+  g.den_dn = 2.0f * -g.half_h;
+  g.inv_up = 1.0f / g.den_up;
+  g.inv_dn = 1.0f / g.den_dn;
+  const bool ordinary =
+      g.R >= 0x1p-8f && g.R <= 0x1p20f && g.half_h >= 0x1p-8f && g.half_h <= 0x1p20f;
+  g.wall_max = ordinary ? 0x1p40f : NAN;
+  // out-of-column radius: the largest float whose rounded root is at most the
+  // float threshold of R - 1e-5 (none when that is negative)
+  const float r_nudge = float_le((double)g.R - 1e-5);
+  g.nudge_sq = -1.0f;
+  if (r_nudge >= 0.0f) {
+    float s = r_nudge * r_nudge;
+    while (s < INFINITY && std::sqrt(s) <= r_nudge) s = std::nextafter(s, INFINITY);
+    while (std::sqrt(s) > r_nudge) s = std::nextafter(s, -INFINITY);
+    g.nudge_sq = s;
+  }
   // cos(asin(r)) = sqrt(1 - r^2); c1 < C  <=>  c1 < float_ge(C) for float c1
   g.cos_tir_in = float_ge(std::sqrt(1.0 - (double)g.ratio21 * (double)g.ratio21));
   g.cos_tir_gap = g.ratio12 <= 1.0f

@@ -249,14 +249,15 @@ template <bool MULTI, bool REC, bool RADIAL>
 __device__ __forceinline__ void finish_photon(const TransportArgs& a,
                                               const GeomDev* __restrict__ geoms,
                                               const fd2_event* __restrict__ events,
-                                              const Photon& p, uint32_t gi,
+                                              Photon& p, uint32_t gi,
                                               uint32_t lane_ev, uint32_t lane_k, uint32_t* s_cnt,
                                               uint32_t* s_tile, int side, int tile_area,
                                               uint32_t* run) {
   atomicAdd(&s_cnt[gi * kCounters + fate_counter(p.fate)], 1u);
-  const bool det = p.fate == kDetect || p.fate == kDetectOut;
+  const bool det = p.fate == kDetectOut;
   if (det) {
     const GeomDev& gt = geoms[MULTI ? gi : 0u];
+    detected_pixel(p, gt);
     if (p.fate == kDetect) {
       bool in_tile = false;
       if ((int)gi < a.n_tiles) {
@@ -415,6 +416,14 @@ __device__ __forceinline__ bool swap_to_backlog(uint32_t* wq, uint32_t& n_back, 
   }
   n_back += m;
   return true;
+}
+
+// The in-column pass's constants of a uniform geometry by scalar loads.
+__device__ __forceinline__ ColumnGeom load_column(
+    const __attribute__((address_space(4))) ColumnGeom* p) {
+  ColumnGeom c;
+  __builtin_memcpy(&c, p, sizeof c);
+  return c;
 }
 
 // QUEUE = false: a lane whose photon reaches the wall-Fresnel branch parks
@@ -614,7 +623,13 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     // the launch rather than spin
     bool progress = __ballot(alive && !parked) != 0ull;
     if (alive && !parked) {
-      const GeomDev& g = geoms[MULTI ? gi : 0u];
+      // One geometry: the pass's constants in one scalar load per pass.  The
+      // pointer is opaque so that they are not kept in scalar registers over
+      // the wall branch (spilled and refilled 16 at a time around every use).
+      auto one = (const __attribute__((address_space(4))) ColumnGeom*)geoms_in;
+      asm volatile("" : "+s"(one));
+      const ColumnGeom column = load_column(one);
+      const ColumnGeom& g = MULTI ? geoms[gi] : column;
       const int r = hot_step<CounterRng, false>(rng, p, g, &nosink);
       if (r == kEnded) {
         ended = true;
@@ -890,7 +905,8 @@ __global__ void __launch_bounds__(64) k_trace_ranecu(
       }
     }
     cnt[fate_counter(p.fate)]++;
-    const bool det = p.fate == kDetect || p.fate == kDetectOut;
+    const bool det = p.fate == kDetectOut;
+    if (det) detected_pixel(p, g);
     if (p.fate == kDetect) atomicAdd(&g.prf[pix_index(p.pix, g)], 1ull);
     if (det && ev.hist >= 1 && ev.hist <= g.num_hist) atomicAdd(&g.hist[ev.hist - 1], 1u);
     if (records) {
@@ -991,6 +1007,12 @@ __global__ void k_debug_math(int fn, const float* x, float* y, int64_t n) {
     case FD2_MATH_FF_SIN: r = fd2x_sin(v).hi; break;
     case FD2_MATH_FF_COS: r = fd2x_cos(v).hi; break;
     case FD2_MATH_FF_LOG: r = fd2x_log(v).hi; break;
+    case FD2_MATH_SQRT_01: r = fd2_sqrt_01(v); break;
+    case FD2_MATH_SQRT_POS: r = fd2_sqrt_pos(v); break;
+    case FD2_MATH_RECIP: r = fd2_recip(v); break;
+    case FD2_MATH_DIV: r = fd2_div(0.7310586f, v); break;
+    case FD2_MATH_SIN_QUARTERS: fd2_sincos_quarters(4.0f * v, &sn, &cs); r = sn; break;
+    case FD2_MATH_COS_QUARTERS: fd2_sincos_quarters(4.0f * v, &sn, &cs); r = cs; break;
     default: r = 0.0f; break;
   }
   y[i] = r;

@@ -21,6 +21,14 @@
  *   fd2_fresnel_r  unpolarised Fresnel reflectance from sines/cosines;
  *   fd2_sqrt_unit  sqrtf for 0 and x >= 2^-96, with fewer instructions
  *               on the GPU (hardware root plus the correctly rounded fix-up);
+ *   fd2_sincos_quarters  sin and cos of t quarter turns, 0 <= t <= 4, with
+ *               the quadrant taken from the rounding constant's low bits and
+ *               applied without branches (same bits as fd2_sincos_turns(t/4));
+ *   fd2_sqrt_01, fd2_recip, fd2_div  the correctly rounded square root,
+ *               reciprocal and quotient of operands far from the ends of the
+ *               exponent range, by one Newton step from the hardware's
+ *               estimate (P. Markstein, "Computation of elementary functions
+ *               on the IBM RISC System/6000 processor", 1990);
  *   fd2_asin / fd2_acos  |x| <= 1 (NaN outside), asin x = x + x z A(z) on
  *               |x| <= 1/2 and the half-angle identity
  *               asin x = pi/2 - 2 asin(sqrt((1-x)/2)) above.
@@ -109,6 +117,100 @@ FD2_HD void fd2_sincos_turns(float u, float* s, float* c) {
   const float k = fd2_rint(t);
   fd2_sincos_quadrant((t - k) * 1.57079637f, k, s, c);
 }
+
+/* x ^ y ^ z, and (x & m) ^ y: one v_bitop3_b32 each on gfx950 (the compiler
+ * emits two instructions for either) */
+FD2_HD unsigned int fd2_xor3(unsigned int x, unsigned int y, unsigned int z) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(x, y, z, 0x96);
+#else
+  return x ^ y ^ z;
+#endif
+}
+FD2_HD unsigned int fd2_and_xor(unsigned int x, unsigned int m, unsigned int y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(x, m, y, 0x6A);
+#else
+  return (x & m) ^ y;
+#endif
+}
+
+/* sin(pi t/2), cos(pi t/2) for 0 <= t <= 4: fd2_sincos_turns(t/4) with the
+ * quadrant q = k mod 4 read from the low mantissa bits of t + 1.5*2^23 (that
+ * sum is 0x4B400000 + k as an integer), and the swap and signs as bit
+ * operations.  As a four-way branch on q a wave ran every quadrant's code in
+ * turn. */
+FD2_HD void fd2_sincos_quarters(float t, float* s, float* c) {
+  const float big = 12582912.0f; /* 1.5 * 2^23 */
+  const float tb = t + big;
+  const float r = (t - (tb - big)) * 1.57079637f;
+  const float z = r * r;
+  float ps = fmaf(z, 2.724937303e-06f, -1.984008122e-04f);
+  ps = fmaf(z, ps, 8.333331905e-03f);
+  ps = fmaf(z, ps, -1.666666716e-01f);
+  const unsigned int sr = fd2_float_to_bits(fmaf(r * z, ps, r));
+  float qc = fmaf(z, -2.730065773e-07f, 2.480059811e-05f);
+  qc = fmaf(z, qc, -1.388888806e-03f);
+  qc = fmaf(z, qc, 4.166666791e-02f);
+  const unsigned int cr = fd2_float_to_bits(fmaf(z * z, qc, fmaf(-0.5f, z, 1.0f)));
+  const unsigned int q = fd2_float_to_bits(tb);
+  const unsigned int odd = 0u - (q & 1u); /* all ones in odd quadrants: swap */
+  const unsigned int hi = q << 30;        /* bit 31: quadrants 2, 3 */
+  *s = fd2_bits_to_float(fd2_and_xor(hi, 0x80000000u, (odd & cr) | (~odd & sr)));
+  *c = fd2_bits_to_float(fd2_and_xor(hi ^ odd, 0x80000000u, (odd & sr) | (~odd & cr)));
+}
+
+/* sqrtf(x) for x = +-0 and 2^-96 <= x <= 2^100: y = rsqrt estimate (1 ulp),
+ * g = x y, then g + (x - g^2) y/2.  Equal to the correctly rounded root for
+ * every float of that range (all mantissas of both exponent parities, at
+ * both ends and between).  6 instructions, where moving the hardware root by
+ * its neighbours' residuals (fd2_sqrt_unit) takes 9. */
+FD2_HD float fd2_sqrt_01(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float y = __builtin_amdgcn_rsqf(fmaxf(x, 0x1p-96f)); /* finite for x = 0 */
+  const float g = x * y;
+  return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+#else
+  return sqrtf(x);
+#endif
+}
+/* the same for 2^-96 <= x <= 2^100 (5 instructions) */
+FD2_HD float fd2_sqrt_pos(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+#else
+  return sqrtf(x);
+#endif
+}
+
+/* 1/b for 2^-100 <= |b| <= 2^100: one Newton step from v_rcp_f32 (1 ulp);
+ * the correctly rounded reciprocal for every float of that range */
+FD2_HD float fd2_recip(float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float y = __builtin_amdgcn_rcpf(b);
+  return fmaf(fmaf(-b, y, 1.0f), y, y);
+#else
+  return 1.0f / b;
+#endif
+}
+/* a/b from y = the correctly rounded 1/b, for a = +-0 or 2^-60 <= |a| <= 2^60
+ * and 2^-60 <= |b| <= 2^60 (no intermediate over- or underflows).  The sum
+ * q + r y (r = a - b q exactly) is within 2^-23 ulp of a/b before its
+ * rounding; every quotient of 24-bit significands that near a rounding
+ * boundary has been enumerated (oracle/check_div.c) and rounds correctly,
+ * so the result is the correctly rounded quotient. */
+FD2_HD float fd2_div_by(float a, float b, float y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float q = a * y;
+  return fmaf(fmaf(-b, q, a), y, q);
+#else
+  (void)y;
+  return a / b;
+#endif
+}
+FD2_HD float fd2_div(float a, float b) { return fd2_div_by(a, b, fd2_recip(b)); }
 
 FD2_HD float fd2_rsqrt(float x) {
   float y = fd2_bits_to_float(0x5f375a86u - (fd2_float_to_bits(x) >> 1));

@@ -140,7 +140,9 @@ def _check(rc: int, what: str) -> None:
 # fd2_debug_math function numbers (FD2_MATH_* in fd2.h)
 MATH_FN = {"sin": 0, "cos": 1, "log": 2, "asin": 3, "acos": 4, "sin_turns": 5,
            "cos_turns": 6, "rsqrt": 7, "sqrt_unit": 8, "angle_over_157": 9,
-           "acosf_libc": 10, "asinf_libc": 11, "ff_sin": 12, "ff_cos": 13, "ff_log": 14}
+           "acosf_libc": 10, "asinf_libc": 11, "ff_sin": 12, "ff_cos": 13, "ff_log": 14,
+           "sqrt_01": 15, "sqrt_pos": 16, "recip": 17, "div": 18, "sin_quarters": 19,
+           "cos_quarters": 20}
 
 
 def debug_math(fn: str, x, device: int = 0) -> np.ndarray:

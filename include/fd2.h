@@ -225,6 +225,8 @@ int fd2_debug_steps(fd2_ctx *ctx, const fd2_event *events, int64_t n,
  * same functions on the CPU by the tests.  FD2_MATH_SQRT_UNIT is defined for
  * x = +-0, x >= 2^-96, +inf and NaN; FD2_MATH_ANGLE_OVER_157 gives 1 when
  * acos x < 0 or > 1.57 (the new-column and reflection angle tests), else 0.
+ * FD2_MATH_DIV is 0.7310586f / x; FD2_MATH_SIN/COS_QUARTERS take the turn u
+ * (0 <= u <= 1).
  * The faithful arithmetic's pieces: FD2_MATH_ACOSF_LIBC / ASINF_LIBC the C
  * library's float arc functions as restated; FF_SIN / FF_COS / FF_LOG the
  * float-pair sin, cos (|x| <= 8) and log (x > 0) rounded to float. */
@@ -234,7 +236,9 @@ enum {
   FD2_MATH_RSQRT = 7, FD2_MATH_SQRT_UNIT = 8, FD2_MATH_ANGLE_OVER_157 = 9,
   FD2_MATH_ACOSF_LIBC = 10, FD2_MATH_ASINF_LIBC = 11, FD2_MATH_FF_SIN = 12,
   FD2_MATH_FF_COS = 13, FD2_MATH_FF_LOG = 14,
-  FD2_MATH_NFN = 15
+  FD2_MATH_SQRT_01 = 15, FD2_MATH_SQRT_POS = 16, FD2_MATH_RECIP = 17,
+  FD2_MATH_DIV = 18, FD2_MATH_SIN_QUARTERS = 19, FD2_MATH_COS_QUARTERS = 20,
+  FD2_MATH_NFN = 21
 };
 int fd2_debug_math(int fn, const float *x, float *y, int64_t n, int device);
 
