@@ -204,24 +204,34 @@ __device__ __forceinline__ void tally_add(T* p, T v) {
                          __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// How a photon ended; its counter is fate - 1 (kDetect: counted before the
+// pixel is known, as kDetectOut).  kGone: a step of length -99, the
+// reference's own mark of a photon lost inside dist_to_surface.
 enum Fate : int {
   kNone = 0, kDetect = 1, kDetectOut = 2, kAbsTop = 3, kAbsBulk = 4,
-  kLost = 5, kOutOfCol = 6, kTheta1 = 7,
-  kResume = 8,     // alive: reflected by the sensor, its next in-column step is due
-  kNewColumn = 9   // alive: a crosstalk's neighbour-column sample is due
-                   // (pix holds the samples rejected so far)
+  kLost = 5, kOutOfCol = 6, kTheta1 = 7, kGone = 8
 };
+static_assert(kDetectOut - 1 == FD2_C_DETECT && kAbsTop - 1 == FD2_C_ABS_TOP &&
+              kAbsBulk - 1 == FD2_C_ABS_BULK && kLost - 1 == FD2_C_LOST &&
+              kOutOfCol - 1 == FD2_C_OUTOFCOL && kTheta1 - 1 == FD2_C_THETA1 &&
+              kGone - 1 == FD2_C_REGEN, "fates in counter order");
 
 // photon state, all in registers.  The event's position and history stay
 // in the event record; the caller passes them where they are needed.
+// `st` is the photon's loop passes so far (kMaxLoops cap, 21 bits) and where
+// its next pass starts: kStResume after a reflection by the sensor (its next
+// in-column step is due), kStNewColumn when a crosstalk's neighbour-column
+// sample is due, with the samples rejected so far (<= 100) in bits 24-30.  One
+// word, so that a photon moves through the queues without packing.
+constexpr uint32_t kStLoops = 0x1fffffu, kStResume = 1u << 21, kStNewColumn = 1u << 31;
+constexpr int kStRejected = 24;
 struct Photon {
   float px, py, pz;   // position (the detection point once detected)
   float ux, uy, uz;   // direction cosines
   float nx, ny, nz;   // surface normal
   float xc, yc;       // current column axis (the event's first column at start)
-  int32_t loops;      // loop passes so far (kMaxLoops cap)
-  int fate;
-  int32_t pix;        // detected pixel as row << 16 | column (pix_index)
+  uint32_t st;
+  int fate;           // set when the photon ends
 };
 
 // A new photon of event ev at its emission point.  The first column is
@@ -234,18 +244,19 @@ __device__ __forceinline__ void start_photon(Photon& p, const fd2_event& ev) {
   p.pz = ev.z;
   p.xc = ev.x - ev.col_dx;
   p.yc = ev.y;
-  p.loops = 0;
+  p.st = 0;
   p.fate = kNone;
-  p.pix = -1;
   p.nx = p.ny = p.nz = 0.0f;
 }
 
 // Detection: pixel floor((x-lb)/pitch), inside iff lb <= x <= ub
 // (main/kernel_cuda_c_ver1_0.cu:3402-3419).  A detected photon ends with
-// fate kDetectOut; when the kernels count it, this sets its pixel (row << 16 |
-// column, sides <= FD2_MAX_PRF_SIDE) and kDetect if it lies in the image.
-__device__ __forceinline__ void detected_pixel(Photon& p, const GeomDev& g) {
-  p.pix = -1;
+// fate kDetectOut; when the kernels count it, this gives its pixel and makes
+// the fate kDetect if it lies in the image.
+struct Pixel {
+  int i, j;
+};
+__device__ __forceinline__ Pixel detected_pixel(Photon& p, const GeomDev& g) {
   const float ax = p.px - g.lbx, ay = p.py - g.lby;
   float qx, qy;
   if (g.inv_pixel != 0.0f) {
@@ -255,18 +266,16 @@ __device__ __forceinline__ void detected_pixel(Photon& p, const GeomDev& g) {
     qx = ax / (float)g.pixel;
     qy = ay / (float)g.pixel;
   }
-  int i = (int)floorf(qx);
-  int j = (int)floorf(qy);
+  const Pixel x{(int)floorf(qx), (int)floorf(qy)};
   if (p.px <= g.ubx && p.py <= g.uby && p.px >= g.lbx && p.py >= g.lby &&
-      i >= 0 && i < g.xdim && j >= 0 && j < g.ydim) {
+      x.i >= 0 && x.i < g.xdim && x.j >= 0 && x.j < g.ydim)
     p.fate = kDetect;
-    p.pix = (i << 16) | j;
-  }
+  return x;
 }
 
-// PRF index (row-major, xdim x ydim) of a detected photon's pixel
-__device__ __forceinline__ int32_t pix_index(int32_t pix, const GeomDev& g) {
-  return (pix >> 16) * g.ydim + (pix & 0xFFFF);
+// PRF index (row-major, xdim x ydim) of a pixel
+__device__ __forceinline__ int32_t pix_index(const Pixel& x, const GeomDev& g) {
+  return x.i * g.ydim + x.j;
 }
 
 // ------------------------------------------------------- vector helpers
@@ -557,11 +566,14 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
 template <class Rng, bool TRACE, class M = MathDevice>
 __device__ __forceinline__ bool isotropic(Rng& rng, Photon& p, const ColumnGeom& g,
                                           StepSink* sink) {
+  p.fate = kGone;
   const float ds = dist_to_surface<TRACE, M>(p, g, sink);
+  const bool ended = fabsf(ds - (-99.0f)) < kEpsLt;
   const bool bulk = __float_as_uint(g.neg_inv_bulk) != 0u;
+  bool absorbed = false;
   if (M::kFaithful && bulk) {  // (float)((double)(-1/mu) * log(u)), K:712
     const float da = fd2x_scaled_log(g.neg_inv_bulk, rng.u());
-    if (ds >= da && ds >= 0.0f) p.fate = kAbsBulk;
+    absorbed = ds >= da && ds >= 0.0f;
   } else if (bulk) {
     const float u = rng.u();
     // -ln u >= 1 - u, so the absorption length da = -ln(u)/bulk exceeds a
@@ -571,12 +583,13 @@ __device__ __forceinline__ bool isotropic(Rng& rng, Photon& p, const ColumnGeom&
     // is the same
     if (!(ds < ((1.0f - u) * -g.neg_inv_bulk) * 0.99999904632568359375f)) {
       const float da = g.neg_inv_bulk * fd2_log(u);
-      if (ds >= da && ds >= 0.0f) p.fate = kAbsBulk;
+      absorbed = ds >= da && ds >= 0.0f;
     }
-  } else if (ds >= 999999.0f) {
-    p.fate = kAbsBulk;
+  } else {
+    absorbed = ds >= 999999.0f;
   }
-  return p.fate == kAbsBulk || fabsf(ds - (-99.0f)) < kEpsLt;
+  if (absorbed) p.fate = kAbsBulk;
+  return ended || absorbed;
 }
 
 // detection (main/kernel_cuda_c_ver1_0.cu:3372-3427) of a photon on the
@@ -774,7 +787,7 @@ __device__ __forceinline__ bool transmit_gap(Rng& rng, Photon& p,
     return true;
   }
 top:
-  if (++p.loops > kMaxLoops) {
+  if (++p.st > (uint32_t)kMaxLoops) {
     p.fate = kLost;
     return true;
   }
@@ -895,7 +908,7 @@ __device__ __forceinline__ int prpt_loop(Rng& rng, Photon& p, const GeomDev& g, 
   }
 
 prpt:
-  if (++p.loops > kMaxLoops) {
+  if (++p.st > (uint32_t)kMaxLoops) {
     p.fate = kLost;
     return kPrEnded;
   }
@@ -1060,7 +1073,7 @@ __device__ __forceinline__ bool ba_prpt(Rng& rng, Photon& p, const GeomDev& g) {
 // Crosstalk moves the photon to a neighbour column whose orientation is
 // sampled from -d until a sample passes the angle test, at most 101 samples
 // (K:2452-2488).  A pass takes one sample: a rejected photon is left in
-// state kNewColumn with its rejected samples in pix and its next pass samples
+// state kStNewColumn with its rejected samples counted and its next pass samples
 // again instead of stepping, so its draws and arithmetic are the same, and
 // lanes that need one sample do not wait in a loop for lanes that need
 // several.  The top reflector's new direction (one lane of a wave in two
@@ -1079,25 +1092,23 @@ template <class Rng, bool TRACE, class M = MathDevice>
 __device__ __forceinline__ int hot_step(Rng& rng, Photon& p, const ColumnGeom& g,
                                         StepSink* sink) {
   bool sample = true, top = false;
-  int rejected = p.pix, result = kAlive;
-  if (p.fate != kNewColumn) {
+  int result = kAlive;
+  if ((int32_t)p.st >= 0) {  // not kStNewColumn
     // a pass resumed after a sensor reflection is the rest of the previous
     // pass: no loop count, no second sensor check
-    const bool resumed = p.fate == kResume;
-    p.fate = kNone;
-    p.loops += resumed ? 0 : 1;
-    if (p.loops > kMaxLoops && !resumed) {
+    const bool resumed = (p.st & kStResume) != 0u;
+    p.st = resumed ? p.st & kStLoops : p.st + 1u;
+    if (p.st > (uint32_t)kMaxLoops && !resumed) {
       p.fate = kLost;
       return kEnded;
     }
-    rejected = 0;
     sample = false;
     if (isotropic<Rng, TRACE, M>(rng, p, g, sink)) {
       result = kEnded;
     } else if (!resumed && fabsf(p.pz - (-g.half_h)) < kEpsLt) {
       const int d = detection<Rng, M>(rng, p, g);
       result = d == kSensorDetect ? kEnded : kAlive;
-      if (d == kSensorReflect) p.fate = kResume;
+      if (d == kSensorReflect) p.st |= kStResume;
     } else if (fabsf(p.uz) < kEpsLt) {
       result = kTrapped;
     } else if (fabsf(p.pz - g.half_h) < kEpsLt && p.uz > 0.0f) {
@@ -1153,13 +1164,12 @@ __device__ __forceinline__ int hot_step(Rng& rng, Photon& p, const ColumnGeom& g
       if (!over) {
         p.xc = p.px - g.R * nx;
         p.yc = p.py - g.R * ny;
-        p.fate = kNone;
-      } else if (rejected >= 100) {
+        p.st &= kStLoops;
+      } else if ((p.st >> kStRejected) == (kStNewColumn >> kStRejected) + 100u) {
         p.fate = kTheta1;
         result = kEnded;
       } else {
-        p.fate = kNewColumn;
-        p.pix = rejected + 1;
+        p.st = (p.st | kStNewColumn) + (1u << kStRejected);
       }
     }
   }

@@ -255,7 +255,7 @@ Launch make_launch(const fd2_ctx* c, const QueueBufs& b, const fd2_event* d_ev, 
   L.radial = d_radial != nullptr;
   const int per_cu = c->tune.waves_per_cu / (kTransportThreads / 64);
   const size_t smem = (size_t)a.n_tiles * a.tile_side * a.tile_side * sizeof(uint32_t);
-  const int occ = transport_max_blocks_per_cu(L.multi, L.record, L.radial, smem, queue);
+  const int occ = transport_max_blocks_per_cu(L.multi, L.record, L.radial, smem);
   L.blocks = c->n_cu * (per_cu < 1 ? 1 : (per_cu > occ ? occ : per_cu));
   if (queue && L.blocks * (kTransportThreads / 64) > c->max_waves)
     L.blocks = c->max_waves / (kTransportThreads / 64);
@@ -419,10 +419,10 @@ int fd2_create(const fd2_params* params, int n_geoms, int device, fd2_ctx** out)
   c->device = device;
   c->n_geoms = n_geoms;
   c->tune.chunk = 128;
-  c->tune.waves_per_cu = 20;
+  c->tune.waves_per_cu = 24;
   c->tune.lds_tile = 0;
   c->tune.park_lanes = 32;
-  c->tune.refill_lanes = 4;
+  c->tune.refill_lanes = 8;
   c->tune.wall_queue = 0;
   c->tune.max_chunks = FD2_MAX_CHUNKS;
   int rc = FD2_OK;
@@ -469,8 +469,7 @@ int fd2_create(const fd2_params* params, int n_geoms, int device, fd2_ctx** out)
     {
       int occ = 1;
       for (int v = 0; v < 5; ++v) {
-        const int o = transport_max_blocks_per_cu(v == 1 || v == 3, v == 2 || v == 3, v == 4, 0,
-                                                  true);
+        const int o = transport_max_blocks_per_cu(v == 1 || v == 3, v == 2 || v == 3, v == 4, 0);
         if (o > occ) occ = o;
       }
       c->max_waves = c->n_cu * occ * (kTransportThreads / 64);
@@ -1022,7 +1021,7 @@ int fd2_autotune(fd2_ctx* c, const fd2_event* d_events, int64_t n, int32_t repea
   // coordinate descent from the context's current shape, two sweeps over
   // chunk, waves per CU, parked lanes and LDS tile side
   static const int chunks[] = {16, 32, 64, 128, 256};
-  static const int waves[] = {12, 16, 20};
+  static const int waves[] = {16, 20, 24};
   static const int parks[] = {8, 16, 32, 48};
   static const int tiles[] = {-1, 32, 48, 64, 80};
   static const int refills[] = {1, 4, 8, 16, 32};

@@ -40,13 +40,13 @@ constexpr int kTileDefault = 0;  // no tile: the LDS holds the wall queues
 constexpr int kTileBudget = 64 * 64;   // u32 entries per block (16 KiB)
 // started photons of a wave's chunk in LDS (direction + stream words)
 constexpr int kStartWords = 7;
-// per-wave photon queues of the persistent kernel: the wall queue in LDS
-// (kWallCap slots of kWallWords words, word-major), the gap queue and the
-// backlog in HBM (slots in that order)
-constexpr int kWallCap = 64;
-constexpr int kWallWords = 16;  // the photon words of a queue entry
+// per-wave photon queues of the persistent kernel: photons waiting for the
+// wall branch and photons ready to step in LDS (at most 64, and 8 slots to
+// write before reading), the gap queue and the backlog in HBM (slots in that
+// order).  At most 64 + 64 + kGapCap photons are in flight per wave.
+constexpr int kWallSlots = 72;
 constexpr int kGapCap = 128;
-constexpr int kBackCap = 64 + kWallCap + kGapCap;
+constexpr int kBackCap = 64 + 64 + kGapCap;
 constexpr int kGapBase = 0;
 constexpr int kBackBase = kGapCap;
 constexpr int kQSlots = kGapCap + kBackCap;
@@ -100,7 +100,7 @@ hipError_t launch_fill_u64(unsigned long long* p, size_t n, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, size_t n, hipStream_t s);
 hipError_t launch_set_u32(uint32_t* p, uint32_t v, hipStream_t s);
 hipError_t launch_set_u64(unsigned long long* p, unsigned long long v, hipStream_t s);
-int transport_max_blocks_per_cu(bool multi, bool record, bool radial, size_t smem, bool queue);
+int transport_max_blocks_per_cu(bool multi, bool record, bool radial, size_t smem);
 size_t transport_static_lds();  // largest static LDS of the transport kernels
 
 }  // namespace fd2

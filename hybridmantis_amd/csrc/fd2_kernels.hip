@@ -164,26 +164,13 @@ hipError_t launch_queue_build(const QueueArgs& q, hipStream_t s) {
 
 // ------------------------------------------------------------ tallies
 
-__device__ __forceinline__ int fate_counter(int fate) {
-  switch (fate) {
-    case kDetect:
-    case kDetectOut: return FD2_C_DETECT;
-    case kAbsTop: return FD2_C_ABS_TOP;
-    case kAbsBulk: return FD2_C_ABS_BULK;
-    case kLost: return FD2_C_LOST;
-    case kOutOfCol: return FD2_C_OUTOFCOL;
-    case kTheta1: return FD2_C_THETA1;
-    default: return FD2_C_REGEN;  // unreachable for an ended photon
-  }
-}
-
 // Counter-mode initial direction of photon k: photon 0 takes the driver's
 // first direction (|2u-1| > 0.01, main/hybridMANTIS_c_ver1_0.c:257-277),
 // the others the direction algo() draws at the previous photon's end
 // (main/kernel_cuda_c_ver1_0.cu:578-602) followed by the RoughSurface draws
 // of the (never read) initial normal.
 __device__ __forceinline__ void counter_initial_dir(CounterRng& rng, Photon& p,
-                                                    uint32_t k, const GeomDev& g) {
+                                                    uint32_t k, const ColumnGeom& g) {
   if (k == 0) {
     emit_first_dir(rng, p, g);
   } else {
@@ -197,14 +184,13 @@ __device__ __forceinline__ void counter_initial_dir(CounterRng& rng, Photon& p,
 
 // ------------------------------------------------------- transport
 
-// Register budget of the transport kernel: 5 waves per SIMD (96 VGPRs).  The
-// wall branch's live set needs 114 VGPRs (66 without it), so 10 values are
-// spilled to scratch at this budget; the fifth wave still wins: 149.8 ->
-// 140.6 ms per mono25x50 launch on MI355X at 20 waves per CU (6 waves, 80
-// VGPRs and 25 spilled values, lose).  FD2_WAVES_PER_EU=0 lets the compiler
-// choose.
+// Register budget of the transport kernel: 6 waves per SIMD (80 VGPRs, 7
+// values of rare paths in scratch; without a limit the wall branch takes 92).
+// mono25x50 on MI355X at 20 and 24 waves per CU: 117.4 ms with 5 waves per
+// SIMD, 112.1 ms with 6; the LDS (26.5 KB per workgroup) holds no more.
+// FD2_WAVES_PER_EU=0 lets the compiler choose.
 #ifndef FD2_WAVES_PER_EU
-#define FD2_WAVES_PER_EU 5
+#define FD2_WAVES_PER_EU 6
 #endif
 // With several geometries per launch (the geometry table in LDS, read per
 // lane) the kernel needs more registers and keeps 4 waves per SIMD.
@@ -232,88 +218,77 @@ __device__ __forceinline__ int tile_origin(int dim, int side) {
 
 // Adds a lane's run of detections of one event to the event's history
 // count (the event's history and geometry are read here, once per run, not
-// once per detection).
+// once per detection).  `gt` is the launch's geometry unless MULTI.
 template <bool MULTI>
-__device__ __forceinline__ void flush_run(const GeomDev* __restrict__ geoms,
+__device__ __forceinline__ void flush_run(const GeomDev& gt, const GeomDev* geoms,
                                           const fd2_event* __restrict__ events, uint32_t run_ev,
                                           uint32_t run_cnt) {
   const fd2_event& ev = events[run_ev];
   const int32_t hist = ev.hist;
-  const GeomDev& g = geoms[MULTI ? ev.geom : 0u];
+  const GeomDev& g = MULTI ? geoms[ev.geom] : gt;
   if (hist >= 1 && hist <= g.num_hist) tally_add(&g.hist[hist - 1], run_cnt);
 }
 
 // Tallies of an ended photon: fate counter, PRF pixel (LDS tile or HBM),
 // per-lane run of the event's detections, radial bin, record.
 template <bool MULTI, bool REC, bool RADIAL>
-__device__ __forceinline__ void finish_photon(const TransportArgs& a,
-                                              const GeomDev* __restrict__ geoms,
-                                              const fd2_event* __restrict__ events,
-                                              Photon& p, uint32_t gi,
-                                              uint32_t lane_ev, uint32_t lane_k, uint32_t* s_cnt,
-                                              uint32_t* s_tile, int side, int tile_area,
-                                              uint32_t* run) {
-  atomicAdd(&s_cnt[gi * kCounters + fate_counter(p.fate)], 1u);
+__device__ __forceinline__ void finish_photon(const TransportArgs& a, const GeomDev& gt,
+                                              const GeomDev* geoms,
+                                              const fd2_event* __restrict__ events, Photon& p,
+                                              uint32_t gi, uint32_t lane_ev, uint32_t lane_k,
+                                              uint32_t* s_cnt, uint32_t* s_tile, uint32_t* run) {
+  atomicAdd(&s_cnt[gi * kCounters + p.fate - 1], 1u);
   const bool det = p.fate == kDetectOut;
+  Pixel x{0, 0};
   if (det) {
-    const GeomDev& gt = geoms[MULTI ? gi : 0u];
-    detected_pixel(p, gt);
+    x = detected_pixel(p, gt);
     if (p.fate == kDetect) {
       bool in_tile = false;
       if ((int)gi < a.n_tiles) {
-        const uint32_t ti = (uint32_t)((p.pix >> 16) - tile_origin(gt.xdim, side));
-        const uint32_t tj = (uint32_t)((p.pix & 0xFFFF) - tile_origin(gt.ydim, side));
+        const int side = a.tile_side;
+        const uint32_t ti = (uint32_t)(x.i - tile_origin(gt.xdim, side));
+        const uint32_t tj = (uint32_t)(x.j - tile_origin(gt.ydim, side));
         if (ti < (uint32_t)side && tj < (uint32_t)side) {
-          atomicAdd(&s_tile[gi * tile_area + ti * side + tj], 1u);
+          atomicAdd(&s_tile[(gi * side + ti) * side + tj], 1u);
           in_tile = true;
         }
       }
-      if (!in_tile) tally_add(&gt.prf[pix_index(p.pix, gt)], 1ull);
+      if (!in_tile) tally_add(&gt.prf[pix_index(x, gt)], 1ull);
     }
     if (lane_ev == run[0]) {
       ++run[1];
     } else {
-      if (run[1]) flush_run<MULTI>(geoms, events, run[0], run[1]);
+      if (run[1]) flush_run<MULTI>(gt, geoms, events, run[0], run[1]);
       run[0] = lane_ev;
       run[1] = 1;
     }
-  }
-  if (RADIAL && det) {
-    const fd2_event& ev = events[lane_ev];
-    tally_add(&a.radial[(size_t)lane_ev * FD2_RADIAL_BINS + radial_bin(p.px - ev.x, p.py - ev.y)],
-              1u);
+    if (RADIAL) {
+      const fd2_event& ev = events[lane_ev];
+      tally_add(
+          &a.radial[(size_t)lane_ev * FD2_RADIAL_BINS + radial_bin(p.px - ev.x, p.py - ev.y)], 1u);
+    }
   }
   if (REC) {
     fd2_photon rec;
-    rec.fate = p.fate;
-    rec.pix = p.fate == kDetect ? pix_index(p.pix, geoms[MULTI ? gi : 0u]) : -1;
+    rec.fate = p.fate == kGone ? kNone : p.fate;
+    rec.pix = p.fate == kDetect ? pix_index(x, gt) : -1;
     rec.x = det ? p.px : 0.0f;
     rec.y = det ? p.py : 0.0f;
     a.records[a.photon_off[lane_ev] + lane_k] = rec;
   }
 }
 
-// Per-wave photon queues in HBM (wall queue, gap queue, backlog: kQSlots
-// entries of kQWords words).  Slots come in blocks of kQBlock = 32; word j
-// of slot s is at [(s / 32) * 32 * kQWords + 32 j + s % 32], so the lanes of
-// a wave write whole 128-byte lines and all words of a slot lie within
-// 3 KB of its first (one address per lane, the rest immediate offsets).  An
-// entry is everything a photon in flight carries: position, direction,
-// column axis, loop count and flags, random stream, event, geometry and
-// photon index (not the surface normal: every path writes it before reading
-// it); gap-queue entries also the wall branch's loop state (PrptState).
-__device__ __forceinline__ size_t q_base(uint32_t slot) {
-  return (size_t)(slot / kQBlock) * (kQBlock * kQWords) + slot % kQBlock;
-}
-
-// An entry's words lie `S` words apart from its first: kQBlock in the HBM
-// queues, kWallCap in a wave's LDS wall queue (word-major, one row of
-// kWallCap slots per word).  The geometry index is stored only for several
-// geometries per launch (MULTI; else 0) and the photon index only for
-// per-photon records (REC).
-template <bool MULTI, bool REC, int S = kQBlock>
-__device__ __forceinline__ void q_put_at(uint32_t* w, const Photon& p, const CounterRng& r,
-                                         uint32_t ev, uint32_t gi, uint32_t k, bool parked) {
+// A photon's words in the LDS queue and the HBM queues: everything a photon
+// in flight carries (not the surface normal: every path writes it before
+// reading it); gap-queue entries also the wall branch's loop state
+// (PrptState).  An entry's words lie `S` words apart from its first: kQBlock
+// in the HBM queues, kWallSlots in a wave's LDS queue (word-major, one row of
+// slots per word).  The geometry index is stored only for several geometries
+// per launch (MULTI; else 0) and the photon index only for per-photon records
+// (REC).
+template <bool MULTI, bool REC, int S>
+__device__ __forceinline__ void q_put(uint32_t* w, const Photon& p, const CounterRng& r,
+                                      uint32_t ev, uint32_t gi, uint32_t k) {
   w[0 * S] = __float_as_uint(p.px);
   w[1 * S] = __float_as_uint(p.py);
   w[2 * S] = __float_as_uint(p.pz);
@@ -322,11 +297,7 @@ __device__ __forceinline__ void q_put_at(uint32_t* w, const Photon& p, const Cou
   w[5 * S] = __float_as_uint(p.uz);
   w[6 * S] = __float_as_uint(p.xc);
   w[7 * S] = __float_as_uint(p.yc);
-  // loops (21 bits) | sensor resume (bit 22) | parked | new-column sample
-  // due, with its rejected samples (<= 100) in bits 25-31
-  w[8 * S] = (uint32_t)p.loops |
-             (p.fate == kResume ? 1u << 22 : 0u) | (parked ? 1u << 23 : 0u) |
-             (p.fate == kNewColumn ? (1u << 24) | ((uint32_t)p.pix << 25) : 0u);
+  w[8 * S] = p.st;
   w[9 * S] = r.s0;
   w[10 * S] = r.s1;
   w[11 * S] = r.s2;
@@ -336,32 +307,9 @@ __device__ __forceinline__ void q_put_at(uint32_t* w, const Photon& p, const Cou
   if (REC) w[15 * S] = k;
 }
 
-template <bool MULTI, bool REC>
-__device__ __forceinline__ void q_put(uint32_t* wq, uint32_t slot, const Photon& p,
-                                      const CounterRng& r, uint32_t ev, uint32_t gi, uint32_t k,
-                                      bool parked) {
-  q_put_at<MULTI, REC>(wq + q_base(slot), p, r, ev, gi, k, parked);
-}
-
-__device__ __forceinline__ void q_put_state(uint32_t* wq, uint32_t slot, const PrptState& st) {
-  uint32_t* w = wq + q_base(slot);
-  w[16 * kQBlock] = st.tries;
-  w[17 * kQBlock] = __float_as_uint(st.pr);
-  w[18 * kQBlock] = __float_as_uint(st.s2);
-  w[19 * kQBlock] = __float_as_uint(st.c2);
-}
-
-__device__ __forceinline__ void q_get_state(const uint32_t* wq, uint32_t slot, PrptState& st) {
-  const uint32_t* w = wq + q_base(slot);
-  st.tries = w[16 * kQBlock];
-  st.pr = __uint_as_float(w[17 * kQBlock]);
-  st.s2 = __uint_as_float(w[18 * kQBlock]);
-  st.c2 = __uint_as_float(w[19 * kQBlock]);
-}
-
-template <bool MULTI, bool REC, int S = kQBlock>
-__device__ __forceinline__ void q_get_at(const uint32_t* w, Photon& p, CounterRng& r,
-                                         uint32_t& ev, uint32_t& gi, uint32_t& k, bool& parked) {
+template <bool MULTI, bool REC, int S>
+__device__ __forceinline__ void q_get(const uint32_t* w, Photon& p, CounterRng& r, uint32_t& ev,
+                                      uint32_t& gi, uint32_t& k) {
   p.px = __uint_as_float(w[0 * S]);
   p.py = __uint_as_float(w[1 * S]);
   p.pz = __uint_as_float(w[2 * S]);
@@ -371,11 +319,7 @@ __device__ __forceinline__ void q_get_at(const uint32_t* w, Photon& p, CounterRn
   p.nx = p.ny = p.nz = 0.0f;  // written before it is read
   p.xc = __uint_as_float(w[6 * S]);
   p.yc = __uint_as_float(w[7 * S]);
-  const uint32_t f = w[8 * S];
-  p.loops = (int32_t)(f & 0x1fffffu);
-  p.fate = ((f >> 22) & 1u) ? kResume : ((f >> 24) & 1u) ? kNewColumn : kNone;
-  parked = (f >> 23) & 1u;
-  p.pix = ((f >> 24) & 1u) ? (int32_t)(f >> 25) : -1;
+  p.st = w[8 * S];
   r.s0 = w[9 * S];
   r.s1 = w[10 * S];
   r.s2 = w[11 * S];
@@ -385,10 +329,27 @@ __device__ __forceinline__ void q_get_at(const uint32_t* w, Photon& p, CounterRn
   k = REC ? w[15 * S] : 0u;
 }
 
-template <bool MULTI, bool REC>
-__device__ __forceinline__ void q_get(const uint32_t* wq, uint32_t slot, Photon& p, CounterRng& r,
-                                      uint32_t& ev, uint32_t& gi, uint32_t& k, bool& parked) {
-  q_get_at<MULTI, REC>(wq + q_base(slot), p, r, ev, gi, k, parked);
+// Per-wave gap queue and backlog in HBM (kQSlots entries of kQWords words).
+// Slots come in blocks of kQBlock = 32; word j of slot s is at
+// [(s / 32) * 32 * kQWords + 32 j + s % 32], so the lanes of a wave write
+// whole 128-byte lines and all words of a slot lie within 3 KB of its first
+// (one address per lane, the rest immediate offsets).
+__device__ __forceinline__ size_t q_base(uint32_t slot) {
+  return (size_t)(slot / kQBlock) * (kQBlock * kQWords) + slot % kQBlock;
+}
+
+__device__ __forceinline__ void q_put_state(uint32_t* w, const PrptState& st) {
+  w[16 * kQBlock] = st.tries;
+  w[17 * kQBlock] = __float_as_uint(st.pr);
+  w[18 * kQBlock] = __float_as_uint(st.s2);
+  w[19 * kQBlock] = __float_as_uint(st.c2);
+}
+
+__device__ __forceinline__ void q_get_state(const uint32_t* w, PrptState& st) {
+  st.tries = w[16 * kQBlock];
+  st.pr = __uint_as_float(w[17 * kQBlock]);
+  st.s2 = __uint_as_float(w[18 * kQBlock]);
+  st.c2 = __uint_as_float(w[19 * kQBlock]);
 }
 
 // number of set bits of a wave-wide mask below this lane (v_mbcnt)
@@ -396,50 +357,60 @@ __device__ __forceinline__ uint32_t rank_below(unsigned long long mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
-
-// Moves the wave's photons in flight (stepping or waiting for the wall
-// queue) to the top of its backlog; false if the backlog would overflow,
-// which the in-flight bound rules out.
-template <bool MULTI, bool REC>
-__device__ __forceinline__ bool swap_to_backlog(uint32_t* wq, uint32_t& n_back, bool& alive,
-                                                bool& parked, const Photon& p,
-                                                const CounterRng& rng, uint32_t lane_ev,
-                                                uint32_t gi, uint32_t lane_k) {
-  const unsigned long long am = __ballot(alive);
-  const uint32_t m = (uint32_t)__popcll(am);
-  if (n_back + m > (uint32_t)kBackCap) return false;
-  if (alive) {
-    q_put<MULTI, REC>(wq, kBackBase + n_back + rank_below(am), p, rng,
-                      lane_ev, gi, lane_k, parked);
-    alive = false;
-    parked = false;
-  }
-  n_back += m;
-  return true;
+__device__ __forceinline__ uint32_t count(unsigned long long mask) {
+  return (uint32_t)__popcll(mask);
+}
+// whether this lane is in a wave-wide mask (the mask becomes the lane predicate)
+__device__ __forceinline__ bool in(unsigned long long mask) {
+  return __builtin_amdgcn_inverse_ballot_w64(mask);
 }
 
-// The in-column pass's constants of a uniform geometry by scalar loads.
-__device__ __forceinline__ ColumnGeom load_column(
-    const __attribute__((address_space(4))) ColumnGeom* p) {
-  ColumnGeom c;
-  __builtin_memcpy(&c, p, sizeof c);
+// A table entry at a wave-uniform address by scalar loads of the members that
+// are used.  The pointer is opaque: the loads stay where they are asked for,
+// instead of the values being kept in scalar registers over the whole loop
+// (spilled, and refilled 16 at a time around every use).
+template <class T>
+__device__ __forceinline__ T load_uniform(const void* p) {
+  auto one = (const __attribute__((address_space(4))) T*)p;
+  asm volatile("" : "+s"(one));
+  T c;
+  __builtin_memcpy(&c, one, sizeof c);  // typed: the alignment makes them scalar loads
   return c;
 }
 
-// QUEUE = false: a lane whose photon reaches the wall-Fresnel branch parks
-// in place and the wave runs the branch for its parked lanes once
-// park_lanes of them wait.  QUEUE = true: the photon moves to the wave's
-// wall queue in HBM and the lane takes new work; when 64 photons wait, the
-// wave moves its photons in flight to its backlog and runs the branch with
-// all 64 lanes, up to a refraction out of the column; those photons wait in
-// the gap queue and their flights through the gap run, again 64 at a time,
-// one flight per photon and pass, in a phase of their own (a photon
-// reflected off the next column's outside waits for another flight).  Free
-// lanes refill from the backlog before the work queue, so no more than
-// 64 + kWallCap + kGapCap photons are ever in flight per wave and the
-// backlog (kBackCap) cannot overflow; the gap queue holds at most 127.
-// Every photon keeps its own state and random stream, so the results are
-// the same either way.
+// Persistent transport.  A wave keeps the state of its lanes in wave-uniform
+// masks: step_m (a photon that takes in-column passes), wall_m (a photon that
+// waits for the wall's Fresnel branch), end_m (a photon that has ended and is
+// not tallied yet); the other lanes are free.  Its loop:
+//
+//   serve   once refill_lanes lanes do not step: tally the ended photons, put
+//           the waiting ones into the wave's LDS queue and fill the free lanes
+//           (LDS queue, HBM backlog, then new photons of the work queue)
+//   pass    one in-column pass of the stepping lanes
+//   wall    once 64 photons wait (in lanes and in the LDS queue): the branch
+//           runs with all 64 lanes, up to a refraction out of the column;
+//           photons that were stepping change places with queue entries, so
+//           they stay in LDS
+//   gap     the flights through the gap between columns, again 64 at a time
+//           (HBM gap queue), one flight per photon and round; photons that
+//           were stepping go to the HBM backlog meanwhile
+//
+// The LDS queue holds waiting photons from its bottom up (n_wall) and photons
+// ready to step from its top down (n_ready).  n_wall + n_ready <= 64 outside
+// of serve: a waiting photon enters from a lane that then takes a ready one,
+// and the wall phase swaps at most as many in as it takes out.  The 8 slots
+// above 64 let a lane write before it reads.  Moving the stepping photons to
+// HBM and back around every wall phase, as the gap phase still does, took
+// 1.2e11 of 1.5e11 bytes of a mono25x50 launch and a wait for HBM at each
+// refill.
+//
+// Draining (no chunk, ready photon or backlog left), and throughout when
+// there are no queues (wave_queue null), waiting photons stay in their lanes:
+// the branch and the flights run where they are, with the other lanes masked
+// off, once at least as many wait as step (without queues: park_lanes).
+//
+// Every photon keeps its own state and random stream, so the results are the
+// same in either mode and in any order.
 //
 // `geoms_in`, `events` and `chunk_off` are a.geoms, a.events and
 // a.chunk_off again, as parameters of their own: the kernel never writes
@@ -447,33 +418,32 @@ __device__ __forceinline__ ColumnGeom load_column(
 // (__restrict__) lets the compiler read them with scalar loads where they
 // are uniform instead of reloading them with vector loads around every
 // store.
-template <bool MULTI, bool REC, bool RADIAL, bool QUEUE>
+template <bool MULTI, bool REC, bool RADIAL>
 __global__ void __launch_bounds__(kTransportThreads) FD2_TRANSPORT_ATTR
 k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
             const fd2_event* __restrict__ events, const uint32_t* __restrict__ chunk_off) {
   // With several geometries a lane's geometry is its own, so their constants
-  // cannot be scalar loads: the table goes to LDS instead (160 B each).
+  // cannot be scalar loads: the table goes to LDS instead.
   static_assert(sizeof(GeomDev) % 4 == 0, "GeomDev copied as words");
-  __shared__ GeomDev s_geoms[MULTI ? FD2_MAX_GEOMS : 1];
+  __shared__ __align__(16) uint32_t s_geom_words[MULTI ? FD2_MAX_GEOMS * sizeof(GeomDev) / 4 : 2];
   if (MULTI) {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(geoms_in);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(s_geoms);
     const int nw = a.n_geoms * (int)(sizeof(GeomDev) / 4);
-    for (int i = threadIdx.x; i < nw; i += blockDim.x) dst[i] = src[i];
+    for (int i = threadIdx.x; i < nw; i += blockDim.x) s_geom_words[i] = src[i];
   }
-  const GeomDev* __restrict__ geoms = MULTI ? s_geoms : geoms_in;
+  const GeomDev* __restrict__ geoms =
+      MULTI ? reinterpret_cast<const GeomDev*>(s_geom_words) : geoms_in;
   __shared__ uint32_t s_cnt[FD2_MAX_GEOMS * kCounters];
   // the next photons of the wave's chunk, started ahead with all lanes:
   // photon start_base + j has its first direction in words 0-2 of slot j
   // and its random stream (after the initial draws) in words 3-6
   __shared__ uint32_t s_start[kTransportThreads / 64][kStartWords][64];
-  // the waves' wall queues (QUEUE): entries in the layout of q_put_at, word-major
-  __shared__ uint32_t s_wall[QUEUE ? kTransportThreads / 64 : 1][kWallWords][kWallCap];
+  // the waves' LDS queues, word-major
+  __shared__ uint32_t s_queue[kTransportThreads / 64][MULTI || REC ? 16 : 14][kWallSlots];
   extern __shared__ uint32_t s_tile[];  // n_tiles x tile_side^2
   for (int i = threadIdx.x; i < a.n_geoms * kCounters; i += blockDim.x) s_cnt[i] = 0;
-  const int side = a.tile_side;
-  const int tile_area = side * side;
-  for (int i = threadIdx.x; i < a.n_tiles * tile_area; i += blockDim.x) s_tile[i] = 0;
+  for (int i = threadIdx.x; i < a.n_tiles * a.tile_side * a.tile_side; i += blockDim.x)
+    s_tile[i] = 0;
   __syncthreads();
 
   // per-lane run of detections of one event (event, count), added to the
@@ -484,14 +454,11 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
   uint32_t* run = s_run[threadIdx.x];
   run[0] = 0u;
   run[1] = 0u;
-  const uint64_t event_base = a.event_base_dev ? *a.event_base_dev : a.event_base;
 
   const int lane = threadIdx.x & 63;
   // the wave's index in the block, uniform across the wave: the compiler
   // then keeps the wave's queue and LDS bases in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t chunk = 1u << a.chunk_log2;
-
   // wave-uniform work pool: photons [pool_next, pool_end) of event pool_ev;
   // those in [start_base, start_end) (up to 64) are started in s_start
   int64_t pool_ev = 0;
@@ -501,293 +468,353 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
 
   Photon p;
   CounterRng rng;
-  bool alive = false;
-  bool parked = false;  // waiting for the wall-Fresnel branch
+  unsigned long long step_m = 0, wall_m = 0, end_m = 0;
   uint32_t gi = 0;
   uint32_t lane_ev = 0;  // the lane's event (index into events)
   uint32_t lane_k = 0;   // photon index within the event
   StepSink nosink{nullptr, nullptr, 0, 0, false};
 
-  // wave queues (QUEUE): wall [0, n_wall) in LDS, gap [0, n_gap) and backlog
-  // [0, n_back) in HBM
-  uint32_t* wq = nullptr;
-  uint32_t* wall = &s_wall[QUEUE ? wave : 0][0][0];
-  uint32_t n_wall = 0, n_gap = 0, n_back = 0, idle = 0;
-  if (QUEUE)
+  uint32_t* lq = &s_queue[wave][0][0];
+  uint32_t* wq = nullptr;  // gap queue [0, n_gap), backlog [0, n_back)
+  uint32_t n_wall = 0, n_ready = 0, n_gap = 0, n_back = 0, idle = 0;
+  if (a.wave_queue)
     wq = a.wave_queue + (size_t)(blockIdx.x * (kTransportThreads / 64) + wave) *
                             (kQWords * kQSlots);
+  const bool queued = a.wave_queue != nullptr;
+
+  // the launch's arguments, read again where they are needed: held over the
+  // loop they would take the scalar registers of its lane masks
+  const void* kernarg = (const void*)__builtin_amdgcn_kernarg_segment_ptr();
+  auto args = [&]() { return load_uniform<TransportArgs>(kernarg); };
+  // f(the lane's geometry)
+  auto with_geom = [&](auto f) {
+    if constexpr (MULTI)
+      f(geoms[gi]);
+    else
+      f(load_uniform<GeomDev>(geoms_in));
+  };
+  auto finish = [&](unsigned long long m) {
+    if (in(m))
+      with_geom([&](const GeomDev& g) {
+        finish_photon<MULTI, REC, RADIAL>(args(), g, geoms, events, p, gi, lane_ev, lane_k, s_cnt,
+                                          s_tile, run);
+      });
+  };
+  auto lds_put = [&](uint32_t slot) {
+    q_put<MULTI, REC, kWallSlots>(lq + slot, p, rng, lane_ev, gi, lane_k);
+  };
+  auto lds_get = [&](uint32_t slot) {
+    q_get<MULTI, REC, kWallSlots>(lq + slot, p, rng, lane_ev, gi, lane_k);
+  };
+  // fills up to n_ready of the lanes in `want` from the ready photons; the
+  // barrier keeps the compiler from moving LDS accesses across (a wave's
+  // complete in order)
+  auto take_ready = [&](unsigned long long want) {
+    const uint32_t t = min(count(want), n_ready);
+    if (t == 0u) return;
+    const uint32_t rank = rank_below(want);
+    const bool got = in(want) && rank < t;
+    __builtin_amdgcn_wave_barrier();
+    if (got) lds_get((uint32_t)kWallSlots - n_ready + rank);
+    __builtin_amdgcn_wave_barrier();
+    n_ready -= t;
+    step_m |= __ballot(got);
+  };
 
   for (;;) {
-    // Starting a photon (stream seeding, first direction) is long and would
-    // run with one or two lanes if done whenever a photon ends: wait until
-    // refill_lanes lanes are free, or no lane is left to step.
-    unsigned long long need = __ballot(!alive);
-    if ((int)__popcll(need) < a.refill_lanes && need != ~0ull) need = 0ull;
-    if (QUEUE && need != 0ull && n_back != 0u) {
-      __threadfence_block();  // the wave's queue stores are complete before its loads
-      const uint32_t take = min((uint32_t)__popcll(need), n_back);
-      const uint32_t rank = rank_below(need);
-      if (!alive && rank < take) {
-        q_get<MULTI, REC>(wq, kBackBase + n_back - 1u - rank, p, rng, lane_ev, gi, lane_k, parked);
-        alive = true;
-      }
-      n_back -= take;
-      need = __ballot(!alive);
-    }
-    while (need != 0ull && !pool_done) {
-      if (pool_next >= pool_end) {
-        uint32_t c = 0;
-        if (lane == 0) c = atomicAdd(a.cursor, 1u);
-        c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
-        if (c >= chunk_off[a.n_events]) {
-          pool_done = true;
-          break;
-        }
-        // largest e with chunk_off[e] <= c (skips events without photons):
-        // each round the 64 lanes (all active here) probe 64 points of
-        // [lo, hi) with one vector load, and the wave keeps the step after
-        // the last probe at or below c -- 3 rounds for 2e5 events where a
-        // binary search makes 18 dependent loads
-        int64_t lo = 0, hi = a.n_events;
-        while (hi - lo > 1) {
-          const int64_t step = (hi - lo + 63) >> 6;
-          const int64_t pos = lo + (int64_t)lane * step;
-          const bool le = pos < hi && chunk_off[pos] <= c;
-          const unsigned long long m = __ballot(le);
-          lo += (int64_t)(63 - __clzll(m)) * step;
-          hi = min(hi, lo + step);
-        }
-        pool_ev = lo;
-        const int32_t n_ph = events[lo].N;
-        pool_next = (int32_t)((c - chunk_off[lo]) << a.chunk_log2);
-        pool_end = min(n_ph, pool_next + (int32_t)chunk);
-        if (lane == 0) {
-          const uint32_t gg = MULTI ? events[lo].geom : 0u;
-          atomicAdd(&s_cnt[gg * kCounters + FD2_C_GENERATED], (uint32_t)(pool_end - pool_next));
-        }
-        start_end = pool_next;
-      }
-      if (pool_next >= start_end) {
-        // Seeding a stream (Philox) and drawing the first direction are
-        // long; every lane starts one of the next 64 photons of the chunk
-        // here, at full width, instead of the few lanes that take photons
-        // in a pass.
-        start_base = pool_next;
-        start_end = min(pool_end, pool_next + 64);
-        if (start_base + lane < start_end) {
-          const uint32_t k = (uint32_t)(start_base + lane);
-          CounterRng r;
-          Photon q;
-          r.seed(a.seed, event_base + (uint64_t)pool_ev, k);
-          counter_initial_dir(r, q, k, geoms[MULTI ? events[pool_ev].geom : 0u]);
-          start[0][lane] = __float_as_uint(q.ux);
-          start[1][lane] = __float_as_uint(q.uy);
-          start[2][lane] = __float_as_uint(q.uz);
-          start[3][lane] = r.s0;
-          start[4][lane] = r.s1;
-          start[5][lane] = r.s2;
-          start[6][lane] = r.s3;
-        }
-        // lanes read other lanes' slots below; the wave's LDS accesses
-        // complete in order
-        __builtin_amdgcn_wave_barrier();
-      }
-      const int avail = start_end - pool_next;  // started, not yet taken
-      const int rank = (int)rank_below(need);
-      if (!alive && rank < avail) {
-        const fd2_event ev = events[pool_ev];
-        gi = MULTI ? ev.geom : 0u;
-        const uint32_t k = (uint32_t)(pool_next + rank);
-        const uint32_t j = k - (uint32_t)start_base;
-        start_photon(p, ev);
-        p.ux = __uint_as_float(start[0][j]);
-        p.uy = __uint_as_float(start[1][j]);
-        p.uz = __uint_as_float(start[2][j]);
-        rng.s0 = start[3][j];
-        rng.s1 = start[4][j];
-        rng.s2 = start[5][j];
-        rng.s3 = start[6][j];
-        lane_ev = (uint32_t)pool_ev;
-        lane_k = k;
-        parked = false;
-        alive = true;
-      }
-      pool_next += min((int)__popcll(need), avail);
-      need = __ballot(!alive);
-    }
-    // with no lane alive the work queue and the backlog are empty
-    if (__ballot(alive) == 0ull && (!QUEUE || (n_wall == 0u && n_gap == 0u))) break;
-    bool ended = false;
-    // every pass steps a photon or runs the wall branch; a wave that does
-    // neither for many passes has a broken queue state: it stops and flags
-    // the launch rather than spin
-    bool progress = __ballot(alive && !parked) != 0ull;
-    if (alive && !parked) {
-      // One geometry: the pass's constants in one scalar load per pass.  The
-      // pointer is opaque so that they are not kept in scalar registers over
-      // the wall branch (spilled and refilled 16 at a time around every use).
-      auto one = (const __attribute__((address_space(4))) ColumnGeom*)geoms_in;
-      asm volatile("" : "+s"(one));
-      const ColumnGeom column = load_column(one);
-      const ColumnGeom& g = MULTI ? geoms[gi] : column;
-      const int r = hot_step<CounterRng, false>(rng, p, g, &nosink);
-      if (r == kEnded) {
-        ended = true;
-      } else if (r == kTrapped) {
-        atomicAdd(&s_cnt[gi * kCounters + FD2_C_REGEN], 1u);
-        restart_trapped(rng, p, g, events[lane_ev]);
-      } else if (r == kNeedPrpt) {
-        parked = true;
-      }
-    }
-    if (QUEUE) {
-      if (ended) {
-        finish_photon<MULTI, REC, RADIAL>(a, geoms, events, p, gi, lane_ev, lane_k, s_cnt, s_tile, side,
-                                          tile_area, run);
-        alive = false;
-        ended = false;
-      }
-      // parked photons move to the wall queue while it has room
-      const unsigned long long pm = __ballot(alive && parked);
-      if (pm != 0ull) {
-        const uint32_t k = min((uint32_t)__popcll(pm), (uint32_t)kWallCap - n_wall);
-        const uint32_t rank = rank_below(pm);
-        if (alive && parked && rank < k) {
-          q_put_at<MULTI, REC, kWallCap>(wall + n_wall + rank, p, rng, lane_ev, gi, lane_k, false);
-          alive = false;
-          parked = false;
-        }
-        n_wall += k;
-      }
-      // Once the chunks and the backlog are used up, the wall branch runs as
-      // soon as at least as many photons wait for it as are stepping (the
-      // stepping ones go to the backlog), not only when every lane is idle:
-      // a wave's last photons would otherwise wait in the queue for its
-      // slowest in-column photon on every wall hit, which made the launch's
-      // drain about 12 ms of a 163-ms launch (3 ms this way).
-      const bool draining = pool_done && n_back == 0u;
-      const uint32_t n_alive = (uint32_t)__popcll(__ballot(alive));
-      if (n_wall >= 64u || (draining && n_wall != 0u && n_wall >= n_alive)) {
-        progress = true;
-        if (!swap_to_backlog<MULTI, REC>(wq, n_back, alive, parked, p, rng, lane_ev, gi, lane_k)) {
-          if (lane == 0) atomicOr(a.error_flag, 2u);
-          break;
-        }
-        const uint32_t take = min(n_wall, 64u);
-        // the wall entries are this wave's LDS writes, which complete in
-        // order; the barrier keeps the compiler from moving the reads
-        // above them
-        __builtin_amdgcn_wave_barrier();
-        if ((uint32_t)lane < take) {
-          bool pk;
-          q_get_at<MULTI, REC, kWallCap>(wall + n_wall - take + (uint32_t)lane, p, rng, lane_ev,
-                                         gi, lane_k, pk);
-          alive = true;
-        }
-        n_wall -= take;
-        PrptState st = prpt_initial();
-        int r = kPrAlive;
-        if (alive) r = prpt_loop(rng, p, geoms[MULTI ? gi : 0u], st, true, true);
-        if (alive && r == kPrEnded) {
-          finish_photon<MULTI, REC, RADIAL>(a, geoms, events, p, gi, lane_ev, lane_k, s_cnt, s_tile, side,
-                                            tile_area, run);
-          alive = false;
-        }
-        // refracted out of the column: the gap flight waits in the gap queue
-        // (it holds at most 63 + 64 entries here: the gap phase below runs
-        // whenever 64 wait)
-        const unsigned long long gm = __ballot(alive && r == kPrGap);
-        if (gm != 0ull) {
-          if (alive && r == kPrGap) {
-            const uint32_t slot = kGapBase + n_gap + rank_below(gm);
-            q_put<MULTI, REC>(wq, slot, p, rng, lane_ev, gi, lane_k, false);
-            q_put_state(wq, slot, st);
-            alive = false;
+    unsigned long long gap_m = 0;  // lanes whose photon's gap flight is next
+    PrptState st = prpt_initial();
+    bool drain = pool_done && n_ready == 0u && n_back == 0u;
+    // ---- serve
+    {
+      const unsigned long long waiting = drain || !queued ? wall_m : 0ull;
+      const bool due = !drain || end_m != 0ull || n_wall != 0u || n_gap != 0u;
+      if (step_m == 0ull ||
+          (due && (int)count(~(step_m | waiting)) >= a.refill_lanes)) {
+        if (end_m != 0ull) finish(end_m);
+        end_m = 0ull;
+        if (queued && !drain && n_wall + count(wall_m) < 64u) {
+          while (wall_m != 0ull) {
+            const uint32_t k =
+                min(count(wall_m), (uint32_t)kWallSlots - n_wall - n_ready);
+            const uint32_t rank = rank_below(wall_m);
+            const bool put = in(wall_m) && rank < k;
+            if (put) lds_put(n_wall + rank);
+            n_wall += k;
+            wall_m &= ~__ballot(put);
+            take_ready(~(step_m | wall_m));
           }
-          n_gap += (uint32_t)__popcll(gm);
         }
+        take_ready(~(step_m | wall_m));
+        unsigned long long need = ~(step_m | wall_m);
+        if (need != 0ull && n_back != 0u) {
+          __threadfence_block();  // the wave's queue stores are complete before its loads
+          const uint32_t t = min(count(need), n_back);
+          const uint32_t rank = rank_below(need);
+          const bool got = in(need) && rank < t;
+          if (got)
+            q_get<MULTI, REC, kQBlock>(wq + q_base(kBackBase + n_back - 1u - rank), p, rng,
+                                       lane_ev, gi, lane_k);
+          n_back -= t;
+          step_m |= __ballot(got);
+          need = ~(step_m | wall_m);
+        }
+        while (need != 0ull && !pool_done) {
+          const TransportArgs b = args();
+          const uint32_t chunk = 1u << b.chunk_log2;
+          if (pool_next >= pool_end) {
+            uint32_t c = 0;
+            if (lane == 0) c = atomicAdd(b.cursor, 1u);
+            c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
+            if (c >= chunk_off[b.n_events]) {
+              pool_done = true;
+              break;
+            }
+            // largest e with chunk_off[e] <= c (skips events without photons):
+            // each round the 64 lanes (all active here) probe 64 points of
+            // [lo, hi) with one vector load, and the wave keeps the step after
+            // the last probe at or below c -- 3 rounds for 2e5 events where a
+            // binary search makes 18 dependent loads
+            int64_t lo = 0, hi = b.n_events;
+            while (hi - lo > 1) {
+              const int64_t step = (hi - lo + 63) >> 6;
+              const int64_t pos = lo + (int64_t)lane * step;
+              const bool le = pos < hi && chunk_off[pos] <= c;
+              const unsigned long long m = __ballot(le);
+              lo += (int64_t)(63 - __clzll(m)) * step;
+              hi = min(hi, lo + step);
+            }
+            pool_ev = lo;
+            const int32_t n_ph = events[lo].N;
+            pool_next = (int32_t)((c - chunk_off[lo]) << b.chunk_log2);
+            pool_end = min(n_ph, pool_next + (int32_t)chunk);
+            if (lane == 0) {
+              const uint32_t gg = MULTI ? events[lo].geom : 0u;
+              atomicAdd(&s_cnt[gg * kCounters + FD2_C_GENERATED], (uint32_t)(pool_end - pool_next));
+            }
+            start_end = pool_next;
+          }
+          if (pool_next >= start_end) {
+            // Seeding a stream (Philox) and drawing the first direction are
+            // long; every lane starts one of the next 64 photons of the chunk
+            // here, at full width, instead of the few lanes that take photons
+            // in a pass.
+            start_base = pool_next;
+            start_end = min(pool_end, pool_next + 64);
+            if (start_base + lane < start_end) {
+              const uint32_t k = (uint32_t)(start_base + lane);
+              CounterRng r;
+              Photon q;
+              const uint64_t event_base = b.event_base_dev ? *b.event_base_dev : b.event_base;
+              r.seed(b.seed, event_base + (uint64_t)pool_ev, k);
+              if constexpr (MULTI)
+                counter_initial_dir(r, q, k, geoms[events[pool_ev].geom]);
+              else
+                counter_initial_dir(r, q, k, load_uniform<ColumnGeom>(geoms_in));
+              start[0][lane] = __float_as_uint(q.ux);
+              start[1][lane] = __float_as_uint(q.uy);
+              start[2][lane] = __float_as_uint(q.uz);
+              start[3][lane] = r.s0;
+              start[4][lane] = r.s1;
+              start[5][lane] = r.s2;
+              start[6][lane] = r.s3;
+            }
+            // lanes read other lanes' slots below; the wave's LDS accesses
+            // complete in order
+            __builtin_amdgcn_wave_barrier();
+          }
+          const int avail = start_end - pool_next;  // started, not yet taken
+          const int rank = (int)rank_below(need);
+          const bool got = in(need) && rank < avail;
+          if (got) {
+            const fd2_event ev = events[pool_ev];
+            gi = MULTI ? ev.geom : 0u;
+            const uint32_t k = (uint32_t)(pool_next + rank);
+            const uint32_t j = k - (uint32_t)start_base;
+            start_photon(p, ev);
+            p.ux = __uint_as_float(start[0][j]);
+            p.uy = __uint_as_float(start[1][j]);
+            p.uz = __uint_as_float(start[2][j]);
+            rng.s0 = start[3][j];
+            rng.s1 = start[4][j];
+            rng.s2 = start[5][j];
+            rng.s3 = start[6][j];
+            lane_ev = (uint32_t)pool_ev;
+            lane_k = k;
+          }
+          pool_next += min((int)count(need), avail);
+          step_m |= __ballot(got);
+          need = ~(step_m | wall_m);
+        }
+        drain = pool_done && n_ready == 0u && n_back == 0u;
+        if (drain && queued && need != 0ull && (n_wall | n_gap) != 0u) {
+          // the queues' last photons back into free lanes
+          uint32_t t = min(count(need), n_wall);
+          uint32_t rank = rank_below(need);
+          bool got = in(need) && rank < t;
+          __builtin_amdgcn_wave_barrier();
+          if (got) lds_get(n_wall - t + rank);
+          n_wall -= t;
+          wall_m |= __ballot(got);
+          need = ~(step_m | wall_m);
+          t = min(count(need), n_gap);
+          if (t != 0u) {
+            __threadfence_block();
+            rank = rank_below(need);
+            got = in(need) && rank < t;
+            if (got) {
+              const uint32_t* w = wq + q_base(kGapBase + n_gap - t + rank);
+              q_get<MULTI, REC, kQBlock>(w, p, rng, lane_ev, gi, lane_k);
+              q_get_state(w, st);
+            }
+            n_gap -= t;
+            gap_m = __ballot(got);
+          }
+        }
+        // nothing in a lane: the queues and the work queue are empty
+        if ((step_m | wall_m | gap_m) == 0ull) break;
       }
-      // Gap flights: a pass takes up to 64 waiting photons and runs one
-      // flight each (to the next column and its Fresnel decision); a photon
-      // reflected off the outside of that column goes back to the gap queue
-      // for its next flight.  Passes repeat while 64 wait, so the queue
-      // holds at most 63 entries after this loop and 127 during it.  While
-      // draining (as for the wall queue) they also run once at least as
-      // many flights wait as photons step.
-      bool failed = false;
-      while (n_gap >= 64u || (n_gap != 0u && n_wall == 0u && pool_done && n_back == 0u &&
-                              n_gap >= (uint32_t)__popcll(__ballot(alive)))) {
-        progress = true;
-        if (!swap_to_backlog<MULTI, REC>(wq, n_back, alive, parked, p, rng, lane_ev, gi, lane_k)) {
+    }
+    // every round steps a photon or runs a phase; a wave that does neither
+    // for many rounds has a broken queue state: it stops and flags the launch
+    // rather than spin
+    bool progress = step_m != 0ull;
+    // ---- pass
+    {
+      int r = kAlive;
+      if (in(step_m)) {
+        auto pass = [&](const ColumnGeom& g) {
+          r = hot_step<CounterRng, false>(rng, p, g, &nosink);
+          if (r == kTrapped) {
+            atomicAdd(&s_cnt[gi * kCounters + FD2_C_REGEN], 1u);
+            restart_trapped(rng, p, g, events[lane_ev]);
+          }
+        };
+        if constexpr (MULTI)
+          pass(geoms[gi]);
+        else
+          pass(load_uniform<ColumnGeom>(geoms_in));
+      }
+      const unsigned long long e = __ballot(r == kEnded), w = __ballot(r == kNeedPrpt);
+      end_m |= e;
+      wall_m |= w;
+      step_m &= ~(e | w);
+    }
+    // ---- wall
+    drain = pool_done && n_ready == 0u && n_back == 0u;
+    const bool in_place = drain || !queued;
+    const uint32_t n_lane = count(wall_m), n_step = count(step_m);
+    const bool full = !in_place && n_wall + n_lane >= 64u;
+    const bool place =
+        in_place && n_lane != 0u &&
+        (n_step == 0u || (queued ? n_lane >= n_step : (int)n_lane >= args().park_lanes));
+    if (full || place) {
+      progress = true;
+      if (end_m != 0ull) finish(end_m);
+      end_m = 0ull;
+      if (full) {
+        // every lane without a waiting photon takes one; a photon that was
+        // stepping takes a ready slot (all reads come before the writes)
+        const unsigned long long need = ~wall_m;
+        const uint32_t t = 64u - n_lane, rank = rank_below(need);
+        Photon q;
+        CounterRng r;
+        uint32_t ev = 0, g2 = 0, k2 = 0;
+        __builtin_amdgcn_wave_barrier();
+        if (in(need)) {
+          q_get<MULTI, REC, kWallSlots>(lq + n_wall - t + rank, q, r, ev, g2, k2);
+          __builtin_amdgcn_wave_barrier();
+          if (in(step_m))
+            lds_put((uint32_t)kWallSlots - n_ready - n_step + rank_below(step_m));
+          p = q;
+          rng = r;
+          lane_ev = ev;
+          gi = g2;
+          lane_k = k2;
+        }
+        n_wall -= t;
+        n_ready += n_step;
+        step_m = 0ull;
+        wall_m = ~0ull;
+      }
+      int r = kPrAlive;
+      const bool mine = in(wall_m);
+      if (mine)
+        with_geom([&](const GeomDev& g) { r = prpt_loop(rng, p, g, st, true, true); });
+      end_m = __ballot(mine && r == kPrEnded);
+      const unsigned long long flight = __ballot(mine && r == kPrGap);
+      step_m |= wall_m & ~(end_m | flight);
+      gap_m |= flight;
+      wall_m = 0ull;
+    }
+    // ---- gap: one flight per photon and round (to the next column and its
+    // Fresnel decision); a photon reflected off the outside of that column
+    // waits for its next flight.  The gap queue holds at most 63 + 64 entries
+    // here, and 63 between rounds.
+    bool failed = false;
+    for (;;) {
+      if (!in_place) {
+        if (gap_m != 0ull) {
+          if (in(gap_m)) {
+            uint32_t* w = wq + q_base(kGapBase + n_gap + rank_below(gap_m));
+            q_put<MULTI, REC, kQBlock>(w, p, rng, lane_ev, gi, lane_k);
+            q_put_state(w, st);
+          }
+          n_gap += count(gap_m);
+          gap_m = 0ull;
+        }
+        if (n_gap < 64u) break;
+        if (end_m != 0ull) finish(end_m);
+        end_m = 0ull;
+        const uint32_t s = count(step_m);
+        if (n_back + s > (uint32_t)kBackCap) {  // ruled out by the photons in flight
           failed = true;
           break;
         }
-        const uint32_t take = min(n_gap, 64u);
-        PrptState st = prpt_initial();
+        if (in(step_m))
+          q_put<MULTI, REC, kQBlock>(wq + q_base(kBackBase + n_back + rank_below(step_m)), p, rng,
+                                     lane_ev, gi, lane_k);
+        n_back += s;
+        step_m = 0ull;
         __threadfence_block();
-        if ((uint32_t)lane < take) {
-          bool pk;
-          const uint32_t slot = kGapBase + n_gap - take + (uint32_t)lane;
-          q_get<MULTI, REC>(wq, slot, p, rng, lane_ev, gi, lane_k, pk);
-          q_get_state(wq, slot, st);
-          alive = true;
-        }
-        n_gap -= take;
-        int r = kPrAlive;
-        if (alive) r = prpt_loop(rng, p, geoms[MULTI ? gi : 0u], st, false, true);
-        if (alive && r == kPrEnded) {
-          finish_photon<MULTI, REC, RADIAL>(a, geoms, events, p, gi, lane_ev, lane_k, s_cnt, s_tile, side,
-                                            tile_area, run);
-          alive = false;
-        }
-        // the slots just read are free again: [n_gap, n_gap + take)
-        const unsigned long long gm = __ballot(alive && r == kPrGap);
-        if (gm != 0ull) {
-          if (alive && r == kPrGap) {
-            const uint32_t slot = kGapBase + n_gap + rank_below(gm);
-            q_put<MULTI, REC>(wq, slot, p, rng, lane_ev, gi, lane_k, false);
-            q_put_state(wq, slot, st);
-            alive = false;
-          }
-          n_gap += (uint32_t)__popcll(gm);
-        }
-      }
-      if (failed) {
-        if (lane == 0) atomicOr(a.error_flag, 2u);
+        const uint32_t* w = wq + q_base(kGapBase + n_gap - 64u + (uint32_t)lane);
+        q_get<MULTI, REC, kQBlock>(w, p, rng, lane_ev, gi, lane_k);
+        q_get_state(w, st);
+        n_gap -= 64u;
+        gap_m = ~0ull;
+      } else if (gap_m == 0ull) {
         break;
       }
-      if (progress) {
-        idle = 0;
-      } else if (++idle > kMaxIdlePasses) {
-        if (lane == 0) atomicOr(a.error_flag, 2u);
-        break;
-      }
-    } else {
-      // The wall-Fresnel branch (with the gap flights it leads to) is long
-      // and taken by few lanes at a time: run it once enough lanes wait for
-      // it, or when nothing else can run.
-      const unsigned long long parked_mask = __ballot(parked);
-      if (parked_mask != 0ull &&
-          ((int)__popcll(parked_mask) >= a.park_lanes || __ballot(alive && !parked) == 0ull)) {
-        if (parked) {
-          const GeomDev& g = geoms[MULTI ? gi : 0u];
-          ended = ba_prpt(rng, p, g);
-          parked = false;
-        }
-      }
-      if (ended) {
-        finish_photon<MULTI, REC, RADIAL>(a, geoms, events, p, gi, lane_ev, lane_k, s_cnt, s_tile, side,
-                                          tile_area, run);
-        alive = false;
-      }
+      progress = true;
+      int r = kPrAlive;
+      const bool mine = in(gap_m);
+      if (mine)
+        with_geom([&](const GeomDev& g) { r = prpt_loop(rng, p, g, st, false, true); });
+      const unsigned long long e = __ballot(mine && r == kPrEnded);
+      const unsigned long long again = __ballot(mine && r == kPrGap);
+      end_m |= e;
+      step_m |= gap_m & ~(e | again);
+      gap_m = again;
+    }
+    if (progress) {
+      idle = 0;
+    } else if (++idle > kMaxIdlePasses) {
+      failed = true;
+    }
+    if (failed) {
+      if (lane == 0) atomicOr(args().error_flag, 2u);
+      break;
     }
   }
 
-  if (run[1]) flush_run<MULTI>(geoms, events, run[0], run[1]);
+  if (run[1]) flush_run<MULTI>(geoms_in[0], geoms, events, run[0], run[1]);
   __syncthreads();
-  for (int i = threadIdx.x; i < a.n_geoms * kCounters; i += blockDim.x)
-    if (s_cnt[i]) tally_add(&a.counters[i], (unsigned long long)s_cnt[i]);
-  for (int t = 0; t < a.n_tiles; ++t) {
+  const TransportArgs b = args();
+  const int side = b.tile_side;
+  const int tile_area = side * side;
+  for (int i = threadIdx.x; i < b.n_geoms * kCounters; i += blockDim.x)
+    if (s_cnt[i]) tally_add(&b.counters[i], (unsigned long long)s_cnt[i]);
+  for (int t = 0; t < b.n_tiles; ++t) {
     const GeomDev& gt = geoms[t];
     const int i0 = tile_origin(gt.xdim, side), j0 = tile_origin(gt.ydim, side);
     for (int e = threadIdx.x; e < tile_area; e += blockDim.x) {
@@ -804,12 +831,8 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
 template <bool MULTI, bool REC, bool RADIAL>
 static void launch_one(const TransportArgs& a, dim3 grid, hipStream_t s) {
   const size_t smem = (size_t)a.n_tiles * a.tile_side * a.tile_side * sizeof(uint32_t);
-  if (a.wave_queue)
-    hipLaunchKernelGGL((k_transport<MULTI, REC, RADIAL, true>), grid, dim3(kTransportThreads),
-                       smem, s, a, a.geoms, a.events, a.chunk_off);
-  else
-    hipLaunchKernelGGL((k_transport<MULTI, REC, RADIAL, false>), grid, dim3(kTransportThreads),
-                       smem, s, a, a.geoms, a.events, a.chunk_off);
+  hipLaunchKernelGGL((k_transport<MULTI, REC, RADIAL>), grid, dim3(kTransportThreads), smem, s, a,
+                     a.geoms, a.events, a.chunk_off);
 }
 
 hipError_t launch_transport(const TransportArgs& a, bool multi, bool record,
@@ -829,46 +852,38 @@ hipError_t launch_transport(const TransportArgs& a, bool multi, bool record,
 }
 
 template <bool MULTI, bool REC, bool RADIAL>
-static int occupancy_of(size_t smem, bool queue) {
+static int occupancy_of(size_t smem) {
   int nb = 0;
-  const hipError_t e =
-      queue ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                  &nb, k_transport<MULTI, REC, RADIAL, true>, kTransportThreads, smem)
-            : hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                  &nb, k_transport<MULTI, REC, RADIAL, false>, kTransportThreads, smem);
-  if (e != hipSuccess) return 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_transport<MULTI, REC, RADIAL>,
+                                                   kTransportThreads, smem) != hipSuccess)
+    return 1;
   return nb > 0 ? nb : 1;
 }
 
-template <bool MULTI, bool REC, bool RADIAL, bool QUEUE>
+template <bool MULTI, bool REC, bool RADIAL>
 static size_t static_lds_of() {
   hipFuncAttributes at{};
-  if (hipFuncGetAttributes(&at, reinterpret_cast<const void*>(
-                                    &k_transport<MULTI, REC, RADIAL, QUEUE>)) != hipSuccess)
+  if (hipFuncGetAttributes(&at, reinterpret_cast<const void*>(&k_transport<MULTI, REC, RADIAL>)) !=
+      hipSuccess)
     return 0;
   return at.sharedSizeBytes;
 }
 
 size_t transport_static_lds() {
   // the several-geometry variants hold the geometry table: the largest
-  const size_t a = static_lds_of<true, false, false, true>();
-  const size_t b = static_lds_of<true, true, false, true>();
-  const size_t c = static_lds_of<true, false, true, true>();
-  const size_t d = static_lds_of<true, false, false, false>();
-  size_t m = a > b ? a : b;
-  m = m > c ? m : c;
-  return m > d ? m : d;
+  const size_t a = static_lds_of<true, false, false>();
+  const size_t b = static_lds_of<true, true, false>();
+  const size_t c = static_lds_of<true, false, true>();
+  const size_t m = a > b ? a : b;
+  return m > c ? m : c;
 }
 
-int transport_max_blocks_per_cu(bool multi, bool record, bool radial, size_t smem, bool queue) {
+int transport_max_blocks_per_cu(bool multi, bool record, bool radial, size_t smem) {
   if (radial)
-    return multi ? occupancy_of<true, false, true>(smem, queue)
-                 : occupancy_of<false, false, true>(smem, queue);
+    return multi ? occupancy_of<true, false, true>(smem) : occupancy_of<false, false, true>(smem);
   if (multi)
-    return record ? occupancy_of<true, true, false>(smem, queue)
-                  : occupancy_of<true, false, false>(smem, queue);
-  return record ? occupancy_of<false, true, false>(smem, queue)
-                : occupancy_of<false, false, false>(smem, queue);
+    return record ? occupancy_of<true, true, false>(smem) : occupancy_of<true, false, false>(smem);
+  return record ? occupancy_of<false, true, false>(smem) : occupancy_of<false, false, false>(smem);
 }
 
 // ------------------------------------------------ RANECU trajectory mode
@@ -904,15 +919,15 @@ __global__ void __launch_bounds__(64) k_trace_ranecu(
         restart_trapped<RanecuRng, M>(rng, p, g, ev);
       }
     }
-    cnt[fate_counter(p.fate)]++;
+    cnt[p.fate - 1]++;
     const bool det = p.fate == kDetectOut;
-    if (det) detected_pixel(p, g);
-    if (p.fate == kDetect) atomicAdd(&g.prf[pix_index(p.pix, g)], 1ull);
+    const Pixel x = det ? detected_pixel(p, g) : Pixel{0, 0};
+    if (p.fate == kDetect) atomicAdd(&g.prf[pix_index(x, g)], 1ull);
     if (det && ev.hist >= 1 && ev.hist <= g.num_hist) atomicAdd(&g.hist[ev.hist - 1], 1u);
     if (records) {
       fd2_photon rec;
-      rec.fate = p.fate;
-      rec.pix = p.fate == kDetect ? pix_index(p.pix, g) : -1;
+      rec.fate = p.fate == kGone ? kNone : p.fate;
+      rec.pix = p.fate == kDetect ? pix_index(x, g) : -1;
       rec.x = det ? p.px : 0.0f;
       rec.y = det ? p.py : 0.0f;
       records[photon_off[i] + k] = rec;
