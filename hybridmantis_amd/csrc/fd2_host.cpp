@@ -130,12 +130,9 @@ int grow(fd2_ctx* c, size_t n_events) {
   }
   if (n_events + 1 > c->cap_off) {
     size_t cap = n_events + n_events / 4 + 1025;
-    if (c->d_chunk_off) (void)hipFree(c->d_chunk_off);
     if (c->d_photon_off) (void)hipFree(c->d_photon_off);
-    c->d_chunk_off = nullptr;
     c->d_photon_off = nullptr;
     c->cap_off = 0;
-    FD2_HIP(hipMalloc(&c->d_chunk_off, cap * sizeof(uint32_t)));
     FD2_HIP(hipMalloc(&c->d_photon_off, cap * sizeof(unsigned long long)));
     c->cap_off = cap;
   }
@@ -189,7 +186,6 @@ void tile_shape(int lds_tile, int n_geoms, int32_t* side, int32_t* n_tiles) {
 
 // Work-queue buffers of one launch (the context's own, or a graph's).
 struct QueueBufs {
-  uint32_t* chunk_off;
   unsigned long long* photon_off;
   uint32_t* block_chunks;
   unsigned long long* block_photons;
@@ -203,24 +199,22 @@ struct Launch {
   bool multi = false, record = false, radial = false;
 };
 
-// Queue cursor and error flag of a launch other than the context's own,
-// with the transport in park-in-place mode (no per-wave queues).
-struct NoQueueScratch {
-  uint32_t* cursor;
+// Queue plan and error flag of a launch other than the context's own.
+struct OwnScratch {
+  QueuePlan* plan;
   uint32_t* error_flag;
 };
 
 Launch make_launch(const fd2_ctx* c, const QueueBufs& b, const fd2_event* d_ev, int64_t n,
                    fd2_photon* d_records, uint32_t* d_radial,
-                   const NoQueueScratch* own = nullptr) {
+                   const OwnScratch* own = nullptr) {
   Launch L;
   QueueArgs& q = L.q;
   q.events = d_ev;
-  q.chunk_off = b.chunk_off;
   q.photon_off = b.photon_off;
   q.block_chunks = b.block_chunks;
   q.block_photons = b.block_photons;
-  q.cursor = own ? own->cursor : c->d_cursor;
+  q.plan = own ? own->plan : c->d_plan;
   q.error_flag = own ? own->error_flag : c->d_error;
   q.n_events = n;
   q.n_geoms = c->n_geoms;
@@ -230,22 +224,20 @@ Launch make_launch(const fd2_ctx* c, const QueueBufs& b, const fd2_event* d_ev, 
 
   TransportArgs& a = L.a;
   a.events = d_ev;
-  a.chunk_off = b.chunk_off;
   a.photon_off = b.photon_off;
   a.geoms = c->d_geoms;
   a.counters = c->d_counters;
-  a.cursor = q.cursor;
+  a.plan = q.plan;
   a.records = d_records;
   a.radial = d_radial;
   a.event_base_dev = nullptr;
-  const bool queue = !own && c->tune.wall_queue >= 0 && c->d_wave_queue != nullptr;
+  const bool queue = c->tune.wall_queue >= 0 && c->d_wave_queue != nullptr;
   a.wave_queue = queue ? c->d_wave_queue : nullptr;
   a.error_flag = q.error_flag;
   a.n_events = n;
   a.seed = c->seed;
   a.event_base = (uint64_t)c->next_event;
   a.n_geoms = c->n_geoms;
-  a.chunk_log2 = q.chunk_log2;
   a.park_lanes = c->tune.park_lanes;
   a.refill_lanes = c->tune.refill_lanes;
   tile_shape(c->tune.lds_tile, c->n_geoms, &a.tile_side, &a.n_tiles);
@@ -254,11 +246,14 @@ Launch make_launch(const fd2_ctx* c, const QueueBufs& b, const fd2_event* d_ev, 
   L.record = d_records != nullptr;
   L.radial = d_radial != nullptr;
   const int per_cu = c->tune.waves_per_cu / (kTransportThreads / 64);
-  const size_t smem = (size_t)a.n_tiles * a.tile_side * a.tile_side * sizeof(uint32_t);
+  const size_t smem = transport_dynamic_lds(L.multi, c->n_geoms,
+                                            (size_t)a.n_tiles * a.tile_side * a.tile_side);
   const int occ = transport_max_blocks_per_cu(L.multi, L.record, L.radial, smem);
   L.blocks = c->n_cu * (per_cu < 1 ? 1 : (per_cu > occ ? occ : per_cu));
   if (queue && L.blocks * (kTransportThreads / 64) > c->max_waves)
     L.blocks = c->max_waves / (kTransportThreads / 64);
+  q.n_simds = (uint32_t)(c->n_cu * 4);
+  q.n_waves = (uint32_t)(L.blocks * (kTransportThreads / 64));
   return L;
 }
 
@@ -279,7 +274,7 @@ int enqueue(fd2_ctx* c, const fd2_event* d_ev, int64_t n, bool record,
   if (n <= 0) return FD2_OK;
   int rc = grow(c, (size_t)n);
   if (rc) return rc;
-  const QueueBufs b{c->d_chunk_off, c->d_photon_off, c->d_block_chunks, c->d_block_photons};
+  const QueueBufs b{c->d_photon_off, c->d_block_chunks, c->d_block_photons};
   const uint64_t chunk = (uint64_t)c->tune.chunk, limit = (uint64_t)c->tune.max_chunks;
   FD2_HIP(hipEventRecord(c->ev_start, c->stream));
   uint64_t photons_before = 0;
@@ -326,20 +321,21 @@ int check_error_flag(fd2_ctx* c) {
 
 // ------------------------------------------- allocation-free submit scratch
 //
-// fd2_submit_device_noalloc keeps its work-queue scratch -- cursor, error
-// flag, block totals and the per-event chunk and photon offsets of at most
-// FD2_NOALLOC_MAX_EVENTS events -- in this file-scope device array, 12.6 MB
-// that each GPU the library runs on holds until the process ends.  Host
+// fd2_submit_device_noalloc keeps its work-queue scratch -- plan, error
+// flag, block totals and the per-event photon offsets of at most
+// FD2_NOALLOC_MAX_EVENTS events -- in this file-scope device array, 8.4 MB
+// that each GPU the library runs on holds until the process ends (the
+// per-wave photon queues are the context's, made by fd2_create).  Host
 // code uses the array only through the address hipGetSymbolAddress gives
 // on each device (its own copy there), looked up once per device at
 // fd2_create with that device current.
 constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 constexpr int64_t kNaEvents = FD2_NOALLOC_MAX_EVENTS;
 constexpr int64_t kNaBlocks = (kNaEvents + kScanTile - 1) / kScanTile;
-constexpr size_t kNaBlockChunks = 256;  // [0, 256): cursor, error flag
+constexpr size_t kNaErrorFlag = 64;     // [0, 64): plan
+constexpr size_t kNaBlockChunks = 256;
 constexpr size_t kNaBlockPhotons = align256(kNaBlockChunks + sizeof(uint32_t) * kNaBlocks);
-constexpr size_t kNaChunkOff = align256(kNaBlockPhotons + sizeof(unsigned long long) * kNaBlocks);
-constexpr size_t kNaPhotonOff = align256(kNaChunkOff + sizeof(uint32_t) * (kNaEvents + 1));
+constexpr size_t kNaPhotonOff = align256(kNaBlockPhotons + sizeof(unsigned long long) * kNaBlocks);
 constexpr size_t kNaBytes = align256(kNaPhotonOff + sizeof(unsigned long long) * (kNaEvents + 1));
 constexpr int kNaMaxDevices = 64;
 
@@ -455,7 +451,7 @@ int fd2_create(const fd2_params* params, int n_geoms, int device, fd2_ctx** out)
     if (rc) break;
     if (hipMalloc(&c->d_geoms, sizeof(GeomDev) * n_geoms) != hipSuccess ||
         hipMalloc(&c->d_counters, sizeof(unsigned long long) * kCounters * n_geoms) != hipSuccess ||
-        hipMalloc(&c->d_cursor, sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc(&c->d_plan, sizeof(QueuePlan)) != hipSuccess ||
         hipMalloc(&c->d_error, sizeof(uint32_t)) != hipSuccess) {
       rc = FD2_E_NOMEM;
       break;
@@ -469,7 +465,9 @@ int fd2_create(const fd2_params* params, int n_geoms, int device, fd2_ctx** out)
     {
       int occ = 1;
       for (int v = 0; v < 5; ++v) {
-        const int o = transport_max_blocks_per_cu(v == 1 || v == 3, v == 2 || v == 3, v == 4, 0);
+        const bool multi = v == 1 || v == 3;
+        const int o = transport_max_blocks_per_cu(multi, v == 2 || v == 3, v == 4,
+                                                  transport_dynamic_lds(multi, 2, 0));
         if (o > occ) occ = o;
       }
       c->max_waves = c->n_cu * occ * (kTransportThreads / 64);
@@ -477,7 +475,6 @@ int fd2_create(const fd2_params* params, int n_geoms, int device, fd2_ctx** out)
       if (hipMalloc(&c->d_wave_queue, qbytes) != hipSuccess) { rc = FD2_E_NOMEM; break; }
     }
     if (launch_fill_u32(c->d_error, 1, c->stream) != hipSuccess) { rc = FD2_E_DEVICE; break; }
-    if (launch_fill_u32(c->d_cursor, 1, c->stream) != hipSuccess) { rc = FD2_E_DEVICE; break; }
     rc = fd2_reset(c);
   } while (0);
   if (rc) {
@@ -496,9 +493,8 @@ void fd2_destroy(fd2_ctx* c) {
     if (c->d_prf[i]) (void)hipFree(c->d_prf[i]);
     if (c->d_hist[i]) (void)hipFree(c->d_hist[i]);
   }
-  void* bufs[] = {c->d_geoms, c->d_wave_queue, c->d_counters, c->d_events, c->d_chunk_off,
-                  c->d_photon_off, c->d_block_chunks, c->d_block_photons,
-                  c->d_cursor, c->d_error};
+  void* bufs[] = {c->d_geoms, c->d_wave_queue, c->d_counters, c->d_events, c->d_photon_off,
+                  c->d_block_chunks, c->d_block_photons, c->d_plan, c->d_error};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   if (c->h_stage) (void)hipHostFree(c->h_stage);
@@ -529,8 +525,8 @@ int fd2_set_tuning(fd2_ctx* c, const fd2_tuning* t) {
   {  // the tiles and the kernel's static LDS must fit one workgroup's LDS
     int32_t side = 0, n_tiles = 0;
     tile_shape(t->lds_tile, c->n_geoms, &side, &n_tiles);
-    const size_t tiles = (size_t)n_tiles * side * side * sizeof(uint32_t);
-    if (c->lds_per_block && tiles + c->lds_static > c->lds_per_block) return FD2_E_INVAL;
+    const size_t dyn = transport_dynamic_lds(c->n_geoms > 1, c->n_geoms, (size_t)n_tiles * side * side);
+    if (c->lds_per_block && dyn + c->lds_static > c->lds_per_block) return FD2_E_INVAL;
   }
   n.lds_tile = t->lds_tile;
   if (t->park_lanes) {
@@ -609,12 +605,12 @@ int fd2_submit_device_noalloc(fd2_ctx* c, const fd2_event* d_events, int64_t n) 
   if (!s) return FD2_E_STATE;
   if (n == 0) return FD2_OK;
   FD2_HIP(hipSetDevice(c->device));
-  const NoQueueScratch own{(uint32_t*)s, (uint32_t*)s + 1};
-  const QueueBufs b{(uint32_t*)(s + kNaChunkOff), (unsigned long long*)(s + kNaPhotonOff),
-                    (uint32_t*)(s + kNaBlockChunks), (unsigned long long*)(s + kNaBlockPhotons)};
+  const OwnScratch own{(QueuePlan*)s, (uint32_t*)(s + kNaErrorFlag)};
+  const QueueBufs b{(unsigned long long*)(s + kNaPhotonOff), (uint32_t*)(s + kNaBlockChunks),
+                    (unsigned long long*)(s + kNaBlockPhotons)};
   const Launch L = make_launch(c, b, d_events, n, nullptr, nullptr, &own);
   // the array keeps the last call's contents: the error flag starts at zero
-  // here, the queue build zeroes the cursor, and the offsets are rewritten
+  // here, the queue build writes the plan, and the offsets are rewritten
   FD2_HIP(launch_fill_u32(own.error_flag, 1, c->stream));
   FD2_HIP(hipEventRecord(c->ev_start, c->stream));
   FD2_HIP(issue(L, c->stream));
@@ -906,7 +902,6 @@ int fd2_last_kernel_ms(fd2_ctx* c, float* ms) {
 struct fd2_graph {
   fd2_ctx* c = nullptr;
   int64_t n = 0;
-  uint32_t* d_chunk_off = nullptr;
   unsigned long long* d_photon_off = nullptr;
   uint32_t* d_block_chunks = nullptr;
   unsigned long long* d_block_photons = nullptr;
@@ -925,8 +920,7 @@ void fd2_graph_destroy(fd2_graph* g) {
   }
   if (g->exec) (void)hipGraphExecDestroy(g->exec);
   if (g->graph) (void)hipGraphDestroy(g->graph);
-  void* bufs[] = {g->d_chunk_off, g->d_photon_off, g->d_block_chunks, g->d_block_photons,
-                  g->d_base};
+  void* bufs[] = {g->d_photon_off, g->d_block_chunks, g->d_block_photons, g->d_base};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   delete g;
@@ -943,14 +937,13 @@ int fd2_graph_create(fd2_ctx* c, const fd2_event* d_events, int64_t n, fd2_graph
   g->n = n;
   const size_t nb = (size_t)((n + kScanTile - 1) / kScanTile) + 1;
   int rc = FD2_OK;
-  if (hipMalloc(&g->d_chunk_off, (size_t)(n + 1) * sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&g->d_photon_off, (size_t)(n + 1) * sizeof(unsigned long long)) != hipSuccess ||
+  if (hipMalloc(&g->d_photon_off, (size_t)(n + 1) * sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc(&g->d_block_chunks, nb * sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&g->d_block_photons, nb * sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc(&g->d_base, sizeof(unsigned long long)) != hipSuccess)
     rc = FD2_E_NOMEM;
   if (!rc) {
-    const QueueBufs b{g->d_chunk_off, g->d_photon_off, g->d_block_chunks, g->d_block_photons};
+    const QueueBufs b{g->d_photon_off, g->d_block_chunks, g->d_block_photons};
     Launch L = make_launch(c, b, d_events, n, nullptr, nullptr);
     L.a.event_base_dev = g->d_base;
     if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {

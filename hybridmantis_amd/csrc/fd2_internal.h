@@ -10,13 +10,20 @@ namespace fd2 {
 
 enum { kCounters = FD2_NCOUNT };
 
+// How a launch's photons are handed out, made by the queue build.
+struct QueuePlan {
+  uint32_t cursor;      // spans taken so far
+  uint32_t span_log2;   // photons per span
+  uint32_t lane_cap;    // lanes of a wave that take photons
+  uint32_t blocks;      // workgroups of the transport that take part
+};
+
 struct TransportArgs {
   const fd2_event* events;             // device
-  const uint32_t* chunk_off;           // n_events + 1 (exclusive scan)
   const unsigned long long* photon_off;  // n_events + 1 (exclusive scan)
   const GeomDev* geoms;                // n_geoms
   unsigned long long* counters;        // n_geoms * FD2_NCOUNT
-  uint32_t* cursor;                    // work-queue cursor (zeroed by the scan)
+  QueuePlan* plan;
   fd2_photon* records;                 // per-photon records (recording only)
   uint32_t* radial;                    // n_events x FD2_RADIAL_BINS (radial mode)
   const unsigned long long* event_base_dev;  // if set, read the number of events[0] here
@@ -26,7 +33,6 @@ struct TransportArgs {
   uint32_t seed;
   uint64_t event_base;                 // global number of events[0]
   int32_t n_geoms;
-  int32_t chunk_log2;
   int32_t park_lanes;                  // lanes waiting before a Fresnel phase
   int32_t refill_lanes;                // free lanes before new photons start
   int32_t tile_side;                   // LDS PRF tile side (pixels), 0 = none
@@ -38,15 +44,16 @@ struct TransportArgs {
 // (u32) and adds the block's counts to the PRF at the end.
 constexpr int kTileDefault = 0;  // no tile: the LDS holds the wall queues
 constexpr int kTileBudget = 64 * 64;   // u32 entries per block (16 KiB)
-// started photons of a wave's chunk in LDS (direction + stream words)
-constexpr int kStartWords = 7;
 // per-wave photon queues of the persistent kernel: photons waiting for the
-// wall branch and photons ready to step in LDS (at most 64, and 8 slots to
-// write before reading), the gap queue and the backlog in HBM (slots in that
-// order).  At most 64 + 64 + kGapCap photons are in flight per wave.
-constexpr int kWallSlots = 72;
+// wall branch (at most 63) and photons ready to step in LDS, together at most
+// kLdsCap (so that new photons always start at least 33 at a time), and 8
+// slots to write before reading; the gap queue and the backlog in HBM (slots
+// in that order).  At most 64 + kLdsCap + kGapCap photons are in flight per
+// wave.
+constexpr int kLdsCap = 96;
+constexpr int kWallSlots = kLdsCap + 8;
 constexpr int kGapCap = 128;
-constexpr int kBackCap = 64 + 64 + kGapCap;
+constexpr int kBackCap = 64 + kLdsCap + kGapCap;
 constexpr int kGapBase = 0;
 constexpr int kBackBase = kGapCap;
 constexpr int kQSlots = kGapCap + kBackCap;
@@ -62,16 +69,17 @@ constexpr int kTileMax = 112;
 
 struct QueueArgs {
   const fd2_event* events;
-  uint32_t* chunk_off;
   unsigned long long* photon_off;
   uint32_t* block_chunks;      // per scan block
   unsigned long long* block_photons;
-  uint32_t* cursor;
+  QueuePlan* plan;
   uint32_t* error_flag;        // set when an event is invalid
   int64_t n_events;
   int32_t n_geoms;
   int32_t chunk_log2;
   int32_t n_blocks;
+  uint32_t n_waves;            // waves of the transport launch
+  uint32_t n_simds;            // SIMDs of the device
   uint64_t max_chunks;         // more work items than this: error bit 4, nothing runs
 };
 
@@ -79,6 +87,12 @@ constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanThreads * kScanItems;
 constexpr int kTransportThreads = 256;
+
+// dynamic LDS of the transport: the geometry table (several geometries) and
+// `tile_words` words of PRF tiles
+inline size_t transport_dynamic_lds(bool multi, int n_geoms, size_t tile_words) {
+  return (multi ? (size_t)n_geoms * sizeof(GeomDev) : 0) + tile_words * sizeof(uint32_t);
+}
 
 // launch wrappers (fd2_kernels.hip)
 hipError_t launch_queue_build(const QueueArgs& q, hipStream_t s);
@@ -128,13 +142,12 @@ struct fd2_ctx {
   size_t cap_stage = 0;
   fd2_event* d_events = nullptr;
   size_t cap_events = 0;
-  uint32_t* d_chunk_off = nullptr;
   unsigned long long* d_photon_off = nullptr;
   size_t cap_off = 0;
   uint32_t* d_block_chunks = nullptr;
   unsigned long long* d_block_photons = nullptr;
   size_t cap_blocks = 0;
-  uint32_t* d_cursor = nullptr;
+  fd2::QueuePlan* d_plan = nullptr;
   uint32_t* d_error = nullptr;
   uint32_t* d_wave_queue = nullptr;    // kQWords x kQSlots words per resident wave
   int max_waves = 0;

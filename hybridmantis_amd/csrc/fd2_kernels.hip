@@ -1,14 +1,14 @@
 // fd2_kernels.hip -- HIP kernels of the MI355X fastDETECT2 transport.
 //
-//   k_queue_*     device work queue: exclusive scans of per-event chunk and
-//                 photon counts (replaces the reference's host load
+//   k_queue_*     device work queue: exclusive scan of the events' photon
+//                 counts (replaces the reference's host load
 //                 balancer, main/hybridMANTIS_tallyEnergyDepositionEvents.f:
 //                 195-250, and its one-thread-per-event launch,
 //                 main/hybridMANTIS_cuda_ver1_0.cu:277)
-//   k_transport   persistent kernel: each wave takes chunks of photons from
-//                 the queue with one atomic per chunk and hands photons to
-//                 its idle lanes, so events of very uneven size keep every
-//                 lane busy
+//   k_transport   persistent kernel: each wave takes spans of consecutive
+//                 photons from the queue with one atomic per span and hands
+//                 photons to its idle lanes, so events of very uneven size
+//                 keep every lane busy
 //   k_trace_ranecu one lane per event, photons in sequence, the reference's
 //                 per-event RANECU stream (trajectory test)
 //   k_debug_steps per-step FP32 trace of a few photons (FP64 re-trace check)
@@ -30,134 +30,167 @@ __device__ __forceinline__ T wave_incl_scan(T x) {
   return x;
 }
 
-// exclusive scan over the block (kScanThreads threads); returns the
-// exclusive prefix of `v` and the block total in `total`
-template <typename T>
-__device__ __forceinline__ T block_excl_scan(T v, T* s_wave, T& total) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  constexpr int kWaves = kScanThreads / 64;
-  T inc = wave_incl_scan(v);
-  if (lane == 63) s_wave[wid] = inc;
-  __syncthreads();
-  if (wid == 0) {
-    T w = lane < kWaves ? s_wave[lane] : T(0);
-    T wi = wave_incl_scan(w);
-    if (lane < kWaves) s_wave[lane] = wi - w;
-    if (lane == kWaves - 1) s_wave[kWaves] = wi;
-  }
-  __syncthreads();
-  total = s_wave[kWaves];
-  T r = s_wave[wid] + inc - v;
-  __syncthreads();
-  return r;
-}
-
+// photon and work-item (chunk) counts of event e; an event with a bad count
+// or geometry has none and flags the launch
 __device__ __forceinline__ void event_counts(const QueueArgs& q, int64_t e,
                                              uint32_t& chunks, uint32_t& photons) {
   chunks = 0;
   photons = 0;
   if (e >= q.n_events) return;
-  const fd2_event ev = q.events[e];
-  if (ev.N < 0 || ev.N > FD2_MAX_PHOTONS_PER_EVENT || ev.geom >= (uint32_t)q.n_geoms) {
-    if (ev.N != 0) atomicOr(q.error_flag, 1u);
+  const int32_t n = q.events[e].N;
+  const uint32_t geom = q.events[e].geom;
+  if (n < 0 || n > FD2_MAX_PHOTONS_PER_EVENT || geom >= (uint32_t)q.n_geoms) {
+    if (n != 0) atomicOr(q.error_flag, 1u);
     return;
   }
-  photons = (uint32_t)ev.N;
+  photons = (uint32_t)n;
   chunks = (photons + (1u << q.chunk_log2) - 1u) >> q.chunk_log2;
+}
+
+// A block's kScanTile events, a wave's 256 consecutive ones as kScanItems
+// rows of 64 (each row one coalesced load): photon counts per row in ph, the
+// number of photons before this wave's events in `before`, block totals in
+// tp (photons) and tc (work items).  A block's totals fit 32 bits (4096
+// events of at most 900,000 photons).
+__device__ __forceinline__ void block_counts(const QueueArgs& q, int64_t base,
+                                             uint32_t (&ph)[kScanItems], uint32_t& before,
+                                             uint32_t& tp, uint32_t& tc) {
+  constexpr int kWaves = kScanThreads / 64;
+  __shared__ uint32_t s_p[kWaves], s_c[kWaves];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  uint32_t p = 0, c = 0;
+#pragma unroll
+  for (int i = 0; i < kScanItems; ++i) {
+    uint32_t cc;
+    event_counts(q, base + wid * (64 * kScanItems) + i * 64 + lane, cc, ph[i]);
+    p += ph[i];
+    c += cc;
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    p += __shfl_xor(p, o, 64);
+    c += __shfl_xor(c, o, 64);
+  }
+  __syncthreads();
+  if (lane == 0) {
+    s_p[wid] = p;
+    s_c[wid] = c;
+  }
+  __syncthreads();
+  before = tp = tc = 0;
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < wid) before += s_p[w];
+    tp += s_p[w];
+    tc += s_c[w];
+  }
+}
+
+// photon_off of the block's events, `start` photons before the block
+__device__ __forceinline__ void write_offsets(const QueueArgs& q, int64_t base,
+                                              const uint32_t (&ph)[kScanItems],
+                                              unsigned long long start) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+  for (int i = 0; i < kScanItems; ++i) {
+    const uint32_t inc = wave_incl_scan(ph[i]);
+    const int64_t e = base + wid * (64 * kScanItems) + i * 64 + lane;
+    if (e < q.n_events) q.photon_off[e] = start + inc - ph[i];
+    start += (uint32_t)__shfl((int)inc, 63, 64);
+  }
+}
+
+// Totals, and how the launch is cut up (one thread).  A launch of more work
+// items than q.max_chunks sets error bit 4 and gets a total of 0, so the
+// transport takes nothing.
+//
+// A large launch uses all its workgroups and takes spans of half a wave's
+// share, at most the tuning's chunk.  A small one lasts as long as its longest
+// photon's chain of passes (up to some hundreds), and a pass takes the longer
+// the more waves share a SIMD (a wave alone waits for its own instructions;
+// six issue 3 times as many as fit meanwhile) and the more lanes take its rare
+// branches.  So the photons go to one wave per SIMD first, evenly, lane_cap
+// to a wave; then to more waves, 64 lanes at kLaneShare photons each.  On
+// MI355X, kernel time before (spans of 128 photons of one event, all waves)
+// and now: one event of 1,375 photons 0.89 -> 0.5 ms, 200 histories at 60 keV
+// (5.3e5 photons) 6.1 -> 3.3 ms; kLaneShare 1, 2, 4, 8, 16 on 500 histories at
+// 25 keV: 3.9, 3.8, 3.1, 3.7, 3.8 ms.
+__device__ __forceinline__ void plan_queue(const QueueArgs& q, unsigned long long photons,
+                                           uint64_t chunks) {
+  constexpr uint32_t kWaves = kTransportThreads / 64;
+  constexpr unsigned long long kLaneShare = 4;
+  const bool over = chunks > q.max_chunks;
+  if (over) atomicOr(q.error_flag, 4u);
+  q.photon_off[q.n_events] = over ? 0ull : photons;
+  const uint32_t alone = min(q.n_simds, q.n_waves);
+  unsigned long long waves = photons / (64u * kLaneShare);
+  if (waves < alone) waves = alone;
+  if (waves > q.n_waves) waves = q.n_waves;
+  uint32_t span_log2 = 0, lane_cap = 64;
+  if (photons >= 64u * waves) {
+    const unsigned long long share = photons / waves;
+    while (span_log2 < (uint32_t)q.chunk_log2 && (4ull << span_log2) <= share) ++span_log2;
+  } else {
+    while ((waves << span_log2) < photons) ++span_log2;
+    lane_cap = 1u << span_log2;
+    if ((uint32_t)q.chunk_log2 < span_log2) span_log2 = (uint32_t)q.chunk_log2;
+  }
+  q.plan->cursor = 0u;
+  q.plan->span_log2 = span_log2;
+  q.plan->lane_cap = lane_cap;
+  q.plan->blocks = (uint32_t)((waves + kWaves - 1u) / kWaves);
+}
+
+// the whole build for at most kScanTile events (one block)
+__global__ void __launch_bounds__(kScanThreads) k_queue_small(QueueArgs q) {
+  uint32_t ph[kScanItems], before, tp, tc;
+  block_counts(q, 0, ph, before, tp, tc);
+  write_offsets(q, 0, ph, before);
+  if (threadIdx.x == 0) plan_queue(q, tp, tc);
 }
 
 // pass 1: per-block totals
 __global__ void __launch_bounds__(kScanThreads) k_queue_totals(QueueArgs q) {
-  __shared__ uint32_t s_c[kScanThreads / 64 + 1];
-  __shared__ unsigned long long s_p[kScanThreads / 64 + 1];
-  const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-  uint32_t c = 0;
-  unsigned long long ph = 0;
-#pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    uint32_t cc, pp;
-    event_counts(q, base + i, cc, pp);
-    c += cc;
-    ph += pp;
-  }
-  uint32_t tc;
-  unsigned long long tp;
-  block_excl_scan<uint32_t>(c, s_c, tc);
-  block_excl_scan<unsigned long long>(ph, s_p, tp);
+  uint32_t ph[kScanItems], before, tp, tc;
+  block_counts(q, (int64_t)blockIdx.x * kScanTile, ph, before, tp, tc);
   if (threadIdx.x == 0) {
     q.block_chunks[blockIdx.x] = tc;
     q.block_photons[blockIdx.x] = tp;
   }
 }
 
-// pass 2: scan of the block totals (one block), grand totals, cursor reset.
-// The work-item total is summed in 64 bits: a launch of more than
-// q.max_chunks items (which the 32-bit offsets and cursor cannot number)
-// sets error bit 4 and gets a total of 0, so the transport takes nothing.
-__global__ void __launch_bounds__(kScanThreads) k_queue_blocks(QueueArgs q) {
-  __shared__ uint32_t s_c[kScanThreads / 64 + 1];
-  __shared__ unsigned long long s_p[kScanThreads / 64 + 1];
-  uint64_t carry_c = 0;
-  unsigned long long carry_p = 0;
-  for (int b0 = 0; b0 < q.n_blocks; b0 += kScanThreads) {
-    const int b = b0 + threadIdx.x;
-    const uint32_t c = b < q.n_blocks ? q.block_chunks[b] : 0u;
+// pass 2: scan of the block totals and grand totals (one wave)
+__global__ void __launch_bounds__(64) k_queue_blocks(QueueArgs q) {
+  uint64_t chunks = 0;
+  unsigned long long photons = 0;
+  for (int b0 = 0; b0 < q.n_blocks; b0 += 64) {
+    const int b = b0 + (int)threadIdx.x;
+    const uint64_t c = b < q.n_blocks ? q.block_chunks[b] : 0u;
     const unsigned long long p = b < q.n_blocks ? q.block_photons[b] : 0ull;
-    uint32_t tc;
-    unsigned long long tp;
-    const uint32_t ec = block_excl_scan<uint32_t>(c, s_c, tc);
-    const unsigned long long ep = block_excl_scan<unsigned long long>(p, s_p, tp);
-    if (b < q.n_blocks) {
-      q.block_chunks[b] = (uint32_t)(carry_c + ec);
-      q.block_photons[b] = carry_p + ep;
-    }
-    carry_c += tc;
-    carry_p += tp;
+    const uint64_t ic = wave_incl_scan(c);
+    const unsigned long long ip = wave_incl_scan(p);
+    if (b < q.n_blocks) q.block_photons[b] = photons + ip - p;
+    chunks += __shfl(ic, 63, 64);
+    photons += __shfl(ip, 63, 64);
   }
-  if (threadIdx.x == 0) {
-    const bool over = carry_c > q.max_chunks;
-    if (over) atomicOr(q.error_flag, 4u);
-    q.chunk_off[q.n_events] = over ? 0u : (uint32_t)carry_c;
-    q.photon_off[q.n_events] = carry_p;
-    *q.cursor = 0u;
-  }
+  if (threadIdx.x == 0) plan_queue(q, photons, chunks);
 }
 
 // pass 3: per-event exclusive offsets
 __global__ void __launch_bounds__(kScanThreads) k_queue_offsets(QueueArgs q) {
-  __shared__ uint32_t s_c[kScanThreads / 64 + 1];
-  __shared__ unsigned long long s_p[kScanThreads / 64 + 1];
-  const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-  uint32_t cc[kScanItems], pp[kScanItems];
-  uint32_t c = 0;
-  unsigned long long ph = 0;
-#pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    event_counts(q, base + i, cc[i], pp[i]);
-    c += cc[i];
-    ph += pp[i];
-  }
-  uint32_t tc;
-  unsigned long long tp;
-  uint32_t oc = block_excl_scan<uint32_t>(c, s_c, tc) + q.block_chunks[blockIdx.x];
-  unsigned long long op =
-      block_excl_scan<unsigned long long>(ph, s_p, tp) + q.block_photons[blockIdx.x];
-#pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    const int64_t e = base + i;
-    if (e < q.n_events) {
-      q.chunk_off[e] = oc;
-      q.photon_off[e] = op;
-    }
-    oc += cc[i];
-    op += pp[i];
-  }
+  const int64_t base = (int64_t)blockIdx.x * kScanTile;
+  uint32_t ph[kScanItems], before, tp, tc;
+  block_counts(q, base, ph, before, tp, tc);
+  write_offsets(q, base, ph, q.block_photons[blockIdx.x] + before);
 }
 
 hipError_t launch_queue_build(const QueueArgs& q, hipStream_t s) {
-  if (q.n_blocks <= 0) return hipErrorInvalidValue;
+  if (q.n_blocks <= 0 || q.n_waves == 0u) return hipErrorInvalidValue;
+  if (q.n_blocks == 1) {
+    hipLaunchKernelGGL(k_queue_small, dim3(1), dim3(kScanThreads), 0, s, q);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_queue_totals, dim3(q.n_blocks), dim3(kScanThreads), 0, s, q);
-  hipLaunchKernelGGL(k_queue_blocks, dim3(1), dim3(kScanThreads), 0, s, q);
+  hipLaunchKernelGGL(k_queue_blocks, dim3(1), dim3(64), 0, s, q);
   hipLaunchKernelGGL(k_queue_offsets, dim3(q.n_blocks), dim3(kScanThreads), 0, s, q);
   return hipGetLastError();
 }
@@ -165,20 +198,21 @@ hipError_t launch_queue_build(const QueueArgs& q, hipStream_t s) {
 // ------------------------------------------------------------ tallies
 
 // Counter-mode initial direction of photon k: photon 0 takes the driver's
-// first direction (|2u-1| > 0.01, main/hybridMANTIS_c_ver1_0.c:257-277),
-// the others the direction algo() draws at the previous photon's end
-// (main/kernel_cuda_c_ver1_0.cu:578-602) followed by the RoughSurface draws
-// of the (never read) initial normal.
+// first direction (|2u-1| > 0.01 by rejection,
+// main/hybridMANTIS_c_ver1_0.c:257-277), the others the direction algo()
+// draws at the previous photon's end (main/kernel_cuda_c_ver1_0.cu:578-602)
+// followed by the RoughSurface draws of the (never read) initial normal.
 __device__ __forceinline__ void counter_initial_dir(CounterRng& rng, Photon& p,
                                                     uint32_t k, const ColumnGeom& g) {
-  if (k == 0) {
-    emit_first_dir(rng, p, g);
-  } else {
-    emit_dir(rng, p, g);
-    if (g.beta > 0.0f) {
-      (void)rng.u();
-      (void)rng.u();
-    }
+  float r = rng.u() * 2.0f - 1.0f;
+  if (k == 0)
+    while (fabsf(r) <= 0.01f) r = rng.u() * 2.0f - 1.0f;
+  p.uz = r;
+  azimuth<MathDevice>(fd2_sqrt_01(1.0f - r * r), rng, p.ux, p.uy);
+  renorm(p.ux, p.uy, p.uz, g);
+  if (k != 0 && g.beta > 0.0f) {
+    (void)rng.u();
+    (void)rng.u();
   }
 }
 
@@ -193,10 +227,11 @@ __device__ __forceinline__ void counter_initial_dir(CounterRng& rng, Photon& p,
 #define FD2_WAVES_PER_EU 6
 #endif
 // With several geometries per launch (the geometry table in LDS, read per
-// lane) the kernel needs more registers and keeps 4 waves per SIMD.
+// lane, and a geometry index per photon) and with records the LDS holds 5.
 #if FD2_WAVES_PER_EU > 0
 #define FD2_TRANSPORT_ATTR \
-  __attribute__((amdgpu_waves_per_eu(MULTI ? 4 : FD2_WAVES_PER_EU, MULTI ? 4 : FD2_WAVES_PER_EU)))
+  __attribute__((amdgpu_waves_per_eu(MULTI || REC ? FD2_WAVES_PER_EU - 1 : FD2_WAVES_PER_EU, \
+                                     MULTI || REC ? FD2_WAVES_PER_EU - 1 : FD2_WAVES_PER_EU)))
 #else
 #define FD2_TRANSPORT_ATTR
 #endif
@@ -304,7 +339,7 @@ __device__ __forceinline__ void q_put(uint32_t* w, const Photon& p, const Counte
   w[12 * S] = r.s3;
   w[13 * S] = ev;
   if (MULTI) w[14 * S] = gi;
-  if (REC) w[15 * S] = k;
+  if (REC) w[(14 + MULTI) * S] = k;
 }
 
 template <bool MULTI, bool REC, int S>
@@ -326,7 +361,7 @@ __device__ __forceinline__ void q_get(const uint32_t* w, Photon& p, CounterRng& 
   r.s3 = w[12 * S];
   ev = w[13 * S];
   gi = MULTI ? w[14 * S] : 0u;
-  k = REC ? w[15 * S] : 0u;
+  k = REC ? w[(14 + MULTI) * S] : 0u;
 }
 
 // Per-wave gap queue and backlog in HBM (kQSlots entries of kQWords words).
@@ -378,6 +413,65 @@ __device__ __forceinline__ T load_uniform(const void* p) {
   return c;
 }
 
+// Event of photon g of the launch: the largest e with photon_off[e] <= g
+// (skips events without photons).  Each round the 64 lanes (all active) probe
+// 64 points of [lo, hi) with one vector load, and the wave keeps the step
+// after the last probe at or below g -- 3 rounds for 2e5 events where a
+// binary search makes 18 dependent loads.
+__device__ __forceinline__ uint32_t event_of(const unsigned long long* __restrict__ photon_off,
+                                             int64_t n_events, uint64_t g, int lane) {
+  int64_t lo = 0, hi = n_events;
+  while (hi - lo > 1) {
+    const int64_t step = (hi - lo + 63) >> 6;
+    const int64_t pos = lo + (int64_t)lane * step;
+    const bool le = pos < hi && photon_off[pos] <= g;
+    const unsigned long long m = __ballot(le);
+    lo += (int64_t)(63 - __clzll(m)) * step;
+    hi = min(hi, lo + step);
+  }
+  return (uint32_t)lo;
+}
+
+// Events of photons g .. g + n - 1 (n <= 64, lane j's of photon g + j), the
+// first of event e0, where they span several (reference event buffers hold
+// about two photons per event).  A round reads the starts of the 64 events
+// after the current one and every unresolved lane counts those at or before
+// its photon (a binary search over the lanes' values); a window without a
+// photon's event (a long run of empty events) is left by a search.
+__device__ __forceinline__ uint32_t events_of(const unsigned long long* __restrict__ photon_off,
+                                              int64_t n_events, uint32_t e0, uint64_t g,
+                                              uint32_t n, int lane) {
+  uint32_t e = e0, done = 0;
+  while (done < n) {
+    const uint64_t first = g + done;
+    const int64_t i = (int64_t)e0 + 1 + lane;
+    uint32_t v = 0xffffffffu;  // start of event i, in photons after `first`
+    if (i <= n_events) {
+      const uint64_t o = photon_off[i];
+      v = o <= first ? 0u : (uint32_t)min(o - first, (uint64_t)0xffffffffu);
+    }
+    const bool open = (uint32_t)lane >= done && (uint32_t)lane < n;
+    const uint32_t rel = (uint32_t)lane - done;
+    uint32_t at = 0;
+#pragma unroll
+    for (uint32_t s = 32; s != 0u; s >>= 1) {
+      const uint32_t t = (uint32_t)__shfl((int)v, (int)(at + s - 1u), 64);
+      if (t <= rel) at += s;
+    }
+    const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+    const bool found = open && last > rel;
+    if (found) e = e0 + at;
+    const uint32_t m = (uint32_t)__popcll(__ballot(found));
+    if (m != 0u) {
+      done += m;
+      e0 = (uint32_t)__builtin_amdgcn_readlane((int)e, (int)(done - 1u));
+    } else {
+      e0 = event_of(photon_off, n_events, first, lane);
+    }
+  }
+  return e;
+}
+
 // Persistent transport.  A wave keeps the state of its lanes in wave-uniform
 // masks: step_m (a photon that takes in-column passes), wall_m (a photon that
 // waits for the wall's Fresnel branch), end_m (a photon that has ended and is
@@ -385,7 +479,8 @@ __device__ __forceinline__ T load_uniform(const void* p) {
 //
 //   serve   once refill_lanes lanes do not step: tally the ended photons, put
 //           the waiting ones into the wave's LDS queue and fill the free lanes
-//           (LDS queue, HBM backlog, then new photons of the work queue)
+//           (LDS queue, HBM backlog, then new photons of the work queue,
+//           which all lanes start together into the LDS queue)
 //   pass    one in-column pass of the stepping lanes
 //   wall    once 64 photons wait (in lanes and in the LDS queue): the branch
 //           runs with all 64 lanes, up to a refraction out of the column;
@@ -396,24 +491,25 @@ __device__ __forceinline__ T load_uniform(const void* p) {
 //           were stepping go to the HBM backlog meanwhile
 //
 // The LDS queue holds waiting photons from its bottom up (n_wall) and photons
-// ready to step from its top down (n_ready).  n_wall + n_ready <= 64 outside
-// of serve: a waiting photon enters from a lane that then takes a ready one,
-// and the wall phase swaps at most as many in as it takes out.  The 8 slots
-// above 64 let a lane write before it reads.  Moving the stepping photons to
+// ready to step from its top down (n_ready).  n_wall + n_ready <= kLdsCap
+// outside of serve: a waiting photon enters from a lane that then takes a
+// ready one, and the wall phase swaps at most as many in as it takes out.  The
+// slots above kLdsCap let a lane write before it reads.  Moving the stepping photons to
 // HBM and back around every wall phase, as the gap phase still does, took
 // 1.2e11 of 1.5e11 bytes of a mono25x50 launch and a wait for HBM at each
 // refill.
 //
-// Draining (no chunk, ready photon or backlog left), and throughout when
-// there are no queues (wave_queue null), waiting photons stay in their lanes:
-// the branch and the flights run where they are, with the other lanes masked
-// off, once at least as many wait as step (without queues: park_lanes).
+// Draining (no span, ready photon or backlog left), and throughout when
+// there are no queues (wave_queue null) or a launch has less than 64 photons
+// per wave, waiting photons stay in their lanes: the branch and the flights
+// run where they are, with the other lanes masked off, once at least as many
+// wait as step (without queues: park_lanes).
 //
 // Every photon keeps its own state and random stream, so the results are the
 // same in either mode and in any order.
 //
-// `geoms_in`, `events` and `chunk_off` are a.geoms, a.events and
-// a.chunk_off again, as parameters of their own: the kernel never writes
+// `geoms_in`, `events` and `photon_off` are a.geoms, a.events and
+// a.photon_off again, as parameters of their own: the kernel never writes
 // these tables (only the tallies the geometries point to), and saying so
 // (__restrict__) lets the compiler read them with scalar loads where they
 // are uniform instead of reloading them with vector loads around every
@@ -421,26 +517,23 @@ __device__ __forceinline__ T load_uniform(const void* p) {
 template <bool MULTI, bool REC, bool RADIAL>
 __global__ void __launch_bounds__(kTransportThreads) FD2_TRANSPORT_ATTR
 k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
-            const fd2_event* __restrict__ events, const uint32_t* __restrict__ chunk_off) {
+            const fd2_event* __restrict__ events,
+            const unsigned long long* __restrict__ photon_off) {
   // With several geometries a lane's geometry is its own, so their constants
   // cannot be scalar loads: the table goes to LDS instead.
-  static_assert(sizeof(GeomDev) % 4 == 0, "GeomDev copied as words");
-  __shared__ __align__(16) uint32_t s_geom_words[MULTI ? FD2_MAX_GEOMS * sizeof(GeomDev) / 4 : 2];
+  static_assert(sizeof(GeomDev) % 8 == 0, "GeomDev copied as words");
+  if (blockIdx.x >= a.plan->blocks) return;  // a small launch (plan_queue)
+  extern __shared__ __align__(16) uint32_t s_dyn[];  // geometry table (MULTI), then PRF tiles
+  const int geom_words = MULTI ? a.n_geoms * (int)(sizeof(GeomDev) / 4) : 0;
   if (MULTI) {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(geoms_in);
-    const int nw = a.n_geoms * (int)(sizeof(GeomDev) / 4);
-    for (int i = threadIdx.x; i < nw; i += blockDim.x) s_geom_words[i] = src[i];
+    for (int i = threadIdx.x; i < geom_words; i += blockDim.x) s_dyn[i] = src[i];
   }
-  const GeomDev* __restrict__ geoms =
-      MULTI ? reinterpret_cast<const GeomDev*>(s_geom_words) : geoms_in;
+  const GeomDev* __restrict__ geoms = MULTI ? reinterpret_cast<const GeomDev*>(s_dyn) : geoms_in;
+  uint32_t* s_tile = s_dyn + geom_words;  // n_tiles x tile_side^2
   __shared__ uint32_t s_cnt[FD2_MAX_GEOMS * kCounters];
-  // the next photons of the wave's chunk, started ahead with all lanes:
-  // photon start_base + j has its first direction in words 0-2 of slot j
-  // and its random stream (after the initial draws) in words 3-6
-  __shared__ uint32_t s_start[kTransportThreads / 64][kStartWords][64];
   // the waves' LDS queues, word-major
-  __shared__ uint32_t s_queue[kTransportThreads / 64][MULTI || REC ? 16 : 14][kWallSlots];
-  extern __shared__ uint32_t s_tile[];  // n_tiles x tile_side^2
+  __shared__ uint32_t s_queue[kTransportThreads / 64][14 + MULTI + REC][kWallSlots];
   for (int i = threadIdx.x; i < a.n_geoms * kCounters; i += blockDim.x) s_cnt[i] = 0;
   for (int i = threadIdx.x; i < a.n_tiles * a.tile_side * a.tile_side; i += blockDim.x)
     s_tile[i] = 0;
@@ -448,7 +541,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
 
   // per-lane run of detections of one event (event, count), added to the
   // event's history count when the lane's detections move on to another
-  // event (photons of a chunk share their event); in LDS, as it is touched
+  // event (consecutive photons share their event); in LDS, as it is touched
   // only when a photon ends
   __shared__ uint32_t s_run[kTransportThreads][2];
   uint32_t* run = s_run[threadIdx.x];
@@ -459,11 +552,10 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
   // the wave's index in the block, uniform across the wave: the compiler
   // then keeps the wave's queue and LDS bases in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  // wave-uniform work pool: photons [pool_next, pool_end) of event pool_ev;
-  // those in [start_base, start_end) (up to 64) are started in s_start
-  int64_t pool_ev = 0;
-  int32_t pool_next = 0, pool_end = 0, start_base = 0, start_end = 0;
-  uint32_t (*start)[64] = s_start[wave];
+  // wave-uniform work pool: the launch's photons [pool_next, pool_end), the
+  // first of event pool_ev
+  uint64_t pool_next = 0, pool_end = 0;
+  uint32_t pool_ev = 0;
   bool pool_done = false;
 
   Photon p;
@@ -480,7 +572,11 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
   if (a.wave_queue)
     wq = a.wave_queue + (size_t)(blockIdx.x * (kTransportThreads / 64) + wave) *
                             (kQWords * kQSlots);
-  const bool queued = a.wave_queue != nullptr;
+  const uint32_t lane_cap = a.plan->lane_cap;
+  const bool queued = a.wave_queue != nullptr && lane_cap == 64u;
+  const uint32_t park = a.wave_queue ? 0u : (uint32_t)a.park_lanes;
+  const uint32_t serve_at = min((uint32_t)a.refill_lanes, lane_cap);
+  const unsigned long long use_m = lane_cap == 64u ? ~0ull : (1ull << lane_cap) - 1ull;
 
   // the launch's arguments, read again where they are needed: held over the
   // loop they would take the scalar registers of its lane masks
@@ -529,8 +625,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     {
       const unsigned long long waiting = drain || !queued ? wall_m : 0ull;
       const bool due = !drain || end_m != 0ull || n_wall != 0u || n_gap != 0u;
-      if (step_m == 0ull ||
-          (due && (int)count(~(step_m | waiting)) >= a.refill_lanes)) {
+      if (step_m == 0ull || (due && count(use_m & ~(step_m | waiting)) >= serve_at)) {
         if (end_m != 0ull) finish(end_m);
         end_m = 0ull;
         if (queued && !drain && n_wall + count(wall_m) < 64u) {
@@ -545,8 +640,8 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
             take_ready(~(step_m | wall_m));
           }
         }
-        take_ready(~(step_m | wall_m));
-        unsigned long long need = ~(step_m | wall_m);
+        take_ready(use_m & ~(step_m | wall_m));
+        unsigned long long need = use_m & ~(step_m | wall_m);
         if (need != 0ull && n_back != 0u) {
           __threadfence_block();  // the wave's queue stores are complete before its loads
           const uint32_t t = min(count(need), n_back);
@@ -557,94 +652,54 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
                                        lane_ev, gi, lane_k);
           n_back -= t;
           step_m |= __ballot(got);
-          need = ~(step_m | wall_m);
+          need = use_m & ~(step_m | wall_m);
         }
         while (need != 0ull && !pool_done) {
           const TransportArgs b = args();
-          const uint32_t chunk = 1u << b.chunk_log2;
           if (pool_next >= pool_end) {
             uint32_t c = 0;
-            if (lane == 0) c = atomicAdd(b.cursor, 1u);
+            if (lane == 0) c = atomicAdd(&b.plan->cursor, 1u);
             c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
-            if (c >= chunk_off[b.n_events]) {
+            const uint64_t total = photon_off[b.n_events];
+            const uint32_t span_log2 = b.plan->span_log2;
+            pool_next = (uint64_t)c << span_log2;
+            if (pool_next >= total) {
               pool_done = true;
               break;
             }
-            // largest e with chunk_off[e] <= c (skips events without photons):
-            // each round the 64 lanes (all active here) probe 64 points of
-            // [lo, hi) with one vector load, and the wave keeps the step after
-            // the last probe at or below c -- 3 rounds for 2e5 events where a
-            // binary search makes 18 dependent loads
-            int64_t lo = 0, hi = b.n_events;
-            while (hi - lo > 1) {
-              const int64_t step = (hi - lo + 63) >> 6;
-              const int64_t pos = lo + (int64_t)lane * step;
-              const bool le = pos < hi && chunk_off[pos] <= c;
-              const unsigned long long m = __ballot(le);
-              lo += (int64_t)(63 - __clzll(m)) * step;
-              hi = min(hi, lo + step);
-            }
-            pool_ev = lo;
-            const int32_t n_ph = events[lo].N;
-            pool_next = (int32_t)((c - chunk_off[lo]) << b.chunk_log2);
-            pool_end = min(n_ph, pool_next + (int32_t)chunk);
-            if (lane == 0) {
-              const uint32_t gg = MULTI ? events[lo].geom : 0u;
-              atomicAdd(&s_cnt[gg * kCounters + FD2_C_GENERATED], (uint32_t)(pool_end - pool_next));
-            }
-            start_end = pool_next;
+            pool_end = min(total, pool_next + (1ull << span_log2));
+            pool_ev = event_of(photon_off, b.n_events, pool_next, lane);
           }
-          if (pool_next >= start_end) {
-            // Seeding a stream (Philox) and drawing the first direction are
-            // long; every lane starts one of the next 64 photons of the chunk
-            // here, at full width, instead of the few lanes that take photons
-            // in a pass.
-            start_base = pool_next;
-            start_end = min(pool_end, pool_next + 64);
-            if (start_base + lane < start_end) {
-              const uint32_t k = (uint32_t)(start_base + lane);
-              CounterRng r;
-              Photon q;
-              const uint64_t event_base = b.event_base_dev ? *b.event_base_dev : b.event_base;
-              r.seed(b.seed, event_base + (uint64_t)pool_ev, k);
-              if constexpr (MULTI)
-                counter_initial_dir(r, q, k, geoms[events[pool_ev].geom]);
-              else
-                counter_initial_dir(r, q, k, load_uniform<ColumnGeom>(geoms_in));
-              start[0][lane] = __float_as_uint(q.ux);
-              start[1][lane] = __float_as_uint(q.uy);
-              start[2][lane] = __float_as_uint(q.uz);
-              start[3][lane] = r.s0;
-              start[4][lane] = r.s1;
-              start[5][lane] = r.s2;
-              start[6][lane] = r.s3;
+          // Seeding a stream (Philox) and drawing the first direction are
+          // long: every lane starts one of the next photons here, as many as
+          // the LDS queue has room for.
+          const uint32_t n = (uint32_t)min((uint64_t)min((uint32_t)kLdsCap - n_wall, 64u), pool_end - pool_next);
+          uint32_t e = pool_ev;
+          if (photon_off[pool_ev + 1u] - pool_next < n)
+            e = events_of(photon_off, b.n_events, pool_ev, pool_next, n, lane);
+          if ((uint32_t)lane < n) {
+            const fd2_event ev = events[e];
+            const uint32_t k = (uint32_t)(pool_next + (uint32_t)lane - photon_off[e]);
+            CounterRng r;
+            Photon q;
+            start_photon(q, ev);
+            const uint64_t event_base = b.event_base_dev ? *b.event_base_dev : b.event_base;
+            r.seed(b.seed, event_base + (uint64_t)e, k);
+            if constexpr (MULTI) {
+              counter_initial_dir(r, q, k, geoms[ev.geom]);
+              atomicAdd(&s_cnt[ev.geom * kCounters + FD2_C_GENERATED], 1u);
+            } else {
+              counter_initial_dir(r, q, k, load_uniform<ColumnGeom>(geoms_in));
+              if (lane == 0) atomicAdd(&s_cnt[FD2_C_GENERATED], n);
             }
-            // lanes read other lanes' slots below; the wave's LDS accesses
-            // complete in order
-            __builtin_amdgcn_wave_barrier();
+            q_put<MULTI, REC, kWallSlots>(lq + (uint32_t)kWallSlots - n + lane, q, r, e,
+                                          MULTI ? ev.geom : 0u, k);
           }
-          const int avail = start_end - pool_next;  // started, not yet taken
-          const int rank = (int)rank_below(need);
-          const bool got = in(need) && rank < avail;
-          if (got) {
-            const fd2_event ev = events[pool_ev];
-            gi = MULTI ? ev.geom : 0u;
-            const uint32_t k = (uint32_t)(pool_next + rank);
-            const uint32_t j = k - (uint32_t)start_base;
-            start_photon(p, ev);
-            p.ux = __uint_as_float(start[0][j]);
-            p.uy = __uint_as_float(start[1][j]);
-            p.uz = __uint_as_float(start[2][j]);
-            rng.s0 = start[3][j];
-            rng.s1 = start[4][j];
-            rng.s2 = start[5][j];
-            rng.s3 = start[6][j];
-            lane_ev = (uint32_t)pool_ev;
-            lane_k = k;
-          }
-          pool_next += min((int)count(need), avail);
-          step_m |= __ballot(got);
-          need = ~(step_m | wall_m);
+          n_ready = n;
+          pool_next += n;
+          pool_ev = (uint32_t)__builtin_amdgcn_readlane((int)e, (int)(n - 1u));
+          take_ready(need);
+          need = use_m & ~(step_m | wall_m);
         }
         drain = pool_done && n_ready == 0u && n_back == 0u;
         if (drain && queued && need != 0ull && (n_wall | n_gap) != 0u) {
@@ -707,7 +762,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     const bool full = !in_place && n_wall + n_lane >= 64u;
     const bool place =
         in_place && n_lane != 0u &&
-        (n_step == 0u || (queued ? n_lane >= n_step : (int)n_lane >= args().park_lanes));
+        (n_step == 0u || n_lane >= (park != 0u ? park : n_step));
     if (full || place) {
       progress = true;
       if (end_m != 0ull) finish(end_m);
@@ -830,9 +885,10 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
 
 template <bool MULTI, bool REC, bool RADIAL>
 static void launch_one(const TransportArgs& a, dim3 grid, hipStream_t s) {
-  const size_t smem = (size_t)a.n_tiles * a.tile_side * a.tile_side * sizeof(uint32_t);
+  const size_t smem =
+      transport_dynamic_lds(MULTI, a.n_geoms, (size_t)a.n_tiles * a.tile_side * a.tile_side);
   hipLaunchKernelGGL((k_transport<MULTI, REC, RADIAL>), grid, dim3(kTransportThreads), smem, s, a,
-                     a.geoms, a.events, a.chunk_off);
+                     a.geoms, a.events, a.photon_off);
 }
 
 hipError_t launch_transport(const TransportArgs& a, bool multi, bool record,
@@ -870,7 +926,6 @@ static size_t static_lds_of() {
 }
 
 size_t transport_static_lds() {
-  // the several-geometry variants hold the geometry table: the largest
   const size_t a = static_lds_of<true, false, false>();
   const size_t b = static_lds_of<true, true, false>();
   const size_t c = static_lds_of<true, false, true>();

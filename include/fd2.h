@@ -158,11 +158,11 @@ int fd2_sync(fd2_ctx *ctx);
 /* fd2_submit_device without any allocation, for callers that cannot call
  * hipMalloc (code under stream/graph capture, tight serving loops,
  * harnesses that forbid it).  No counterpart in the reference.  The work
- * queue's scratch (cursor, error flag, block totals, per-event chunk and
- * photon offsets) lives in a static device array of the library sized for
- * FD2_NOALLOC_MAX_EVENTS events (12.6 MB per GPU, held until the process
- * ends); the transport runs in park-in-place mode (no per-wave photon
- * queues), which gives the same photons as fd2_submit_device.  The events
+ * queue's scratch (plan, error flag, block totals, per-event photon
+ * offsets) lives in a static device array of the library sized for
+ * FD2_NOALLOC_MAX_EVENTS events (8.4 MB per GPU, held until the process
+ * ends); the per-wave photon queues are those that fd2_create made.  The
+ * photons are those of fd2_submit_device.  The events
  * are in device memory (d_events, valid for the call); the tallies
  * accumulate in the context as for every submit, and the events take the
  * next n event numbers.  Synchronous: returns the launch's status
