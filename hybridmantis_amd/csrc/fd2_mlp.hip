@@ -5,7 +5,7 @@
 // Layout (row-major everywhere, feature dims padded to multiples of 16):
 //   X0 [B x 32] bf16 (5 features + zeros)
 //   W0 [32 x 256], W1, W2 [256 x 256], W3 [256 x 80] (65 outputs + zeros)
-//   Zl = A(l-1) Wl + bl (FP32, kept for backward), Al = bf16(gelu(Zl))
+//   Zl = A(l-1) Wl + bl (FP32), Al = bf16(gelu(Zl))
 //   output logits Z4 [B x 80]: column 0 detection logit, 1..64 radial logits
 // Loss per sample: BCE(sigmoid(z0), y0) + w * CE(softmax(z1..64), q) with
 // y0 the detected fraction, q the radial distribution and w = 1 when the
@@ -29,6 +29,7 @@
 namespace fd2mlp {
 
 typedef short short4_ __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_ __attribute__((ext_vector_type(8)));
 typedef float float4_ __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint16_t f2bf(float f) {
@@ -52,79 +53,49 @@ __device__ __forceinline__ float gelu_grad(float x) {
   return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * du;
 }
 
-// ------------------------------------------------------------- GEMM
+// ------------------------------------------------- layer-by-layer forward
 //
-// C[M x N] = op(A)[M x K] * op(B)[K x N], K a multiple of 16.
-// TA: A is stored transposed ([K x M]); TB: B stored transposed ([N x K]).
-// 256 threads = 4 waves compute a 64 x 64 tile; each wave a 32 x 32 quarter
-// as 2 x 2 blocks of v_mfma_f32_16x16x16bf16_1k.  Operand tiles of 64 x 16
-// go through LDS so every layout is read with coalesced 8-byte loads.
-// Split-K: blockIdx.z takes K range [z*kchunk, (z+1)*kchunk).
-enum Epilogue : int {
-  kStoreF32 = 0,      // C (+bias) -> outf; gelu(C) as bf16 -> outb if set
-  kAtomicF32 = 1,     // outf += C (split-K weight gradients)
-  kGeluGradBf16 = 2,  // outb = bf16(C * gelu'(Z)) and bias grad += colsum
-};
-
+// outf[M x N] = A[M x K] B[K x N] + bias, and outb = bf16(gelu(outf)) if set;
+// K a multiple of 16, all row-major.  The forward that fd2_mlp_logits offers
+// beside the fused one.  256 threads = 4 waves compute a 64 x 64 tile; each
+// wave a 32 x 32 quarter as 2 x 2 blocks of v_mfma_f32_16x16x16bf16_1k.
+// Operand tiles of 64 x 16 go through LDS so that both are read with
+// coalesced 8-byte loads.
 struct GemmArgs {
   const uint16_t* A;
   const uint16_t* B;
   int M, N, K;
-  int lda, ldb;        // leading dims of the stored arrays
-  int kchunk;
-  const float* bias;   // kStoreF32
-  float* outf;         // kStoreF32 / kAtomicF32 (ld = N)
-  uint16_t* outb;      // kStoreF32 (gelu) / kGeluGradBf16 (ld = ldo)
-  const float* Z;      // kGeluGradBf16: pre-activations (ld = N)
-  float* dbias;        // kGeluGradBf16: column sums of the product
-  int ldo;
+  const float* bias;
+  float* outf;
+  uint16_t* outb;
 };
 
-template <bool TA, bool TB, int EPI>
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
   __shared__ uint16_t As[64][16 + 4];
   __shared__ uint16_t Bs[16][64 + 4];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
   const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-  const int kbeg = blockIdx.z * g.kchunk;
-  const int kend = min(g.K, kbeg + g.kchunk);
   float4_ acc[2][2];
   for (int i = 0; i < 2; ++i)
     for (int j = 0; j < 2; ++j) acc[i][j] = float4_{0.f, 0.f, 0.f, 0.f};
 
-  for (int k0 = kbeg; k0 < kend; k0 += 16) {
-    // A tile: 64 rows x 16 k
-    if (!TA) {
+  for (int k0 = 0; k0 < g.K; k0 += 16) {
+    {  // A tile: 64 rows x 16 k
       const int r = t >> 2, kk = (t & 3) * 4;
       const int gm = m0 + r;
       uint16_t v[4] = {0, 0, 0, 0};
       if (gm < g.M) {
-        const uint2 q = *reinterpret_cast<const uint2*>(g.A + (size_t)gm * g.lda + k0 + kk);
+        const uint2 q = *reinterpret_cast<const uint2*>(g.A + (size_t)gm * g.K + k0 + kk);
         v[0] = q.x & 0xFFFF; v[1] = q.x >> 16; v[2] = q.y & 0xFFFF; v[3] = q.y >> 16;
       }
       for (int j = 0; j < 4; ++j) As[r][kk + j] = v[j];
-    } else {
-      const int kk = t >> 4, r = (t & 15) * 4;
-      const int gm = m0 + r;
-      const uint16_t* src = g.A + (size_t)(k0 + kk) * g.lda + gm;
-      for (int j = 0; j < 4; ++j) As[r + j][kk] = (gm + j < g.M) ? src[j] : (uint16_t)0;
     }
-    // B tile: 16 k x 64 cols
-    if (!TB) {
+    {  // B tile: 16 k x 64 cols
       const int kk = t >> 4, c = (t & 15) * 4;
       const int gn = n0 + c;
-      const uint16_t* src = g.B + (size_t)(k0 + kk) * g.ldb + gn;
+      const uint16_t* src = g.B + (size_t)(k0 + kk) * g.N + gn;
       for (int j = 0; j < 4; ++j) Bs[kk][c + j] = (gn + j < g.N) ? src[j] : (uint16_t)0;
-    } else {
-      const int c = t >> 2, kk = (t & 3) * 4;
-      const int gn = n0 + c;
-      uint16_t v[4] = {0, 0, 0, 0};
-      if (gn < g.N) {
-        const uint2 q = *reinterpret_cast<const uint2*>(g.B + (size_t)gn * g.ldb + k0 + kk);
-        v[0] = q.x & 0xFFFF; v[1] = q.x >> 16; v[2] = q.y & 0xFFFF; v[3] = q.y >> 16;
-      }
-      for (int j = 0; j < 4; ++j) Bs[kk + j][c] = v[j];
     }
     __syncthreads();
     // fragments: A lane l -> row l%16, k 4*(l/16)..+3; B lane l -> col l%16
@@ -143,42 +114,17 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
   }
   // D lane l: col l%16, rows 4*(l/16)+r
   const int lc = lane & 15, lr4 = (lane >> 4) * 4;
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < 2; ++i)
     for (int j = 0; j < 2; ++j) {
       const int col = n0 + wn + j * 16 + lc;
-      float colsum = 0.0f;
       for (int r = 0; r < 4; ++r) {
         const int row = m0 + wm + i * 16 + lr4 + r;
-        const float v = acc[i][j][r];
         if (row >= g.M || col >= g.N) continue;
-        if (EPI == kStoreF32) {
-          const float z = v + (g.bias ? g.bias[col] : 0.0f);
-          g.outf[(size_t)row * g.N + col] = z;
-          if (g.outb) g.outb[(size_t)row * g.ldo + col] = f2bf(gelu_f(z));
-        } else if (EPI == kAtomicF32) {
-          atomicAdd(&g.outf[(size_t)row * g.N + col], v);
-        } else {
-          const float d = v * gelu_grad(g.Z[(size_t)row * g.N + col]);
-          const uint16_t h = f2bf(d);
-          g.outb[(size_t)row * g.ldo + col] = h;
-          colsum += bf2f(h);
-        }
-      }
-      if (EPI == kGeluGradBf16 && g.dbias) {
-        // lanes l, l+16, l+32, l+48 share the column
-        colsum += __shfl_xor(colsum, 16, 64);
-        colsum += __shfl_xor(colsum, 32, 64);
-        if ((lane >> 4) == 0 && col < g.N) atomicAdd(&g.dbias[col], colsum);
+        const float z = acc[i][j][r] + g.bias[col];
+        g.outf[(size_t)row * g.N + col] = z;
+        if (g.outb) g.outb[(size_t)row * g.N + col] = f2bf(gelu_f(z));
       }
     }
-  }
-}
-
-template <bool TA, bool TB, int EPI>
-static hipError_t gemm(const GemmArgs& a, int splits, hipStream_t s) {
-  dim3 grid((a.N + 63) / 64, (a.M + 63) / 64, splits);
-  hipLaunchKernelGGL((k_gemm<TA, TB, EPI>), grid, dim3(256), 0, s, a);
-  return hipGetLastError();
 }
 
 // ----------------------------------------------------- elementwise kernels
@@ -189,79 +135,6 @@ __global__ void k_pack_inputs(const float* x, int n, uint16_t* x0) {
   if (i >= n * kIn) return;
   const int row = i / kIn, c = i % kIn;
   x0[(size_t)row * kInPad + c] = c < kFeat ? f2bf(x[(size_t)row * kFeat + c]) : (uint16_t)0;
-}
-
-// gather a minibatch: rows idx[b] of the resident data set, one wave per
-// row (lanes over the row's columns, so the copies are coalesced)
-__global__ void k_gather(const float* xs, const float* ys, const uint32_t* idx, int B,
-                         uint16_t* x0, float* y) {
-  const int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-  if (i >= B) return;
-  const uint32_t r = idx[i];
-  if (lane < kInPad)
-    x0[(size_t)i * kInPad + lane] = lane < kFeat ? f2bf(xs[(size_t)r * kFeat + lane]) : (uint16_t)0;
-  for (int c = lane; c < kTarget; c += 64) y[(size_t)i * kTarget + c] = ys[(size_t)r * kTarget + c];
-}
-
-// loss and dL/dZ4, one sample at a time per wave: lane k handles radial
-// logit k (z[1+k]); lane 0 also the detection logit.  dz -> bf16 [B x 80].
-// The column 0 and 1..64 bias gradients and the loss are summed over the
-// wave's samples in registers, then over the block's waves in LDS, and
-// added with one atomic per column and block: one atomic per sample and
-// column made 4096 x 65 float atomics meet on 65 addresses (142 us per
-// batch of 4096); 32 blocks of long per-wave loops took 69 us.
-constexpr int kHeadLossBlocks = 256;
-__global__ void __launch_bounds__(256) k_head_loss(const float* z4, const float* y, int B,
-                                                   uint16_t* dz, float* db3, float* loss) {
-  __shared__ float s_db[4][kOut];
-  __shared__ float s_loss[4];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int nw = gridDim.x * (blockDim.x >> 6);
-  const float invB = 1.0f / (float)B;
-  float db_r = 0.0f, db_0 = 0.0f, lsum = 0.0f;
-  for (int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; wave < B; wave += nw) {
-    const float* zr = z4 + (size_t)wave * kOutPad;
-    const float* yr = y + (size_t)wave * kTarget;
-    // radial softmax over 64 lanes
-    const float zl = zr[1 + lane];
-    float mx = zl;
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    const float e = expf(zl - mx);
-    float se = e;
-    for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
-    const float prob = e / se;
-    const float q = yr[1 + lane];
-    float qs = q;
-    for (int o = 32; o > 0; o >>= 1) qs += __shfl_xor(qs, o, 64);
-    const float wrad = qs > 0.0f ? 1.0f : 0.0f;
-    float ce = q > 0.0f ? -q * (zl - mx - logf(se)) : 0.0f;
-    for (int o = 32; o > 0; o >>= 1) ce += __shfl_xor(ce, o, 64);
-    const float gr = wrad * (prob - q) * invB;
-    uint16_t* dr = dz + (size_t)wave * kOutPad;
-    const uint16_t grb = f2bf(gr);
-    dr[1 + lane] = grb;
-    db_r += bf2f(grb);
-    if (lane < kOutPad - 1 - 64) dr[65 + lane] = 0;
-    if (lane == 0) {
-      const float z0 = zr[0], y0 = yr[0];
-      const float p = 1.0f / (1.0f + expf(-z0));
-      // BCE with logits: max(z,0) - z y + log(1 + e^-|z|)
-      const float bce = fmaxf(z0, 0.0f) - z0 * y0 + log1pf(expf(-fabsf(z0)));
-      const uint16_t g0 = f2bf((p - y0) * invB);
-      dr[0] = g0;
-      db_0 += bf2f(g0);
-      lsum += (bce + wrad * ce) * invB;
-    }
-  }
-  s_db[w][1 + lane] = db_r;
-  if (lane == 0) {
-    s_db[w][0] = db_0;
-    s_loss[w] = lsum;
-  }
-  __syncthreads();
-  const int t = threadIdx.x;
-  if (t < kOut) atomicAdd(&db3[t], (s_db[0][t] + s_db[1][t]) + (s_db[2][t] + s_db[3][t]));
-  if (t == 0) atomicAdd(loss, (s_loss[0] + s_loss[1]) + (s_loss[2] + s_loss[3]));
 }
 
 // logits -> [p_det, radial probabilities] (FP32 [n x 65])
@@ -281,23 +154,6 @@ __global__ void __launch_bounds__(256) k_head_probs(const float* z4, int n, floa
   if (lane == 0) orow[0] = 1.0f / (1.0f + expf(-zr[0]));
 }
 
-// Adam (Kingma & Ba 2015) on FP32 master weights; refreshes the bf16 copy
-// of weight matrices and clears the gradient.
-__global__ void k_adam(float* w, float* g, float* m, float* v, uint16_t* wb, int n,
-                       float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  w[i] = wi;
-  g[i] = 0.0f;
-  if (wb) wb[i] = f2bf(wi);
-}
-
 __global__ void k_to_bf16(const float* w, uint16_t* wb, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) wb[i] = f2bf(w[i]);
@@ -313,10 +169,14 @@ __global__ void k_zero(float* p, size_t n) {
 
 // Weight matrices in MFMA fragment order for the fused forward: layer l's
 // W [K x N] (row-major at kWOff[l] in the bf16 copy) is stored at the same
-// offset as the B fragments of v_mfma_f32_16x16x16bf16_1k, column block cb
-// (16 columns) by k step ks (16 k) by lane by element: lane 16 q + c holds
-// W[16 ks + 4 q + e][16 cb + c], e = 0..3.  One fragment is then 512
-// contiguous bytes, a lane's part one 8-byte load.  Bias slots are unused.
+// offset as the B fragments of v_mfma_f32_16x16x32_bf16, column block cb
+// (16 columns) by k step ks (32 k) by lane by element: lane 16 q + c holds
+// W[32 ks + 8 q + e][16 cb + c], e = 0..7.  One fragment is then 1024
+// contiguous bytes, a lane's part one 16-byte load.  Bias slots are unused.
+__device__ __forceinline__ size_t forward_slot(int K, int k, int n) {
+  const size_t frag = (size_t)(n >> 4) * (K >> 5) + (k >> 5);
+  return (frag * 64 + 16 * ((k & 31) >> 3) + (n & 15)) * 8 + (k & 7);
+}
 __global__ void k_fragment_weights(const uint16_t* __restrict__ wb, uint16_t* __restrict__ wt) {
   const int ks[4] = {kInPad, kHidden, kHidden, kHidden};
   const int ns[4] = {kHidden, kHidden, kHidden, kOutPad};
@@ -324,9 +184,7 @@ __global__ void k_fragment_weights(const uint16_t* __restrict__ wb, uint16_t* __
   const int K = ks[l], N = ns[l];
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < K * N; i += gridDim.x * blockDim.x) {
     const int k = i / N, n = i - k * N;
-    const int lane = 16 * ((k & 15) >> 2) + (n & 15);
-    const size_t frag = (size_t)(n >> 4) * (K >> 4) + (k >> 4);
-    wt[kWOff[l] + (frag * 64 + lane) * 4 + (k & 3)] = wb[kWOff[l] + i];
+    wt[kWOff[l] + forward_slot(K, k, n)] = wb[kWOff[l] + i];
   }
 }
 
@@ -336,15 +194,21 @@ __global__ void k_fragment_weights(const uint16_t* __restrict__ wb, uint16_t* __
 // (FP32, B x kOutPad), where the layered forward writes every layer's FP32
 // pre-activations and bf16 activations to HBM and reads them back.
 // Hidden layers: wave w computes the 64 rows x columns [64w, 64w + 64) as
-// 4 x 4 tiles of v_mfma_f32_16x16x16bf16_1k, A fragments from LDS and B
+// 4 x 4 tiles of v_mfma_f32_16x16x32_bf16, A fragments from LDS and B
 // fragments straight from the fragment-ordered weights (312 KB in all, read by
 // every workgroup, so they stay in L2); after a barrier the epilogue
 // (bias, GELU, bf16) overwrites the activations in place.  Output layer:
-// wave w takes rows [16w, 16w + 16) and the 5 column tiles.  Fragments,
-// the k order of the accumulation and the epilogue arithmetic are those of
-// k_gemm, so the logits equal the layered forward's bit for bit.
+// wave w takes rows [16w, 16w + 16) and the 5 column tiles.  With lane q of a
+// column holding k = 8q .. 8q + 7, one 32-k step gives the bits of k_gemm's
+// two 16-k steps in k order (measured on 10^6 random elements, and tested
+// through the whole network), so the logits equal the layered forward's bit
+// for bit.
 constexpr int kFuseRows = 64;
 constexpr int kActLd = kHidden + 8;  // LDS row stride (bf16): 528 B
+
+__device__ __forceinline__ bf16x8_ frag(const uint16_t* p) {
+  return *reinterpret_cast<const bf16x8_*>(p);
+}
 
 __global__ void __launch_bounds__(256) k_forward_fused(const uint16_t* __restrict__ x0, int n,
                                                        const uint16_t* __restrict__ wt,
@@ -363,44 +227,25 @@ __global__ void __launch_bounds__(256) k_forward_fused(const uint16_t* __restric
   __syncthreads();
   const int lr = lane & 15, lq = lane >> 4;
   for (int l = 0; l < 3; ++l) {
-    const int K = l == 0 ? kInPad : kHidden;
     const int n0 = wv * 64;
-    const int steps = K / 16;  // 2 or 16
-    // fragment (column block 4 wv + j, k step s) at wl + (j steps + s) 256
-    const uint16_t* wl = wt + kWOff[l] + (size_t)(4 * wv * steps) * 256 + 4 * lane;
+    const int steps = l == 0 ? kInPad / 32 : kHidden / 32;  // 1 or 8
+    // fragment (column block 4 wv + j, k step s) at wl + (j steps + s) 512
+    const uint16_t* wl = wt + kWOff[l] + (size_t)(4 * wv * steps) * 512 + 8 * lane;
     float4_ acc[4][4];
     for (int i = 0; i < 4; ++i)
       for (int j = 0; j < 4; ++j) acc[i][j] = float4_{0.f, 0.f, 0.f, 0.f};
-    // Weight fragments come from L2 and load kPre k steps ahead: a ring of
-    // kPre x 4 fragments, the k loop unrolled by kPre so that the ring
-    // index is a constant.  With the fragment-ordered weights (one 512-byte
-    // read per fragment) depths 2, 4 and 8 time the same on MI355X (0.078
-    // to 0.080 ms per 65,536 rows); with one column per lane from the
-    // row-major transpose (16 partial cache lines per fragment) the forward
-    // took 0.17, 0.16 and 0.14 ms.
-    constexpr int kPre = 2;
-    short4_ bq[kPre][4];
-    for (int d = 0; d < kPre; ++d)
+    // weight fragments come from L2, one k step ahead
+    bf16x8_ bq[4];
+    for (int j = 0; j < 4; ++j) bq[j] = frag(wl + (size_t)(j * steps) * 512);
+    for (int s = 0; s < steps; ++s) {
+      bf16x8_ af[4], next[4];
       for (int j = 0; j < 4; ++j)
-        bq[d][j] = d < steps ? *reinterpret_cast<const short4_*>(wl + (size_t)(j * steps + d) * 256)
-                             : short4_{0, 0, 0, 0};
-    for (int s0 = 0; s0 < steps; s0 += kPre) {
-#pragma unroll
-      for (int d = 0; d < kPre; ++d) {
-        const int s = s0 + d;
-        if (s < steps) {
-          short4_ af[4];
-          for (int i = 0; i < 4; ++i)
-            af[i] = *reinterpret_cast<const short4_*>(&act[i * 16 + lr][16 * s + 4 * lq]);
-          for (int i = 0; i < 4; ++i)
-            for (int j = 0; j < 4; ++j)
-              acc[i][j] =
-                  __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af[i], bq[d][j], acc[i][j], 0, 0, 0);
-          if (s + kPre < steps)
-            for (int j = 0; j < 4; ++j)
-              bq[d][j] = *reinterpret_cast<const short4_*>(wl + (size_t)(j * steps + s + kPre) * 256);
-        }
-      }
+        next[j] = frag(wl + (size_t)(j * steps + min(s + 1, steps - 1)) * 512);
+      for (int i = 0; i < 4; ++i) af[i] = frag(&act[i * 16 + lr][32 * s + 8 * lq]);
+      for (int i = 0; i < 4; ++i)
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bq[j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < 4; ++j) bq[j] = next[j];
     }
     __syncthreads();  // every wave has read this layer's inputs
     const float* b = w + kBOff[l];
@@ -412,25 +257,16 @@ __global__ void __launch_bounds__(256) k_forward_fused(const uint16_t* __restric
     }
     __syncthreads();
   }
-  const uint16_t* wl = wt + kWOff[3] + 4 * lane;  // fragment (j, s) at wl + (16 j + s) 256
+  constexpr int kSteps = kHidden / 32;
+  const uint16_t* wl = wt + kWOff[3] + 8 * lane;  // fragment (j, s) at wl + (8 j + s) 512
   float4_ acc[5];
   for (int j = 0; j < 5; ++j) acc[j] = float4_{0.f, 0.f, 0.f, 0.f};
-  constexpr int kPre = 4, kSteps = kHidden / 16;
-  short4_ bq[kPre][5];
-  for (int d = 0; d < kPre; ++d)
-    for (int j = 0; j < 5; ++j)
-      bq[d][j] = *reinterpret_cast<const short4_*>(wl + (size_t)(j * kSteps + d) * 256);
-  for (int s0 = 0; s0 < kSteps; s0 += kPre) {
 #pragma unroll
-    for (int d = 0; d < kPre; ++d) {
-      const int s = s0 + d;
-      const short4_ af = *reinterpret_cast<const short4_*>(&act[wv * 16 + lr][16 * s + 4 * lq]);
-      for (int j = 0; j < 5; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af, bq[d][j], acc[j], 0, 0, 0);
-      if (s + kPre < kSteps)
-        for (int j = 0; j < 5; ++j)
-          bq[d][j] = *reinterpret_cast<const short4_*>(wl + (size_t)(j * kSteps + s + kPre) * 256);
-    }
+  for (int s = 0; s < kSteps; ++s) {
+    const bf16x8_ af = frag(&act[wv * 16 + lr][32 * s + 8 * lq]);
+    for (int j = 0; j < 5; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, frag(wl + (size_t)(j * kSteps + s) * 512),
+                                                       acc[j], 0, 0, 0);
   }
   const float* b = w + kBOff[3];
   for (int j = 0; j < 5; ++j) {
@@ -443,6 +279,420 @@ __global__ void __launch_bounds__(256) k_forward_fused(const uint16_t* __restric
   }
 }
 
+// --------------------------------------------------------------- training
+//
+// One training step is three kernels: k_train_rows (gather, forward, loss and
+// the gradients' way back to the first layer for 16 rows per workgroup),
+// k_weight_grads (weight and bias gradients from the rows' activations and
+// output gradients) and k_adam or k_sum_grads.  The layer-by-layer step
+// they replace took 14 launches of 5 to 19 us, with every layer's FP32
+// pre-activations and bf16 activations through HBM and FP32 atomics for the
+// split weight gradients: 217 us at batch 4096 on MI355X, now 36.6 us.
+//
+// Operands in MFMA fragment order.  Forward weights: forward_slot, in wt.
+// Backward weights (W^T of layers 1..3, in wg at the same offsets): layers 1,
+// 2 as B fragments of v_mfma_f32_16x16x32_bf16 (lane 16 q + c holds
+// W[16 nb + c][32 ks + 8 q + e]), layer 3 (80 = 5 x 16 columns) as those of
+// v_mfma_f32_16x16x16_bf16 (W[16 nb + c][16 ks + 4 q + e]).
+__device__ __forceinline__ size_t backward_slot(int l, int N, int k, int n) {
+  // element W[k][n]: output column k of the transposed product, reduction n
+  if (l == 3) {
+    const size_t f = (size_t)(k >> 4) * (N >> 4) + (n >> 4);
+    return (f * 64 + 16 * ((n & 15) >> 2) + (k & 15)) * 4 + (n & 3);
+  }
+  const size_t f = (size_t)(k >> 4) * (N >> 5) + (n >> 5);
+  return (f * 64 + 16 * ((n & 31) >> 3) + (k & 15)) * 8 + (n & 7);
+}
+
+__global__ void k_backward_weights(const uint16_t* __restrict__ wb, uint16_t* __restrict__ wg) {
+  const int l = blockIdx.y + 1;
+  const int K = kHidden, N = l == 3 ? kOutPad : kHidden;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < K * N; i += gridDim.x * blockDim.x) {
+    const int k = i / N, n = i - k * N;
+    wg[kWOff[l] + backward_slot(l, N, k, n)] = wb[kWOff[l] + i];
+  }
+}
+
+// Row fragments: what the weight gradients read.  A 16x16 tile's MFMA result
+// lane 16 q + c holds rows 4 q .. 4 q + 3 of column c, which is a lane's part
+// of an operand fragment with the rows as reduction index: 4 bf16, 8 bytes,
+// 512 contiguous bytes per tile.  Per group of 16 rows: the layers' inputs
+// (2 + 16 + 16 + 16 blocks of 16 columns), then their output gradients
+// (16 + 16 + 16 + 5).
+constexpr int kInBlock[4] = {0, 2, 18, 34};
+constexpr int kGradBlock[4] = {50, 66, 82, 98};
+constexpr int kRowBlocks = 103;
+// per group of 16 rows: column sums of the output gradients (bias gradients
+// of layers 0..2, then layer 3's 65) and the loss
+constexpr int kSums = 3 * kHidden + kOut + 1;
+
+__device__ __forceinline__ uint2 pack4(uint16_t a, uint16_t b, uint16_t c, uint16_t d) {
+  return make_uint2((uint32_t)a | ((uint32_t)b << 16), (uint32_t)c | ((uint32_t)d << 16));
+}
+
+// Workgroup of 16 rows; each of its kTrainWaves waves has the same columns of
+// every hidden layer, forward and backward, so a layer's FP32 pre-activations
+// stay in its registers until the backward pass needs them.  A layer's weight
+// fragments do not depend on its input: all of them are loaded before the
+// barrier of the layer above, so that a layer waits for L2 at its bandwidth
+// (128 KB per workgroup and layer) instead of its latency.  What is left is
+// the GELUs and their derivatives and the chain of 7 layers with their
+// barriers, which 4 waves per SIMD hide best: whole step at batch 4096 with
+// 8 and 16 waves 38.9 and 36.6 us.
+// Arithmetic, rounding points and k order are the layered forward's and the
+// loss's own, so the rounded gradients are the same bits.
+constexpr int kTrainWaves = 16;
+constexpr int kCb = kHidden / 16 / kTrainWaves;  // blocks of 16 columns per wave
+
+struct TrainRows {
+  const float* xs;
+  const float* ys;
+  const uint32_t* idx;   // rows of xs/ys (null: row i)
+  int B;                 // multiple of 16
+  const float* w;        // biases
+  const uint16_t* wt;
+  const uint16_t* wg;
+  uint2* frags;          // B / 16 x kRowBlocks x 64
+  float* sums;           // B / 16 x kSums
+};
+
+__global__ void __launch_bounds__(64 * kTrainWaves) k_train_rows(TrainRows a) {
+  __shared__ __attribute__((aligned(16))) uint16_t act[16][kActLd];
+  __shared__ __attribute__((aligned(16))) uint16_t grad[16][kActLd];
+  __shared__ float z4[16][kOutPad + 4];
+  __shared__ float s_db[kTrainWaves][kOut];
+  __shared__ float s_loss[kTrainWaves];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, lr = lane & 15, lq = lane >> 4;
+  const int row0 = blockIdx.x * 16;
+  uint2* const frags = a.frags + (size_t)blockIdx.x * kRowBlocks * 64;
+  float* const sums = a.sums + (size_t)blockIdx.x * kSums;
+  // input rows
+  for (int i = t; i < 16 * kInPad; i += 64 * kTrainWaves) {
+    const int r = i / kInPad, c = i % kInPad;
+    const size_t row = a.idx ? a.idx[row0 + r] : (uint32_t)(row0 + r);
+    act[r][c] = c < kFeat ? f2bf(a.xs[row * kFeat + c]) : (uint16_t)0;
+  }
+  // a layer's weight fragments of this wave
+  bf16x8_ b[8][kCb];
+  auto load = [&](const uint16_t* w, int steps) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if (s < steps)
+#pragma unroll
+        for (int j = 0; j < kCb; ++j)
+          b[s][j] = frag(w + ((size_t)((kCb * wv + j) * steps + s) * 64 + lane) * 8);
+  };
+  // acc = in x the loaded fragments
+  auto product = [&](const uint16_t (*in)[kActLd], int steps, float4_ (&acc)[kCb]) {
+#pragma unroll
+    for (int j = 0; j < kCb; ++j) acc[j] = float4_{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if (s < steps) {
+        const bf16x8_ f = frag(&in[lr][32 * s + 8 * lq]);
+#pragma unroll
+        for (int j = 0; j < kCb; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f, b[s][j], acc[j], 0, 0, 0);
+      }
+  };
+  load(a.wt + kWOff[0], 1);
+  __syncthreads();
+  if (wv < 2) {
+    const int c = 16 * wv + lr;
+    frags[(kInBlock[0] + wv) * 64 + lane] =
+        pack4(act[4 * lq][c], act[4 * lq + 1][c], act[4 * lq + 2][c], act[4 * lq + 3][c]);
+  }
+  float4_ z[3][kCb];
+  static_assert(kTrainWaves >= 5, "a wave per column tile of the output layer");
+  bf16x8_ b4[8] = {};
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+    product(act, l == 0 ? 1 : 8, z[l]);
+    if (l < 2) {
+      load(a.wt + kWOff[l + 1], 8);
+    } else if (wv < 5) {  // the output layer's 5 column tiles: one each
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        b4[s] = frag(a.wt + kWOff[3] + ((size_t)(wv * 8 + s) * 64 + lane) * 8);
+    }
+    uint16_t h[kCb][4];
+#pragma unroll
+    for (int j = 0; j < kCb; ++j) {
+      const float bj = a.w[kBOff[l] + 16 * (kCb * wv + j) + lr];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        z[l][j][r] += bj;
+        h[j][r] = f2bf(gelu_f(z[l][j][r]));
+      }
+      frags[(kInBlock[l + 1] + kCb * wv + j) * 64 + lane] =
+          pack4(h[j][0], h[j][1], h[j][2], h[j][3]);
+    }
+    __syncthreads();  // every wave has read this layer's inputs
+#pragma unroll
+    for (int j = 0; j < kCb; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) act[4 * lq + r][16 * (kCb * wv + j) + lr] = h[j][r];
+    __syncthreads();
+  }
+  if (wv < 5) {
+    float4_ o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(&act[lr][32 * s + 8 * lq]), b4[s], o, 0, 0,
+                                                  0);
+    const int col = 16 * wv + lr;
+    const float bj = a.w[kBOff[3] + col];
+    for (int r = 0; r < 4; ++r) z4[4 * lq + r][col] = o[r] + bj;
+  }
+  // backward weights of the output layer: 5 steps of 16
+  short4_ b3[5][kCb];
+#pragma unroll
+  for (int s = 0; s < 5; ++s)
+#pragma unroll
+    for (int j = 0; j < kCb; ++j)
+      b3[s][j] = *reinterpret_cast<const short4_*>(
+          a.wg + kWOff[3] + ((size_t)((kCb * wv + j) * 5 + s) * 64 + lane) * 4);
+  __syncthreads();
+  // Loss and its gradient, a row per wave at a time: lane k has radial logit
+  // k (z[1 + k]), lane 0 also the detection logit.
+  {
+    const float invB = 1.0f / (float)a.B;
+    float db_r = 0.0f, db_0 = 0.0f, lsum = 0.0f;
+    constexpr int kRows = 16 / kTrainWaves;
+#pragma unroll
+    for (int r = kRows * wv; r < kRows * wv + kRows; ++r) {
+      const size_t row = a.idx ? a.idx[row0 + r] : (uint32_t)(row0 + r);
+      const float* yr = a.ys + row * kTarget;
+      const float zl = z4[r][1 + lane];
+      float mx = zl;
+      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      const float e = expf(zl - mx);
+      float se = e;
+      for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
+      const float prob = e / se;
+      const float q = yr[1 + lane];
+      float qs = q;
+      for (int o = 32; o > 0; o >>= 1) qs += __shfl_xor(qs, o, 64);
+      const float wrad = qs > 0.0f ? 1.0f : 0.0f;
+      float ce = q > 0.0f ? -q * (zl - mx - logf(se)) : 0.0f;
+      for (int o = 32; o > 0; o >>= 1) ce += __shfl_xor(ce, o, 64);
+      const uint16_t grb = f2bf(wrad * (prob - q) * invB);
+      grad[r][1 + lane] = grb;
+      db_r += bf2f(grb);
+      if (lane < kOutPad - 1 - 64) grad[r][65 + lane] = 0;
+      if (lane == 0) {
+        const float z0 = z4[r][0], y0 = yr[0];
+        const float p = 1.0f / (1.0f + expf(-z0));
+        // BCE with logits: max(z,0) - z y + log(1 + e^-|z|)
+        const float bce = fmaxf(z0, 0.0f) - z0 * y0 + log1pf(expf(-fabsf(z0)));
+        const uint16_t g0 = f2bf((p - y0) * invB);
+        grad[r][0] = g0;
+        db_0 += bf2f(g0);
+        lsum += (bce + wrad * ce) * invB;
+      }
+    }
+    s_db[wv][1 + lane] = db_r;
+    if (lane == 0) {
+      s_db[wv][0] = db_0;
+      s_loss[wv] = lsum;
+    }
+  }
+  __syncthreads();
+  if (t <= kOut) {  // in wave order; the last column is the loss
+    float v = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kTrainWaves; ++i) v += t < kOut ? s_db[i][t] : s_loss[i];
+    sums[3 * kHidden + t] = v;
+  }
+  if (wv < 5) {
+    const int c = 16 * wv + lr;
+    frags[(kGradBlock[3] + wv) * 64 + lane] =
+        pack4(grad[4 * lq][c], grad[4 * lq + 1][c], grad[4 * lq + 2][c], grad[4 * lq + 3][c]);
+  }
+  // back through the layers: dZ_{l-1} = (dZ_l W_l^T) gelu'(Z_{l-1})
+  float4_ acc[kCb];
+#pragma unroll
+  for (int j = 0; j < kCb; ++j) acc[j] = float4_{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < 5; ++s) {
+    const short4_ f = *reinterpret_cast<const short4_*>(&grad[lr][16 * s + 4 * lq]);
+#pragma unroll
+    for (int j = 0; j < kCb; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(f, b3[s][j], acc[j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int l = 2; l >= 0; --l) {
+    // the layer's output gradients go to `act` (l = 2, 0) or `grad` (l = 1):
+    // the other one holds the gradients that this layer's product reads
+    uint16_t (*out)[kActLd] = l == 1 ? grad : act;
+    if (l > 0) load(a.wg + kWOff[l], 8);
+#pragma unroll
+    for (int j = 0; j < kCb; ++j) {
+      uint16_t h[4];
+      float colsum = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        h[r] = f2bf(acc[j][r] * gelu_grad(z[l][j][r]));
+        colsum += bf2f(h[r]);
+        if (l > 0) out[4 * lq + r][16 * (kCb * wv + j) + lr] = h[r];
+      }
+      frags[(kGradBlock[l] + kCb * wv + j) * 64 + lane] = pack4(h[0], h[1], h[2], h[3]);
+      colsum += __shfl_xor(colsum, 16, 64);
+      colsum += __shfl_xor(colsum, 32, 64);
+      if (lq == 0) sums[l * kHidden + 16 * (kCb * wv + j) + lr] = colsum;
+    }
+    if (l > 0) {
+      __syncthreads();
+      product(out, 8, acc);
+    }
+  }
+}
+
+// Weight gradients in^T dZ of all layers from the row fragments, and the bias
+// gradients and the loss from the rows' sums: partial results of gridDim.y
+// slices of the batch, added in order by k_adam or k_sum_grads (a fixed order:
+// the same step twice gives the same bits).
+// Workgroups [0, kWeightTiles): a 64 x 64 tile of one layer, the slice's row
+// groups (two per 32-k MFMA step) shared by the 4 waves and added in LDS; the
+// others: 64 columns of the sums each.
+constexpr int kWeightTiles = 4 + 16 + 16 + 8;
+constexpr int kSumBlocks = (kSums + 63) / 64;
+constexpr size_t kPartial = kParams + 16;  // the loss at kParams
+
+__global__ void __launch_bounds__(256) k_weight_grads(const uint2* __restrict__ frags,
+                                                      const float* __restrict__ sums, int groups,
+                                                      float* __restrict__ part) {
+  __shared__ float4_ s_acc[4][16][64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, lr = lane & 15, lq = lane >> 4;
+  const int slices = gridDim.y, slice = blockIdx.y;
+  float* const out = part + (size_t)slice * kPartial;
+  if ((int)blockIdx.x >= kWeightTiles) {
+    float* s_sum = reinterpret_cast<float*>(s_acc);
+    const int c = ((int)blockIdx.x - kWeightTiles) * 64 + lane;
+    float v = 0.0f;
+    if (c < kSums)
+      for (int g = slice * 4 + wv; g < groups; g += 4 * slices) v += sums[(size_t)g * kSums + c];
+    s_sum[t] = v;
+    __syncthreads();
+    if (wv == 0 && c < kSums) {
+      v = (s_sum[lane] + s_sum[64 + lane]) + (s_sum[128 + lane] + s_sum[192 + lane]);
+      const int l = min(c / kHidden, 3);
+      out[c == kSums - 1 ? kParams : kBOff[l] + (size_t)(c - l * kHidden)] = v;
+    }
+    return;
+  }
+  // layer and tile (4 blocks of 16 input columns x 4 of 16 output columns)
+  const int bi = blockIdx.x;
+  const int l = bi < 4 ? 0 : bi < 20 ? 1 : bi < 36 ? 2 : 3;
+  const int in_l = l == 0 ? bi : l == 3 ? bi - 36 : (bi - 4) & 15;
+  const int mt = l == 0 ? 0 : l == 3 ? in_l >> 1 : in_l >> 2;
+  const int nt = l == 0 ? in_l : l == 3 ? in_l & 1 : in_l & 3;
+  const int mv = l == 0 ? 2 : 4;                       // valid blocks
+  const int nv = l == 3 ? (nt == 0 ? 4 : 1) : 4;
+  const int N = l == 3 ? kOutPad : kHidden;
+  const uint2* fa = frags + (size_t)(kInBlock[l] + 4 * mt) * 64 + lane;
+  const uint2* fb = frags + (size_t)(kGradBlock[l] + 4 * nt) * 64 + lane;
+  float4_ acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = float4_{0.f, 0.f, 0.f, 0.f};
+  const int pairs = (groups + 1) >> 1;
+  const uint2 none = make_uint2(0u, 0u);
+  for (int p = slice * 4 + wv; p < pairs; p += 4 * slices) {
+    const size_t g0 = (size_t)(2 * p) * kRowBlocks * 64, g1 = g0 + (size_t)kRowBlocks * 64;
+    const bool two = 2 * p + 1 < groups;
+    uint2 va[4][2], vb[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      va[i][0] = i < mv ? fa[g0 + i * 64] : none;
+      va[i][1] = i < mv && two ? fa[g1 + i * 64] : none;
+      vb[i][0] = i < nv ? fb[g0 + i * 64] : none;
+      vb[i][1] = i < nv && two ? fb[g1 + i * 64] : none;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < mv) {
+        const bf16x8_ x = __builtin_bit_cast(
+            bf16x8_, make_uint4(va[i][0].x, va[i][0].y, va[i][1].x, va[i][1].y));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              x,
+              __builtin_bit_cast(bf16x8_,
+                                 make_uint4(vb[j][0].x, vb[j][0].y, vb[j][1].x, vb[j][1].y)),
+              acc[i][j], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s_acc[wv][i * 4 + j][lane] = acc[i][j];
+  __syncthreads();
+  if (wv < mv) {  // wave w adds and writes the tile's row blocks w
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j >= nv) break;
+      const int k = wv * 4 + j;
+      const float4_ v =
+          (s_acc[0][k][lane] + s_acc[1][k][lane]) + (s_acc[2][k][lane] + s_acc[3][k][lane]);
+      const int row = (4 * mt + wv) * 16 + 4 * lq, col = (4 * nt + j) * 16 + lr;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[kWOff[l] + (size_t)(row + r) * N + col] = v[r];
+    }
+  }
+}
+
+// gradient of parameter i: its slices' partial sums in order
+__device__ __forceinline__ float sum_slices(const float* __restrict__ part, int slices, size_t i) {
+  float g = 0.0f;
+  for (int s = 0; s < slices; ++s) g += part[(size_t)s * kPartial + i];
+  return g;
+}
+
+// parameters without a gradient: the output padding's biases
+__device__ __forceinline__ bool no_gradient(size_t i) { return i >= kBOff[3] + kOut && i < kParams; }
+
+__global__ void k_sum_grads(const float* __restrict__ part, int slices, float* __restrict__ g,
+                            float* __restrict__ loss) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > kParams) return;
+  const float v = no_gradient(i) ? 0.0f : sum_slices(part, slices, i);
+  if (i < kParams)
+    g[i] = v;
+  else
+    *loss = v;
+}
+
+// Adam (Kingma & Ba 2015) on FP32 master weights; refreshes the bf16 copies
+// (row-major, forward and backward fragment order).
+__global__ void k_adam(float* w, const float* __restrict__ part, int slices, float* m, float* v,
+                       uint16_t* wb, uint16_t* wt, uint16_t* wg, float* loss, float lr, float b1,
+                       float b2, float eps, float c1, float c2) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > kParams) return;
+  const float gi = no_gradient(i) ? 0.0f : sum_slices(part, slices, i);
+  if (i == kParams) {
+    *loss = gi;
+    return;
+  }
+  const float mi = b1 * m[i] + (1.0f - b1) * gi;
+  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
+  m[i] = mi;
+  v[i] = vi;
+  const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  w[i] = wi;
+  const uint16_t h = f2bf(wi);
+  wb[i] = h;
+  const int l = i < kWOff[1] ? 0 : i < kWOff[2] ? 1 : i < kWOff[3] ? 2 : 3;
+  const int K = l == 0 ? kInPad : kHidden, N = l == 3 ? kOutPad : kHidden;
+  const int e = (int)(i - kWOff[l]);
+  if (e >= K * N) return;  // a bias
+  const int k = e / N, n = e - k * N;
+  wt[kWOff[l] + forward_slot(K, k, n)] = h;
+  if (l > 0) wg[kWOff[l] + backward_slot(l, N, k, n)] = h;
+}
+
 }  // namespace fd2mlp
 
 using namespace fd2mlp;
@@ -452,25 +702,25 @@ using namespace fd2mlp;
 struct fd2_mlp {
   int device = 0;
   hipStream_t stream = nullptr;
-  int cap = 0;  // batch capacity
+  int cap = 0;          // rows of x0 and z[3]
+  int cap_layers = 0;   // rows of z[0..2] and a (layer-by-layer forward)
+  int cap_train = 0;    // rows of frags and sums
   float* w = nullptr;   // FP32 master parameters (kParams)
-  float* g = nullptr;   // gradients
   float* m = nullptr;   // Adam moments
   float* v = nullptr;
   uint16_t* wb = nullptr;  // bf16 copy (same layout as w)
-  uint16_t* wt = nullptr;  // bf16 weight matrices transposed (fused forward)
-  bool wt_stale = true;    // wb changed since wt was built
+  uint16_t* wt = nullptr;  // bf16 weights in forward fragment order
+  uint16_t* wg = nullptr;  // and in backward fragment order
+  bool wt_stale = true;    // wb changed since wt and wg were built
   uint16_t* x0 = nullptr;
   float* z[4] = {};
   uint16_t* a[3] = {};
-  uint16_t* dz = nullptr;    // bf16 gradient of the current layer's output
-  uint16_t* dz2 = nullptr;
-  float* y = nullptr;
-  float* loss = nullptr;
+  uint2* frags = nullptr;    // training: row fragments, rows' sums, slices' partial gradients
+  float* sums = nullptr;
+  float* part = nullptr;
   float* data_x = nullptr;
   float* data_y = nullptr;
   int64_t n_data = 0;
-  uint32_t* idx = nullptr;
   int64_t step = 0;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   // fd2_surrogate_submit's buffers, kept between calls and grown on demand
@@ -489,18 +739,12 @@ namespace {
     if ((call) != hipSuccess) return FD2_E_DEVICE; \
   } while (0)
 
-void free_batch(fd2_mlp* p) {
-  void* bufs[] = {p->x0, p->z[0], p->z[1], p->z[2], p->z[3], p->a[0], p->a[1], p->a[2],
-                  p->dz, p->dz2, p->y, p->idx};
-  for (void* b : bufs)
-    if (b) (void)hipFree(b);
-  p->x0 = nullptr;
-  for (auto& q : p->z) q = nullptr;
-  for (auto& q : p->a) q = nullptr;
-  p->dz = p->dz2 = nullptr;
-  p->y = nullptr;
-  p->idx = nullptr;
-  p->cap = 0;
+// grows one buffer of the network (its old contents are not needed)
+template <class T>
+bool grow(T** buf, size_t bytes) {
+  if (*buf) (void)hipFree(*buf);
+  *buf = nullptr;
+  return hipMalloc(buf, bytes) == hipSuccess;
 }
 
 // fd2_surrogate_submit's device buffers (fd2_mlp::sbuf)
@@ -526,122 +770,103 @@ bool reserve(fd2_mlp* p, int which, size_t bytes, T** out) {
   return true;
 }
 
+// buffers of B rows for the fused forward
 int ensure_batch(fd2_mlp* p, int B) {
   if (B <= p->cap) return FD2_OK;
-  free_batch(p);
+  p->cap = 0;
   const size_t b = (size_t)B;
-  MLP_HIP(hipMalloc(&p->x0, b * kInPad * 2));
-  for (int l = 0; l < 3; ++l) {
-    MLP_HIP(hipMalloc(&p->z[l], b * kHidden * 4));
-    MLP_HIP(hipMalloc(&p->a[l], b * kHidden * 2));
-  }
-  MLP_HIP(hipMalloc(&p->z[3], b * kOutPad * 4));
-  MLP_HIP(hipMalloc(&p->dz, b * kHidden * 2));
-  MLP_HIP(hipMalloc(&p->dz2, b * kHidden * 2));
-  MLP_HIP(hipMalloc(&p->y, b * kTarget * 4));
-  MLP_HIP(hipMalloc(&p->idx, b * 4));
+  if (!grow(&p->x0, b * kInPad * 2) || !grow(&p->z[3], b * kOutPad * 4)) return FD2_E_DEVICE;
   p->cap = B;
   return FD2_OK;
 }
 
-// forward pass on p->x0 (B rows) -> z[3] logits
-// forward pass of B rows of p->x0; the output layer goes to `out` (B x
-// kOutPad f32) when given, else to p->z[3]
-int forward(fd2_mlp* p, int B, hipStream_t stream, float* out = nullptr) {
+// and for the layer-by-layer forward
+int ensure_layers(fd2_mlp* p, int B) {
+  const int rc = ensure_batch(p, B);
+  if (rc || B <= p->cap_layers) return rc;
+  p->cap_layers = 0;
+  for (int l = 0; l < 3; ++l)
+    if (!grow(&p->z[l], (size_t)B * kHidden * 4) || !grow(&p->a[l], (size_t)B * kHidden * 2))
+      return FD2_E_DEVICE;
+  p->cap_layers = B;
+  return FD2_OK;
+}
+
+// and for a training step.  The weight gradients' slices (kMaxSlices at most)
+// give every wave of k_weight_grads about 4 pairs of row groups.
+constexpr int kMaxSlices = 16;
+int train_slices(int B) {
+  const int s = B / 16 / 32;
+  return s < 1 ? 1 : s > kMaxSlices ? kMaxSlices : s;
+}
+int ensure_train(fd2_mlp* p, int B) {
+  if (!p->part && hipMalloc(&p->part, kMaxSlices * kPartial * 4) != hipSuccess)
+    return FD2_E_DEVICE;
+  if (B <= p->cap_train) return FD2_OK;
+  p->cap_train = 0;
+  const size_t groups = (size_t)B / 16;
+  if (!grow(&p->frags, groups * kRowBlocks * 64 * sizeof(uint2)) ||
+      !grow(&p->sums, groups * kSums * 4))
+    return FD2_E_DEVICE;
+  p->cap_train = B;
+  return FD2_OK;
+}
+
+// forward pass of B rows of p->x0, layer by layer; the logits go to p->z[3]
+int forward_layers(fd2_mlp* p, int B, hipStream_t stream) {
   const int ins[4] = {kInPad, kHidden, kHidden, kHidden};
   const int outs[4] = {kHidden, kHidden, kHidden, kOutPad};
-  const uint16_t* in = p->x0;
   for (int l = 0; l < 4; ++l) {
     GemmArgs a{};
-    a.A = in;
+    a.A = l == 0 ? p->x0 : p->a[l - 1];
     a.B = p->wb + kWOff[l];
     a.M = B;
     a.N = outs[l];
     a.K = ins[l];
-    a.lda = ins[l];
-    a.ldb = outs[l];
-    a.kchunk = ins[l];
     a.bias = p->w + kBOff[l];
-    a.outf = l == 3 && out ? out : p->z[l];
+    a.outf = p->z[l];
     a.outb = l < 3 ? p->a[l] : nullptr;
-    a.ldo = outs[l];
-    MLP_HIP((gemm<false, false, kStoreF32>(a, 1, stream)));
-    in = l < 3 ? p->a[l] : nullptr;
+    hipLaunchKernelGGL(k_gemm, dim3((a.N + 63) / 64, (a.M + 63) / 64), dim3(256), 0, stream, a);
+    MLP_HIP(hipGetLastError());
   }
+  return FD2_OK;
+}
+
+// the fragment-ordered weights after the parameters changed
+int refresh_fragments(fd2_mlp* p, hipStream_t stream) {
+  if (!p->wt_stale) return FD2_OK;
+  hipLaunchKernelGGL(k_fragment_weights, dim3(64, 4), dim3(256), 0, stream, p->wb, p->wt);
+  hipLaunchKernelGGL(k_backward_weights, dim3(64, 3), dim3(256), 0, stream, p->wb, p->wg);
+  MLP_HIP(hipGetLastError());
+  p->wt_stale = false;
   return FD2_OK;
 }
 
 // inference forward of B rows of p->x0 in one kernel (k_forward_fused):
 // the output logits go to `out` (B x kOutPad f32) when given, else to
-// p->z[3]; the other layers' buffers are not written.  Rebuilds the
-// transposed weights first when the parameters changed.
+// p->z[3].  Rebuilds the fragment-ordered weights first when the parameters
+// changed.
 int forward_fused(fd2_mlp* p, int B, hipStream_t stream, float* out = nullptr) {
-  if (p->wt_stale) {
-    hipLaunchKernelGGL(k_fragment_weights, dim3(64, 4), dim3(256), 0, stream, p->wb, p->wt);
-    MLP_HIP(hipGetLastError());
-    p->wt_stale = false;
-  }
-  if (B <= 0) return FD2_OK;
+  const int rc = refresh_fragments(p, stream);
+  if (rc || B <= 0) return rc;
   hipLaunchKernelGGL(k_forward_fused, dim3((unsigned)((B + kFuseRows - 1) / kFuseRows)),
                      dim3(256), 0, stream, p->x0, B, p->wt, p->w, out ? out : p->z[3]);
   MLP_HIP(hipGetLastError());
   return FD2_OK;
 }
 
-// backward from the bf16 output gradient in p->dz (B x 80) into p->g
-int backward(fd2_mlp* p, int B) {
-  const int ins[4] = {kInPad, kHidden, kHidden, kHidden};
-  const int outs[4] = {kHidden, kHidden, kHidden, kOutPad};
-  if (B % 16) return FD2_E_INVAL;
-  const int target = B >= 1024 ? 16 : 1;
-  const int kchunk = ((B + target - 1) / target + 15) / 16 * 16;
-  const int splits = (B + kchunk - 1) / kchunk;
-  uint16_t* dcur = p->dz;   // gradient w.r.t. layer l's output Z_l
-  uint16_t* dnext = p->dz2;
-  for (int l = 3; l >= 0; --l) {
-    const uint16_t* in = l == 0 ? p->x0 : p->a[l - 1];
-    // dW_l = in^T dZ_l  ([ins x B] x [B x outs]), split over B
-    GemmArgs gw{};
-    gw.A = in;
-    gw.B = dcur;
-    gw.M = ins[l];
-    gw.N = outs[l];
-    gw.K = B;
-    gw.lda = ins[l];
-    gw.ldb = outs[l];
-    gw.kchunk = kchunk;
-    gw.outf = p->g + kWOff[l];
-    MLP_HIP((gemm<true, false, kAtomicF32>(gw, splits, p->stream)));
-    if (l == 0) break;
-    // dZ_{l-1} = (dZ_l W_l^T) * gelu'(Z_{l-1}); bias grad of layer l-1
-    GemmArgs gx{};
-    gx.A = dcur;
-    gx.B = p->wb + kWOff[l];
-    gx.M = B;
-    gx.N = ins[l];
-    gx.K = outs[l];
-    gx.lda = outs[l];
-    gx.ldb = outs[l];
-    gx.kchunk = outs[l];
-    gx.Z = p->z[l - 1];
-    gx.outb = dnext;
-    gx.ldo = ins[l];
-    gx.dbias = p->g + kBOff[l - 1];
-    MLP_HIP((gemm<false, true, kGeluGradBf16>(gx, 1, p->stream)));
-    uint16_t* t = dcur;
-    dcur = dnext;
-    dnext = t;
-  }
-  return FD2_OK;
-}
-
-int loss_grad(fd2_mlp* p, int B, float* d_loss) {
-  hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, p->stream, d_loss, (size_t)1);
-  hipLaunchKernelGGL(k_head_loss, dim3(std::min((B * 64 + 255) / 256, kHeadLossBlocks)), dim3(256),
-                     0, p->stream,
-                     p->z[3], p->y, B, p->dz, p->g + kBOff[3], d_loss);
+// rows and weight gradients of one batch (rows idx of xs/ys, or the first B)
+// into p->part; returns the number of slices there, or a negative status
+int batch_gradients(fd2_mlp* p, const float* xs, const float* ys, const uint32_t* idx, int B) {
+  const int rc = refresh_fragments(p, p->stream);
+  if (rc) return rc;
+  TrainRows a{xs, ys, idx, B, p->w, p->wt, p->wg, p->frags, p->sums};
+  const int groups = B / 16, slices = train_slices(B);
+  hipLaunchKernelGGL(k_train_rows, dim3(groups), dim3(64 * kTrainWaves), 0, p->stream, a);
+  hipLaunchKernelGGL(k_weight_grads, dim3(kWeightTiles + kSumBlocks, slices), dim3(256), 0,
+                     p->stream, p->frags, p->sums, groups, p->part);
   MLP_HIP(hipGetLastError());
-  return FD2_OK;
+  return slices;
 }
 
 void init_params(std::vector<float>& w, uint32_t seed) {
@@ -689,10 +914,9 @@ int fd2_mlp_create(int device, uint32_t seed, fd2_mlp** out) {
       break;
     }
     const size_t n = kParams;
-    if (hipMalloc(&p->w, n * 4) != hipSuccess || hipMalloc(&p->g, n * 4) != hipSuccess ||
-        hipMalloc(&p->m, n * 4) != hipSuccess || hipMalloc(&p->v, n * 4) != hipSuccess ||
-        hipMalloc(&p->wb, n * 2) != hipSuccess || hipMalloc(&p->wt, n * 2) != hipSuccess ||
-        hipMalloc(&p->loss, 4) != hipSuccess) {
+    if (hipMalloc(&p->w, n * 4) != hipSuccess || hipMalloc(&p->m, n * 4) != hipSuccess ||
+        hipMalloc(&p->v, n * 4) != hipSuccess || hipMalloc(&p->wb, n * 2) != hipSuccess ||
+        hipMalloc(&p->wt, n * 2) != hipSuccess || hipMalloc(&p->wg, n * 2) != hipSuccess) {
       rc = FD2_E_NOMEM;
       break;
     }
@@ -712,8 +936,9 @@ void fd2_mlp_destroy(fd2_mlp* p) {
   if (!p) return;
   (void)hipSetDevice(p->device);
   if (p->stream) (void)hipStreamSynchronize(p->stream);
-  free_batch(p);
-  void* bufs[] = {p->w, p->g, p->m, p->v, p->wb, p->wt, p->loss, p->data_x, p->data_y};
+  void* bufs[] = {p->w, p->m, p->v, p->wb, p->wt, p->wg, p->data_x, p->data_y, p->x0, p->z[0],
+                  p->z[1], p->z[2], p->z[3], p->a[0], p->a[1], p->a[2], p->frags, p->sums,
+                  p->part};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (void* b : p->sbuf)
@@ -733,7 +958,6 @@ int fd2_mlp_set_params(fd2_mlp* p, const float* host, size_t n) {
                      p->w, p->wb, (int)n);
   p->wt_stale = true;
   const unsigned nb = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(k_zero, dim3(nb), dim3(256), 0, p->stream, p->g, n);
   hipLaunchKernelGGL(k_zero, dim3(nb), dim3(256), 0, p->stream, p->m, n);
   hipLaunchKernelGGL(k_zero, dim3(nb), dim3(256), 0, p->stream, p->v, n);
   MLP_HIP(hipGetLastError());
@@ -791,7 +1015,7 @@ int fd2_mlp_logits(fd2_mlp* p, const float* x, int64_t n, float* logits, int lay
   MLP_HIP(hipSetDevice(p->device));
   const int64_t chunk = 65536;
   float* dx = nullptr;
-  int rc = ensure_batch(p, (int)chunk);
+  int rc = layered ? ensure_layers(p, (int)chunk) : ensure_batch(p, (int)chunk);
   if (rc) return rc;
   MLP_HIP(hipMalloc(&dx, (size_t)chunk * kFeat * 4));
   for (int64_t s = 0; s < n && rc == FD2_OK; s += chunk) {
@@ -803,7 +1027,7 @@ int fd2_mlp_logits(fd2_mlp* p, const float* x, int64_t n, float* logits, int lay
     }
     hipLaunchKernelGGL(k_pack_inputs, dim3((b * kIn + 255) / 256), dim3(256), 0, p->stream,
                        dx, b, p->x0);
-    rc = layered ? forward(p, b, p->stream) : forward_fused(p, b, p->stream);
+    rc = layered ? forward_layers(p, b, p->stream) : forward_fused(p, b, p->stream);
     if (rc) break;
     // the kOut logits of each row (of kOutPad computed)
     if (hipMemcpy2DAsync(logits + s * kOut, kOut * 4, p->z[3], kOutPad * 4, kOut * 4, b,
@@ -839,28 +1063,29 @@ int fd2_mlp_gradients(fd2_mlp* p, const float* x, const float* y, int B, float* 
                       float* loss) {
   if (!p || !x || !y || !grads || B <= 0 || B % 16) return FD2_E_INVAL;
   MLP_HIP(hipSetDevice(p->device));
-  int rc = ensure_batch(p, B);
+  int rc = ensure_train(p, B);
   if (rc) return rc;
-  float* dx = nullptr;
-  MLP_HIP(hipMalloc(&dx, (size_t)B * kFeat * 4));
-  rc = FD2_OK;
-  if (hipMemcpyAsync(dx, x, (size_t)B * kFeat * 4, hipMemcpyHostToDevice, p->stream) != hipSuccess ||
-      hipMemcpyAsync(p->y, y, (size_t)B * kTarget * 4, hipMemcpyHostToDevice, p->stream) != hipSuccess)
+  // inputs, targets, gradients and loss in one buffer
+  const size_t nx = (size_t)B * kFeat, ny = (size_t)B * kTarget;
+  float* d = nullptr;
+  MLP_HIP(hipMalloc(&d, (nx + ny + kParams + 1) * 4));
+  float *dy = d + nx, *dg = dy + ny;
+  int slices = 0;
+  if (hipMemcpyAsync(d, x, nx * 4, hipMemcpyHostToDevice, p->stream) != hipSuccess ||
+      hipMemcpyAsync(dy, y, ny * 4, hipMemcpyHostToDevice, p->stream) != hipSuccess)
     rc = FD2_E_DEVICE;
+  if (!rc && (slices = batch_gradients(p, d, dy, nullptr, B)) < 0) rc = slices;
   if (!rc) {
-    hipLaunchKernelGGL(k_zero, dim3((unsigned)((kParams + 255) / 256)), dim3(256), 0, p->stream,
-                       p->g, (size_t)kParams);
-    hipLaunchKernelGGL(k_pack_inputs, dim3((B * kIn + 255) / 256), dim3(256), 0, p->stream,
-                       dx, B, p->x0);
-    rc = forward(p, B, p->stream);
+    hipLaunchKernelGGL(k_sum_grads, dim3((unsigned)(kParams / 256 + 1)), dim3(256), 0, p->stream,
+                       p->part, slices, dg, dg + kParams);
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpyAsync(grads, dg, kParams * 4, hipMemcpyDeviceToHost, p->stream) != hipSuccess ||
+        (loss && hipMemcpyAsync(loss, dg + kParams, 4, hipMemcpyDeviceToHost, p->stream) !=
+                     hipSuccess))
+      rc = FD2_E_DEVICE;
   }
-  if (!rc) rc = loss_grad(p, B, p->loss);
-  if (!rc) rc = backward(p, B);
-  if (!rc && (hipMemcpyAsync(grads, p->g, kParams * 4, hipMemcpyDeviceToHost, p->stream) != hipSuccess ||
-              (loss && hipMemcpyAsync(loss, p->loss, 4, hipMemcpyDeviceToHost, p->stream) != hipSuccess) ||
-              hipStreamSynchronize(p->stream) != hipSuccess))
-    rc = FD2_E_DEVICE;
-  (void)hipFree(dx);
+  if (hipStreamSynchronize(p->stream) != hipSuccess && !rc) rc = FD2_E_DEVICE;
+  (void)hipFree(d);
   return rc;
 }
 
@@ -885,7 +1110,7 @@ int fd2_mlp_train(fd2_mlp* p, int steps, int B, float lr, uint32_t seed, float* 
                   float* ms) {
   if (!p || steps < 0 || B <= 0 || B % 16 || p->n_data <= 0) return FD2_E_INVAL;
   MLP_HIP(hipSetDevice(p->device));
-  int rc = ensure_batch(p, B);
+  int rc = ensure_train(p, B);
   if (rc) return rc;
   // all minibatch indices drawn up front (xorshift64*, seeded)
   std::vector<uint32_t> idx((size_t)B * steps);
@@ -907,17 +1132,16 @@ int fd2_mlp_train(fd2_mlp* p, int steps, int B, float lr, uint32_t seed, float* 
            ? FD2_OK
            : FD2_E_DEVICE;
   for (int st = 0; st < steps && rc == FD2_OK; ++st) {
-    hipLaunchKernelGGL(k_gather, dim3((B * 64 + 255) / 256), dim3(256), 0, p->stream, p->data_x,
-                       p->data_y, d_idx + (size_t)st * B, B, p->x0, p->y);
-    rc = forward(p, B, p->stream);
-    if (!rc) rc = loss_grad(p, B, d_losses + st);
-    if (!rc) rc = backward(p, B);
-    if (rc) break;
+    const int slices = batch_gradients(p, p->data_x, p->data_y, d_idx + (size_t)st * B, B);
+    if (slices < 0) {
+      rc = slices;
+      break;
+    }
     p->step++;
     const float c1 = 1.0f - std::pow(b1, (float)p->step), c2 = 1.0f - std::pow(b2, (float)p->step);
-    hipLaunchKernelGGL(k_adam, dim3((unsigned)((kParams + 255) / 256)), dim3(256), 0, p->stream,
-                       p->w, p->g, p->m, p->v, p->wb, (int)kParams, lr, b1, b2, eps, c1, c2);
-    p->wt_stale = true;
+    hipLaunchKernelGGL(k_adam, dim3((unsigned)(kParams / 256 + 1)), dim3(256), 0, p->stream, p->w,
+                       p->part, slices, p->m, p->v, p->wb, p->wt, p->wg, d_losses + st, lr, b1, b2,
+                       eps, c1, c2);
     if (hipGetLastError() != hipSuccess) rc = FD2_E_DEVICE;
   }
   if (!rc && (hipEventRecord(p->e1, p->stream) != hipSuccess ||
