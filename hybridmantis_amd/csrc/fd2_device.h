@@ -204,23 +204,27 @@ __device__ __forceinline__ void tally_add(T* p, T v) {
                          __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// How a photon ended; its counter is fate - 1 (kDetect: counted before the
-// pixel is known, as kDetectOut).  kGone: a step of length -99, the
-// reference's own mark of a photon lost inside dist_to_surface.
+// How a photon ended (kNone: by a step of length -99, the reference's own mark
+// of a photon lost inside dist_to_surface).
 enum Fate : int {
   kNone = 0, kDetect = 1, kDetectOut = 2, kAbsTop = 3, kAbsBulk = 4,
-  kLost = 5, kOutOfCol = 6, kTheta1 = 7, kGone = 8
+  kLost = 5, kOutOfCol = 6, kTheta1 = 7
 };
 static_assert(kDetectOut - 1 == FD2_C_DETECT && kAbsTop - 1 == FD2_C_ABS_TOP &&
               kAbsBulk - 1 == FD2_C_ABS_BULK && kLost - 1 == FD2_C_LOST &&
-              kOutOfCol - 1 == FD2_C_OUTOFCOL && kTheta1 - 1 == FD2_C_THETA1 &&
-              kGone - 1 == FD2_C_REGEN, "fates in counter order");
+              kOutOfCol - 1 == FD2_C_OUTOFCOL && kTheta1 - 1 == FD2_C_THETA1,
+              "fates in counter order");
+// counter of an ended photon whose pixel is not known yet (kDetectOut)
+__device__ __forceinline__ int fate_counter(int fate) {
+  return fate == kNone ? (int)FD2_C_REGEN : fate - 1;
+}
 
 // photon state, all in registers.  The event's position and history stay
 // in the event record; the caller passes them where they are needed.
 // `st` is the photon's loop passes so far (kMaxLoops cap, 21 bits) and where
 // its next pass starts: kStResume after a reflection by the sensor (its next
-// in-column step is due), kStNewColumn when a crosstalk's neighbour-column
+// in-column step is due; the count is one less, as that pass counts again),
+// kStNewColumn when a crosstalk's neighbour-column
 // sample is due, with the samples rejected so far (<= 100) in bits 24-30.  One
 // word, so that a photon moves through the queues without packing.
 constexpr uint32_t kStLoops = 0x1fffffu, kStResume = 1u << 21, kStNewColumn = 1u << 31;
@@ -357,7 +361,7 @@ __device__ __forceinline__ void azimuth(float rr, Rng& rng, float& x, float& y) 
 template <class Rng, class M = MathDevice>
 __device__ __forceinline__ void rough_offset(Rng& rng, float& qx, float& qy, float& qz) {
   float s = rng.u();
-  qz = 2.0f * s - 1.0f;
+  qz = fmaf(2.0f, s, -1.0f);  // 2 s - 1, one rounding either way
   if constexpr (M::kFaithful) {
     // theta = s * 2.0f * pi with the double pi (K:3275), the double
     // cos/sin products and sqrt(pow + pow + pow) (K:3277-3285)
@@ -382,7 +386,9 @@ __device__ __forceinline__ void rough(Rng& rng, float& nx, float& ny, float& nz,
                                       float beta) {
   float qx, qy, qz;
   rough_offset<Rng, M>(rng, qx, qy, qz);
-  float rx = beta * qx + nx, ry = beta * qy + ny, rz = beta * qz + nz;
+  const float rx = beta * qx + nx, ry = beta * qy + ny;
+  // a normal in the plane (the constant 0) adds nothing
+  const float rz = __builtin_constant_p(nz) && nz == 0.0f ? beta * qz : beta * qz + nz;
   if constexpr (M::kFaithful) {
     const float nb = fd2x_norm3(rx, ry, rz);
     nx = rx / nb;
@@ -509,21 +515,21 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
   p.px = t0 + d * p.ux;
   p.py = t1 + d * p.uy;
 
-  int code = 0;
+  int code = kNone;
   uint32_t decisions = 0, iters = 0;  // traced nudge moves (1) / halvings (0)
   if (out_of_slab(p, g)) {
-    code = 1;
+    code = kLost;
   } else {
     const float dx = p.px - xc, dy = p.py - yc;
     float s = dx * dx + dy * dy;
     if (s > g.nudge_sq) {
       float step = 0.5f;
-      int moved = 0, shrunk = 0;
-      do {
+      bool farther = false;
+      auto nudge = [&]() {
         const float cx = p.px - step * p.ux, cy = p.py - step * p.uy;
         const float ex = cx - xc, ey = cy - yc;
         const float sc = ex * ex + ey * ey;
-        bool farther = sc > s;
+        farther = sc > s;
         if (farther) {
           asm volatile("");  // kept a branch: the roots are for a lane in 10^3
           farther = sqrtf(sc) > sqrtf(s);
@@ -534,13 +540,21 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
         p.px = farther ? p.px : cx;
         p.py = farther ? p.py : cy;
         s = farther ? s : sc;
-        moved += farther ? 0 : 1;
-        shrunk += farther ? 1 : 0;
-      } while (s > g.nudge_sq && moved < 10 && shrunk < 10);
+      };
+      nudge();  // nearly always enough
+      if (s > g.nudge_sq) {
+        asm volatile("");
+        int moved = farther ? 0 : 1, shrunk = farther ? 1 : 0;
+        do {
+          nudge();
+          moved += farther ? 0 : 1;
+          shrunk += farther ? 1 : 0;
+        } while (s > g.nudge_sq && moved < 10 && shrunk < 10);
+      }
       if (s > g.nudge_sq)
-        code = 2;
+        code = kOutOfCol;
       else if (outside_xy(p, g))
-        code = 1;
+        code = kLost;
     }
   }
   if (TRACE && sink->on) {
@@ -551,13 +565,13 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
       o[3] = p.ux; o[4] = p.uy; o[5] = p.uz;
       o[6] = xc; o[7] = yc;
       o[8] = p.px; o[9] = p.py; o[10] = p.pz;
-      o[11] = __int_as_float(code);
+      o[11] = __int_as_float(code == kLost ? 1 : code == kOutOfCol ? 2 : 0);
       o[12] = __int_as_float(sink->photon);
       o[13] = __uint_as_float(decisions | (iters << 20) | ((uint32_t)plane << 25));
     }
   }
-  if (code != 0) p.fate = code == 1 ? kLost : kOutOfCol;
-  return code != 0 ? -99.0f : d;
+  p.fate = code;
+  return code != kNone ? -99.0f : d;
 }
 
 // isotropic (main/kernel_cuda_c_ver1_0.cu:702-732): in-column step, then
@@ -566,7 +580,6 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
 template <class Rng, bool TRACE, class M = MathDevice>
 __device__ __forceinline__ bool isotropic(Rng& rng, Photon& p, const ColumnGeom& g,
                                           StepSink* sink) {
-  p.fate = kGone;
   const float ds = dist_to_surface<TRACE, M>(p, g, sink);
   const bool ended = fabsf(ds - (-99.0f)) < kEpsLt;
   const bool bulk = __float_as_uint(g.neg_inv_bulk) != 0u;
@@ -620,8 +633,9 @@ __device__ __forceinline__ int detection(Rng& rng, Photon& p, const ColumnGeom& 
 // (fd2_acos_small), evaluated only for a cosine in that band (about one in
 // 10^5).  |x| > 1 and NaN give a NaN angle, which is neither.
 __device__ __forceinline__ bool angle_over_157(float x) {
-  bool over = x >= -1.0f && x <= 7.90e-4f;
-  if (x > 7.90e-4f && x < 8.03e-4f) {
+  const bool below = x <= 7.90e-4f;
+  bool over = below && x >= -1.0f;
+  if (x < 8.03e-4f && !below) {
     asm volatile("");  // kept a branch
     over = fd2_acos_small(x) > 1.57f;
   }
@@ -1096,9 +1110,9 @@ __device__ __forceinline__ int hot_step(Rng& rng, Photon& p, const ColumnGeom& g
   if ((int32_t)p.st >= 0) {  // not kStNewColumn
     // a pass resumed after a sensor reflection is the rest of the previous
     // pass: no loop count, no second sensor check
-    const bool resumed = (p.st & kStResume) != 0u;
-    p.st = resumed ? p.st & kStLoops : p.st + 1u;
-    if (p.st > (uint32_t)kMaxLoops && !resumed) {
+    const bool resumed = p.st >= kStResume;
+    p.st = (p.st + 1u) & kStLoops;
+    if (p.st > (uint32_t)kMaxLoops) {
       p.fate = kLost;
       return kEnded;
     }
@@ -1108,7 +1122,7 @@ __device__ __forceinline__ int hot_step(Rng& rng, Photon& p, const ColumnGeom& g
     } else if (!resumed && fabsf(p.pz - (-g.half_h)) < kEpsLt) {
       const int d = detection<Rng, M>(rng, p, g);
       result = d == kSensorDetect ? kEnded : kAlive;
-      if (d == kSensorReflect) p.st |= kStResume;
+      if (d == kSensorReflect) p.st = (p.st - 1u) | kStResume;
     } else if (fabsf(p.uz) < kEpsLt) {
       result = kTrapped;
     } else if (fabsf(p.pz - g.half_h) < kEpsLt && p.uz > 0.0f) {

@@ -272,7 +272,7 @@ __device__ __forceinline__ void finish_photon(const TransportArgs& a, const Geom
                                               const fd2_event* __restrict__ events, Photon& p,
                                               uint32_t gi, uint32_t lane_ev, uint32_t lane_k,
                                               uint32_t* s_cnt, uint32_t* s_tile, uint32_t* run) {
-  atomicAdd(&s_cnt[gi * kCounters + p.fate - 1], 1u);
+  atomicAdd(&s_cnt[gi * kCounters + fate_counter(p.fate)], 1u);
   const bool det = p.fate == kDetectOut;
   Pixel x{0, 0};
   if (det) {
@@ -305,7 +305,7 @@ __device__ __forceinline__ void finish_photon(const TransportArgs& a, const Geom
   }
   if (REC) {
     fd2_photon rec;
-    rec.fate = p.fate == kGone ? kNone : p.fate;
+    rec.fate = p.fate;
     rec.pix = p.fate == kDetect ? pix_index(x, gt) : -1;
     rec.x = det ? p.px : 0.0f;
     rec.y = det ? p.py : 0.0f;
@@ -974,14 +974,14 @@ __global__ void __launch_bounds__(64) k_trace_ranecu(
         restart_trapped<RanecuRng, M>(rng, p, g, ev);
       }
     }
-    cnt[p.fate - 1]++;
+    cnt[fate_counter(p.fate)]++;
     const bool det = p.fate == kDetectOut;
     const Pixel x = det ? detected_pixel(p, g) : Pixel{0, 0};
     if (p.fate == kDetect) atomicAdd(&g.prf[pix_index(x, g)], 1ull);
     if (det && ev.hist >= 1 && ev.hist <= g.num_hist) atomicAdd(&g.hist[ev.hist - 1], 1u);
     if (records) {
       fd2_photon rec;
-      rec.fate = p.fate == kGone ? kNone : p.fate;
+      rec.fate = p.fate;
       rec.pix = p.fate == kDetect ? pix_index(x, g) : -1;
       rec.x = det ? p.px : 0.0f;
       rec.y = det ? p.py : 0.0f;

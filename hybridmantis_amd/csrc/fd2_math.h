@@ -135,6 +135,15 @@ FD2_HD unsigned int fd2_and_xor(unsigned int x, unsigned int m, unsigned int y) 
 #endif
 }
 
+/* m ? x : y bit by bit */
+FD2_HD unsigned int fd2_select(unsigned int m, unsigned int x, unsigned int y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(m, x, y, 0xCA);
+#else
+  return (m & x) | (~m & y);
+#endif
+}
+
 /* sin(pi t/2), cos(pi t/2) for 0 <= t <= 4: fd2_sincos_turns(t/4) with the
  * quadrant q = k mod 4 read from the low mantissa bits of t + 1.5*2^23 (that
  * sum is 0x4B400000 + k as an integer), and the swap and signs as bit
@@ -154,10 +163,15 @@ FD2_HD void fd2_sincos_quarters(float t, float* s, float* c) {
   qc = fmaf(z, qc, 4.166666791e-02f);
   const unsigned int cr = fd2_float_to_bits(fmaf(z * z, qc, fmaf(-0.5f, z, 1.0f)));
   const unsigned int q = fd2_float_to_bits(tb);
-  const unsigned int odd = 0u - (q & 1u); /* all ones in odd quadrants: swap */
-  const unsigned int hi = q << 30;        /* bit 31: quadrants 2, 3 */
-  *s = fd2_bits_to_float(fd2_and_xor(hi, 0x80000000u, (odd & cr) | (~odd & sr)));
-  *c = fd2_bits_to_float(fd2_and_xor(hi ^ odd, 0x80000000u, (odd & sr) | (~odd & cr)));
+#if defined(__HIP_DEVICE_COMPILE__)
+  const unsigned int odd = (unsigned int)__builtin_amdgcn_sbfe((int)q, 0, 1);
+#else
+  const unsigned int odd = 0u - (q & 1u);
+#endif
+  /* odd: all ones in odd quadrants (swap); bit 31 of hi: quadrants 2, 3 */
+  const unsigned int hi = q << 30;
+  *s = fd2_bits_to_float(fd2_and_xor(hi, 0x80000000u, fd2_select(odd, cr, sr)));
+  *c = fd2_bits_to_float(fd2_and_xor(hi ^ odd, 0x80000000u, fd2_select(odd, sr, cr)));
 }
 
 /* sqrtf(x) for x = +-0 and 2^-96 <= x <= 2^100: y = rsqrt estimate (1 ulp),
