@@ -208,8 +208,12 @@ __device__ __forceinline__ void tally_add(T* p, T v) {
 // of a photon lost inside dist_to_surface).
 enum Fate : int {
   kNone = 0, kDetect = 1, kDetectOut = 2, kAbsTop = 3, kAbsBulk = 4,
-  kLost = 5, kOutOfCol = 6, kTheta1 = 7
+  kLost = 5, kOutOfCol = 6, kTheta1 = 7,
+  // what follows an in-column pass of a photon that has not ended: the next
+  // pass, a restart, the wall's Fresnel branch, a sample of a direction
+  kAlive = 16, kTrapped, kWall, kSample, kSampleTop
 };
+__device__ __forceinline__ bool ended(int fate) { return fate < kAlive; }
 static_assert(kDetectOut - 1 == FD2_C_DETECT && kAbsTop - 1 == FD2_C_ABS_TOP &&
               kAbsBulk - 1 == FD2_C_ABS_BULK && kLost - 1 == FD2_C_LOST &&
               kOutOfCol - 1 == FD2_C_OUTOFCOL && kTheta1 - 1 == FD2_C_THETA1,
@@ -487,7 +491,7 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
     // dcyl is NaN for a negative, zero or infinite discriminant
     general = !((qa >= 0x1p-32f) & (dcyl <= g.wall_max) & (fabsf(p.uz) >= 0x1p-60f));
   }
-  if (general) {
+  if (M::kFaithful || __builtin_expect(general, 0)) {
     float r1, r2;
     if constexpr (M::kFaithful) {  // double root and quotients (K:992-998)
       fd2x_roots(qb, disc, 2.0f * qa, &r1, &r2);
@@ -517,45 +521,40 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
 
   int code = kNone;
   uint32_t decisions = 0, iters = 0;  // traced nudge moves (1) / halvings (0)
-  if (out_of_slab(p, g)) {
-    code = kLost;
-  } else {
-    const float dx = p.px - xc, dy = p.py - yc;
-    float s = dx * dx + dy * dy;
-    if (s > g.nudge_sq) {
-      float step = 0.5f;
-      bool farther = false;
-      auto nudge = [&]() {
-        const float cx = p.px - step * p.ux, cy = p.py - step * p.uy;
-        const float ex = cx - xc, ey = cy - yc;
-        const float sc = ex * ex + ey * ey;
-        farther = sc > s;
-        if (farther) {
-          asm volatile("");  // kept a branch: the roots are for a lane in 10^3
-          farther = sqrtf(sc) > sqrtf(s);
-        }
-        if (TRACE && !farther) decisions |= 1u << iters;
-        if (TRACE) ++iters;
-        step = farther ? step * 0.5f : step;
-        p.px = farther ? p.px : cx;
-        p.py = farther ? p.py : cy;
-        s = farther ? s : sc;
-      };
-      nudge();  // nearly always enough
-      if (s > g.nudge_sq) {
-        asm volatile("");
-        int moved = farther ? 0 : 1, shrunk = farther ? 1 : 0;
-        do {
-          nudge();
-          moved += farther ? 0 : 1;
-          shrunk += farther ? 1 : 0;
-        } while (s > g.nudge_sq && moved < 10 && shrunk < 10);
+  const bool lost = out_of_slab(p, g);
+  if (lost) code = kLost;
+  const float dx = p.px - xc, dy = p.py - yc;
+  float s = dx * dx + dy * dy;
+  if (!lost & (s > g.nudge_sq)) {
+    float step = 0.5f;
+    bool farther = false;
+    auto nudge = [&]() {
+      const float cx = p.px - step * p.ux, cy = p.py - step * p.uy;
+      const float ex = cx - xc, ey = cy - yc;
+      const float sc = ex * ex + ey * ey;
+      farther = sc > s;
+      if (__builtin_expect(farther, 0)) {
+        asm volatile("");  // kept a branch: the roots are for a lane in 10^3
+        farther = sqrtf(sc) > sqrtf(s);
       }
-      if (s > g.nudge_sq)
-        code = kOutOfCol;
-      else if (outside_xy(p, g))
-        code = kLost;
+      if (TRACE && !farther) decisions |= 1u << iters;
+      if (TRACE) ++iters;
+      step = farther ? step * 0.5f : step;
+      p.px = farther ? p.px : cx;
+      p.py = farther ? p.py : cy;
+      s = farther ? s : sc;
+    };
+    nudge();  // nearly always enough
+    if (__builtin_expect(s > g.nudge_sq, 0)) {
+      asm volatile("");
+      int moved = farther ? 0 : 1, shrunk = farther ? 1 : 0;
+      do {
+        nudge();
+        moved += farther ? 0 : 1;
+        shrunk += farther ? 1 : 0;
+      } while (s > g.nudge_sq && moved < 10 && shrunk < 10);
     }
+    code = s > g.nudge_sq ? kOutOfCol : outside_xy(p, g) ? kLost : kNone;
   }
   if (TRACE && sink->on) {
     const int slot = atomicAdd(sink->count, 1);
@@ -605,27 +604,6 @@ __device__ __forceinline__ bool isotropic(Rng& rng, Photon& p, const ColumnGeom&
   return ended || absorbed;
 }
 
-// detection (main/kernel_cuda_c_ver1_0.cu:3372-3427) of a photon on the
-// sensor plane: specular reflection with probability sensorRefl, else
-// detected.  The reference follows the reflection with another in-column step
-// inside the same pass; here the pass returns kSensorReflect and the caller
-// runs that step as the start of the next pass (hot_step), so the step's code
-// exists once.
-enum SensorResult : int { kSensorDetect = 1, kSensorReflect = 2 };
-
-template <class Rng, class M = MathDevice>
-__device__ __forceinline__ int detection(Rng& rng, Photon& p, const ColumnGeom& g) {
-  if (rng.u() < g.sensor_refl) {
-    p.nx = 0.0f;
-    p.ny = 0.0f;
-    p.nz = 1.0f;
-    reflect<M>(p, g);
-    return kSensorReflect;
-  }
-  p.fate = kDetectOut;
-  return kSensorDetect;
-}
-
 // fd2_acos(x) < 0 || fd2_acos(x) > 1.57 from comparisons.  The arc cosine
 // crosses 1.57 at x = cos(1.57) = 7.9633e-4; over all floats x in [-1, 1],
 // fd2_acos(x) >= 0, x <= 7.90e-4 gives an angle above 1.57 and x >= 8.03e-4
@@ -635,7 +613,7 @@ __device__ __forceinline__ int detection(Rng& rng, Photon& p, const ColumnGeom& 
 __device__ __forceinline__ bool angle_over_157(float x) {
   const bool below = x <= 7.90e-4f;
   bool over = below && x >= -1.0f;
-  if (x < 8.03e-4f && !below) {
+  if (__builtin_expect(x < 8.03e-4f && !below, 0)) {
     asm volatile("");  // kept a branch
     over = fd2_acos_small(x) > 1.57f;
   }
@@ -1082,7 +1060,7 @@ __device__ __forceinline__ bool ba_prpt(Rng& rng, Photon& p, const GeomDev& g) {
 // One algo() pass of the reference (main/kernel_cuda_c_ver1_0.cu:553-655)
 // fused with the boundary interaction that follows it: in-column step and
 // sensor check, then (if alive and not trapped) boundary_analysis up to its
-// Fresnel branch; kNeedPrpt asks the caller to run ba_prpt.
+// Fresnel branch, which the caller runs (fate kWall: ba_prpt).
 //
 // Crosstalk moves the photon to a neighbour column whose orientation is
 // sampled from -d until a sample passes the angle test, at most 101 samples
@@ -1100,46 +1078,51 @@ __device__ __forceinline__ bool ba_prpt(Rng& rng, Photon& p, const GeomDev& g) {
 // of roots took the kernel on mono25x50 (100,000 histories at 25 keV, 1.1e8
 // photons) from 972 to 810 vector instructions per photon and from 132 to
 // 118 ms, and a lone event of 1,375 photons from 1.84 to 1.48 ms.
-enum StepResult : int { kAlive = 0, kEnded = 1, kTrapped = 2, kNeedPrpt = 3 };
-
 template <class Rng, bool TRACE, class M = MathDevice>
-__device__ __forceinline__ int hot_step(Rng& rng, Photon& p, const ColumnGeom& g,
-                                        StepSink* sink) {
-  bool sample = true, top = false;
-  int result = kAlive;
-  if ((int32_t)p.st >= 0) {  // not kStNewColumn
-    // a pass resumed after a sensor reflection is the rest of the previous
-    // pass: no loop count, no second sensor check
-    const bool resumed = p.st >= kStResume;
-    p.st = (p.st + 1u) & kStLoops;
-    if (p.st > (uint32_t)kMaxLoops) {
-      p.fate = kLost;
-      return kEnded;
-    }
-    sample = false;
-    if (isotropic<Rng, TRACE, M>(rng, p, g, sink)) {
-      result = kEnded;
-    } else if (!resumed && fabsf(p.pz - (-g.half_h)) < kEpsLt) {
-      const int d = detection<Rng, M>(rng, p, g);
-      result = d == kSensorDetect ? kEnded : kAlive;
-      if (d == kSensorReflect) p.st = (p.st - 1u) | kStResume;
-    } else if (fabsf(p.uz) < kEpsLt) {
-      result = kTrapped;
-    } else if (fabsf(p.pz - g.half_h) < kEpsLt && p.uz > 0.0f) {
-      // top reflector reached inside a column
-      sample = top = true;
-      if (g.top_absfrac > 0.0f && rng.u() < g.top_absfrac) {
-        p.fate = kAbsTop;
-        sample = false;
-        result = kEnded;
+__device__ __forceinline__ void hot_step(Rng& rng, Photon& p, const ColumnGeom& g,
+                                         StepSink* sink) {
+  const bool again = (int32_t)p.st < 0;  // kStNewColumn: only a sample
+  // a pass resumed after a sensor reflection is the rest of the previous
+  // pass: no loop count, no second sensor check
+  const bool resumed = p.st >= kStResume;
+  if (!again) p.st = (p.st + 1u) & kStLoops;
+  p.fate = again ? kSample : kLost;
+  if (!again & (p.st <= (uint32_t)kMaxLoops)) {
+    const bool gone = isotropic<Rng, TRACE, M>(rng, p, g, sink);
+    // what the photon has reached: the sensor plane, nothing (it moves within
+    // a plane z = const), the top reflector inside a column, else the wall
+    const bool sensor = !resumed & (fabsf(p.pz - (-g.half_h)) < kEpsLt);
+    const bool flat = !sensor & (fabsf(p.uz) < kEpsLt);
+    const bool top = (fabsf(p.pz - g.half_h) < kEpsLt) & (p.uz > 0.0f);
+    // one draw decides: specular reflection by the sensor
+    // (main/kernel_cuda_c_ver1_0.cu:3372-3427, else detected), absorption at
+    // the top, crosstalk at the wall
+    if (!gone) {
+      int fate = kTrapped;
+      if (!flat) {
+        const float cct = crosstalk<M>(p.pz, g);
+        const float limit = sensor ? g.sensor_refl : top ? g.top_absfrac : cct;
+        const bool drawn = sensor | !top | (g.top_absfrac > 0.0f);
+        bool hit = false;
+        if (drawn) hit = rng.u() < limit;
+        fate = sensor ? (hit ? kAlive : kDetectOut)
+                      : top ? (hit ? kAbsTop : kSampleTop) : (hit ? kSample : kWall);
+        if (sensor & hit) {
+          // the reference follows the reflection with another in-column step
+          // inside the same pass; here that step is the start of the next
+          // pass, so its code exists once
+          p.nx = 0.0f;
+          p.ny = 0.0f;
+          p.nz = 1.0f;
+          reflect<M>(p, g);
+          p.st = (p.st - 1u) | kStResume;
+        }
       }
-    } else {
-      const float cct = crosstalk<M>(p.pz, g);
-      sample = rng.u() < cct;
-      result = sample ? kAlive : kNeedPrpt;
+      p.fate = fate;
     }
   }
-  if (sample) {
+  if (p.fate >= kSample) {
+    const bool top = p.fate == kSampleTop;
     float qx, qy, w, nx, ny, nz = 0.0f;
     const float mx = -p.ux, my = -p.uy, mz = -p.uz;
     if constexpr (M::kFaithful) {
@@ -1175,28 +1158,21 @@ __device__ __forceinline__ int hot_step(Rng& rng, Photon& p, const ColumnGeom& g
         if (g.beta > 0.0f) rough<Rng, M>(rng, nx, ny, nz, g.beta);
         over = angle_over<M>(mx * nx + my * ny + mz * nz);
       }
-      if (!over) {
-        p.xc = p.px - g.R * nx;
-        p.yc = p.py - g.R * ny;
-        p.st &= kStLoops;
-      } else if ((p.st >> kStRejected) == (kStNewColumn >> kStRejected) + 100u) {
-        p.fate = kTheta1;
-        result = kEnded;
-      } else {
-        p.st = (p.st | kStNewColumn) + (1u << kStRejected);
-      }
+      const bool last = over & ((p.st >> kStRejected) == (kStNewColumn >> kStRejected) + 100u);
+      p.xc = over ? p.xc : p.px - g.R * nx;
+      p.yc = over ? p.yc : p.py - g.R * ny;
+      p.st = over ? (p.st | kStNewColumn) + (1u << kStRejected) : p.st & kStLoops;
+      p.fate = last ? kTheta1 : kAlive;
     }
   }
-  return result;
 }
 
 // the whole pass, for kernels that do not defer the Fresnel branch
 template <class Rng, bool TRACE, class M = MathDevice>
-__device__ __forceinline__ int photon_step(Rng& rng, Photon& p,
-                                           const GeomDev& g, StepSink* sink) {
-  const int r = hot_step<Rng, TRACE, M>(rng, p, g, sink);
-  if (r != kNeedPrpt) return r;
-  return ba_prpt<Rng, M>(rng, p, g) ? kEnded : kAlive;
+__device__ __forceinline__ void photon_step(Rng& rng, Photon& p, const GeomDev& g,
+                                            StepSink* sink) {
+  hot_step<Rng, TRACE, M>(rng, p, g, sink);
+  if (p.fate == kWall) p.fate = ba_prpt<Rng, M>(rng, p, g) ? p.fate : (int)kAlive;
 }
 
 // trapped photon (|dcos.z| < eps): restart from the event with a new

@@ -225,6 +225,7 @@ Launch make_launch(const fd2_ctx* c, const QueueBufs& b, const fd2_event* d_ev, 
   TransportArgs& a = L.a;
   a.events = d_ev;
   a.photon_off = b.photon_off;
+  a.geom0 = c->hgeom[0];
   a.geoms = c->d_geoms;
   a.counters = c->d_counters;
   a.plan = q.plan;

@@ -19,6 +19,9 @@ struct QueuePlan {
 };
 
 struct TransportArgs {
+  // geometry 0, first in the kernel's arguments: with one geometry its
+  // constants are one scalar load away, not two
+  GeomDev geom0;
   const fd2_event* events;             // device
   const unsigned long long* photon_off;  // n_events + 1 (exclusive scan)
   const GeomDev* geoms;                // n_geoms

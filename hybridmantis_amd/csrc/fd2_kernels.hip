@@ -413,6 +413,17 @@ __device__ __forceinline__ T load_uniform(const void* p) {
   return c;
 }
 
+__device__ __forceinline__ ColumnGeom load_column(const void* p) {
+  typedef uint32_t Words __attribute__((ext_vector_type(16)));
+  auto one = (const __attribute__((address_space(4))) Words*)p;
+  asm volatile("" : "+s"(one));
+  Words w = *one;
+  asm volatile("" : "+s"(w));
+  ColumnGeom g;
+  __builtin_memcpy(&g, &w, sizeof g);
+  return g;
+}
+
 // Event of photon g of the launch: the largest e with photon_off[e] <= g
 // (skips events without photons).  Each round the 64 lanes (all active) probe
 // 64 points of [lo, hi) with one vector load, and the wave keeps the step
@@ -587,7 +598,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     if constexpr (MULTI)
       f(geoms[gi]);
     else
-      f(load_uniform<GeomDev>(geoms_in));
+      f(load_uniform<GeomDev>(kernarg));
   };
   auto finish = [&](unsigned long long m) {
     if (in(m))
@@ -689,7 +700,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
               counter_initial_dir(r, q, k, geoms[ev.geom]);
               atomicAdd(&s_cnt[ev.geom * kCounters + FD2_C_GENERATED], 1u);
             } else {
-              counter_initial_dir(r, q, k, load_uniform<ColumnGeom>(geoms_in));
+              counter_initial_dir(r, q, k, load_uniform<ColumnGeom>(kernarg));
               if (lane == 0) atomicAdd(&s_cnt[FD2_C_GENERATED], n);
             }
             q_put<MULTI, REC, kWallSlots>(lq + (uint32_t)kWallSlots - n + lane, q, r, e,
@@ -739,8 +750,9 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
       int r = kAlive;
       if (in(step_m)) {
         auto pass = [&](const ColumnGeom& g) {
-          r = hot_step<CounterRng, false>(rng, p, g, &nosink);
-          if (r == kTrapped) {
+          hot_step<CounterRng, false>(rng, p, g, &nosink);
+          r = p.fate;
+          if (__builtin_expect(r == kTrapped, 0)) {
             atomicAdd(&s_cnt[gi * kCounters + FD2_C_REGEN], 1u);
             restart_trapped(rng, p, g, events[lane_ev]);
           }
@@ -748,9 +760,9 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         if constexpr (MULTI)
           pass(geoms[gi]);
         else
-          pass(load_uniform<ColumnGeom>(geoms_in));
+          pass(load_column(kernarg));
       }
-      const unsigned long long e = __ballot(r == kEnded), w = __ballot(r == kNeedPrpt);
+      const unsigned long long e = __ballot(ended(r)), w = __ballot(r == kWall);
       end_m |= e;
       wall_m |= w;
       step_m &= ~(e | w);
@@ -967,9 +979,9 @@ __global__ void __launch_bounds__(64) k_trace_ranecu(
     p.nx = nx; p.ny = ny; p.nz = nz;
     cnt[FD2_C_GENERATED]++;
     for (;;) {
-      const int r = photon_step<RanecuRng, false, M>(rng, p, g, &nosink);
-      if (r == kEnded) break;
-      if (r == kTrapped) {
+      photon_step<RanecuRng, false, M>(rng, p, g, &nosink);
+      if (ended(p.fate)) break;
+      if (p.fate == kTrapped) {
         cnt[FD2_C_REGEN]++;
         restart_trapped<RanecuRng, M>(rng, p, g, ev);
       }
@@ -1034,9 +1046,9 @@ __global__ void __launch_bounds__(64) k_debug_steps(
   rng.seed(seed, event_base, (uint32_t)k);
   counter_initial_dir(rng, p, (uint32_t)k, g);
   for (;;) {
-    const int r = photon_step<CounterRng, true>(rng, p, g, &sink);
-    if (r == kEnded) break;
-    if (r == kTrapped) restart_trapped(rng, p, g, ev);
+    photon_step<CounterRng, true>(rng, p, g, &sink);
+    if (ended(p.fate)) break;
+    if (p.fate == kTrapped) restart_trapped(rng, p, g, ev);
   }
 }
 
