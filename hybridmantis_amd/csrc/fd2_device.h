@@ -438,7 +438,9 @@ __device__ __forceinline__ void emit_first_dir(Rng& rng, Photon& p,
 // ---------------------------------------------------------- transport
 
 __device__ __forceinline__ bool outside_xy(const Photon& p, const ColumnGeom& g) {
-  return p.px < kEpsLt || p.px > g.xdet || p.py < kEpsLt || p.py > g.ydet;
+  float eps = kEpsLt;  // opaque: the compiler would make one comparison of a
+  asm volatile("" : "+s"(eps));  // minimum, with two more instructions
+  return (p.px < kEpsLt) | (p.px > g.xdet) | (p.py < eps) | (p.py > g.ydet);
 }
 
 __device__ __forceinline__ bool out_of_slab(const Photon& p, const ColumnGeom& g) {
@@ -527,34 +529,36 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
   float s = dx * dx + dy * dy;
   if (!lost & (s > g.nudge_sq)) {
     float step = 0.5f;
-    bool farther = false;
+    int moved = 0, shrunk = 0;
+    // one try; a candidate farther out halves the step instead.  The move is
+    // the ordinary outcome, so the other one undoes it in a branch.
     auto nudge = [&]() {
-      const float cx = p.px - step * p.ux, cy = p.py - step * p.uy;
-      const float ex = cx - xc, ey = cy - yc;
-      const float sc = ex * ex + ey * ey;
-      farther = sc > s;
-      if (__builtin_expect(farther, 0)) {
-        asm volatile("");  // kept a branch: the roots are for a lane in 10^3
-        farther = sqrtf(sc) > sqrtf(s);
+      const float ox = p.px, oy = p.py, os = s;
+      p.px = ox - step * p.ux;
+      p.py = oy - step * p.uy;
+      const float ex = p.px - xc, ey = p.py - yc;
+      s = ex * ex + ey * ey;
+      bool farther = false;
+      if (__builtin_expect(s > os, 0)) {
+        farther = sqrtf(s) > sqrtf(os);
+        if (farther) {
+          p.px = ox;
+          p.py = oy;
+          s = os;
+          step = step * 0.5f;
+          ++shrunk;
+        }
       }
       if (TRACE && !farther) decisions |= 1u << iters;
       if (TRACE) ++iters;
-      step = farther ? step * 0.5f : step;
-      p.px = farther ? p.px : cx;
-      p.py = farther ? p.py : cy;
-      s = farther ? s : sc;
+      ++moved;
     };
     nudge();  // nearly always enough
     if (__builtin_expect(s > g.nudge_sq, 0)) {
-      asm volatile("");
-      int moved = farther ? 0 : 1, shrunk = farther ? 1 : 0;
-      do {
-        nudge();
-        moved += farther ? 0 : 1;
-        shrunk += farther ? 1 : 0;
-      } while (s > g.nudge_sq && moved < 10 && shrunk < 10);
+      do nudge(); while (s > g.nudge_sq && moved - shrunk < 10 && shrunk < 10);
+      if (s > g.nudge_sq) code = kOutOfCol;
     }
-    code = s > g.nudge_sq ? kOutOfCol : outside_xy(p, g) ? kLost : kNone;
+    if (outside_xy(p, g)) code = code > (int)kLost ? code : (int)kLost;
   }
   if (TRACE && sink->on) {
     const int slot = atomicAdd(sink->count, 1);
@@ -593,7 +597,7 @@ __device__ __forceinline__ bool isotropic(Rng& rng, Photon& p, const ColumnGeom&
     // logarithm's error and the roundings, checked for every u the kernel
     // draws); only the remaining steps need the logarithm, and the outcome
     // is the same
-    if (!(ds < ((1.0f - u) * -g.neg_inv_bulk) * 0.99999904632568359375f)) {
+    if (__builtin_expect(!(ds < ((1.0f - u) * -g.neg_inv_bulk) * 0.99999904632568359375f), 0)) {
       const float da = g.neg_inv_bulk * fd2_log(u);
       absorbed = ds >= da && ds >= 0.0f;
     }
@@ -841,15 +845,18 @@ top:
 // [-H/2, H/2] or is NaN (then no crosstalk).
 template <class M>
 __device__ __forceinline__ float crosstalk(float z, const ColumnGeom& g) {
-  const bool upper = z >= 0.0f;
-  const float num = upper ? z : z + g.half_h;
-  const float den = upper ? g.den_up : g.den_dn;
-  float q;
-  if constexpr (M::kFaithful)
-    q = num / den;
-  else
-    q = fd2_div_by(num, den, upper ? g.inv_up : g.inv_dn);
-  const float c = q + (upper ? 0.5f : 1.0f);
+  // both pieces from the uniform constants: selecting the constants instead
+  // takes more instructions
+  const float zl = z + g.half_h;
+  float qu, ql;
+  if constexpr (M::kFaithful) {
+    qu = z / g.den_up;
+    ql = zl / g.den_dn;
+  } else {
+    qu = fd2_div_by(z, g.den_up, g.inv_up);
+    ql = fd2_div_by(zl, g.den_dn, g.inv_dn);
+  }
+  const float c = z >= 0.0f ? qu + 0.5f : ql + 1.0f;
   return z >= g.top20 ? 1.0f : c;
 }
 
@@ -1158,7 +1165,7 @@ __device__ __forceinline__ void hot_step(Rng& rng, Photon& p, const ColumnGeom& 
         if (g.beta > 0.0f) rough<Rng, M>(rng, nx, ny, nz, g.beta);
         over = angle_over<M>(mx * nx + my * ny + mz * nz);
       }
-      const bool last = over & ((p.st >> kStRejected) == (kStNewColumn >> kStRejected) + 100u);
+      const bool last = over & (p.st >= kStNewColumn + (100u << kStRejected));
       p.xc = over ? p.xc : p.px - g.R * nx;
       p.yc = over ? p.yc : p.py - g.R * ny;
       p.st = over ? (p.st | kStNewColumn) + (1u << kStRejected) : p.st & kStLoops;

@@ -232,8 +232,8 @@ Launch make_launch(const fd2_ctx* c, const QueueBufs& b, const fd2_event* d_ev, 
   a.records = d_records;
   a.radial = d_radial;
   a.event_base_dev = nullptr;
-  const bool queue = c->tune.wall_queue >= 0 && c->d_wave_queue != nullptr;
-  a.wave_queue = queue ? c->d_wave_queue : nullptr;
+  a.wave_queue = c->d_wave_queue;
+  a.queues = c->tune.wall_queue >= 0;
   a.error_flag = q.error_flag;
   a.n_events = n;
   a.seed = c->seed;
@@ -251,7 +251,7 @@ Launch make_launch(const fd2_ctx* c, const QueueBufs& b, const fd2_event* d_ev, 
                                             (size_t)a.n_tiles * a.tile_side * a.tile_side);
   const int occ = transport_max_blocks_per_cu(L.multi, L.record, L.radial, smem);
   L.blocks = c->n_cu * (per_cu < 1 ? 1 : (per_cu > occ ? occ : per_cu));
-  if (queue && L.blocks * (kTransportThreads / 64) > c->max_waves)
+  if (L.blocks * (kTransportThreads / 64) > c->max_waves)
     L.blocks = c->max_waves / (kTransportThreads / 64);
   q.n_simds = (uint32_t)(c->n_cu * 4);
   q.n_waves = (uint32_t)(L.blocks * (kTransportThreads / 64));
@@ -472,7 +472,7 @@ int fd2_create(const fd2_params* params, int n_geoms, int device, fd2_ctx** out)
         if (o > occ) occ = o;
       }
       c->max_waves = c->n_cu * occ * (kTransportThreads / 64);
-      const size_t qbytes = (size_t)c->max_waves * kQWords * kQSlots * sizeof(uint32_t);
+      const size_t qbytes = (size_t)c->max_waves * kWaveWords * sizeof(uint32_t);
       if (hipMalloc(&c->d_wave_queue, qbytes) != hipSuccess) { rc = FD2_E_NOMEM; break; }
     }
     if (launch_fill_u32(c->d_error, 1, c->stream) != hipSuccess) { rc = FD2_E_DEVICE; break; }

@@ -30,7 +30,8 @@ struct TransportArgs {
   fd2_photon* records;                 // per-photon records (recording only)
   uint32_t* radial;                    // n_events x FD2_RADIAL_BINS (radial mode)
   const unsigned long long* event_base_dev;  // if set, read the number of events[0] here
-  uint32_t* wave_queue;                // per-wave photon queues (null: park in place)
+  uint32_t* wave_queue;                // per-wave photon queues
+  int32_t queues;                      // use them (0: park in place)
   uint32_t* error_flag;                // bit 1: a wave's loop limit was reached
   int64_t n_events;
   uint32_t seed;
@@ -62,6 +63,10 @@ constexpr int kBackBase = kGapCap;
 constexpr int kQSlots = kGapCap + kBackCap;
 constexpr int kQWords = 20;  // 16 photon words + 4 of wall-branch state
 constexpr int kQBlock = 32;  // queue slots per block (word stride 128 bytes)
+// ended photons that wait to be counted: 63 between rounds, and at most every
+// photon in flight ends in one; 5 words each, kEndCap apart
+constexpr int kEndCap = 64 + 64 + kLdsCap + kGapCap;
+constexpr int kWaveWords = kQWords * kQSlots + 5 * kEndCap;
 static_assert(kQSlots % kQBlock == 0 && kGapBase % kQBlock == 0 && kBackBase % kQBlock == 0,
               "queue regions are whole blocks");
 constexpr uint32_t kMaxIdlePasses = 256;  // passes without a step or a wall branch
@@ -152,7 +157,7 @@ struct fd2_ctx {
   size_t cap_blocks = 0;
   fd2::QueuePlan* d_plan = nullptr;
   uint32_t* d_error = nullptr;
-  uint32_t* d_wave_queue = nullptr;    // kQWords x kQSlots words per resident wave
+  uint32_t* d_wave_queue = nullptr;    // kWaveWords words per resident wave
   int max_waves = 0;
 
   uint32_t seed = 271828182u;

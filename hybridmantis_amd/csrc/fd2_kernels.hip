@@ -571,21 +571,20 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
 
   Photon p;
   CounterRng rng;
-  unsigned long long step_m = 0, wall_m = 0, end_m = 0;
+  unsigned long long step_m = 0, wall_m = 0;
   uint32_t gi = 0;
   uint32_t lane_ev = 0;  // the lane's event (index into events)
   uint32_t lane_k = 0;   // photon index within the event
   StepSink nosink{nullptr, nullptr, 0, 0, false};
 
   uint32_t* lq = &s_queue[wave][0][0];
-  uint32_t* wq = nullptr;  // gap queue [0, n_gap), backlog [0, n_back)
-  uint32_t n_wall = 0, n_ready = 0, n_gap = 0, n_back = 0, idle = 0;
-  if (a.wave_queue)
-    wq = a.wave_queue + (size_t)(blockIdx.x * (kTransportThreads / 64) + wave) *
-                            (kQWords * kQSlots);
+  // the wave's queues in HBM: gap queue [0, n_gap), backlog [0, n_back), ended
+  // photons [0, n_end)
+  uint32_t* wq = a.wave_queue + (size_t)(blockIdx.x * (kTransportThreads / 64) + wave) * kWaveWords;
+  uint32_t n_wall = 0, n_ready = 0, n_gap = 0, n_back = 0, n_end = 0, idle = 0;
   const uint32_t lane_cap = a.plan->lane_cap;
-  const bool queued = a.wave_queue != nullptr && lane_cap == 64u;
-  const uint32_t park = a.wave_queue ? 0u : (uint32_t)a.park_lanes;
+  const bool queued = a.queues != 0 && lane_cap == 64u;
+  const uint32_t park = a.queues != 0 ? 0u : (uint32_t)a.park_lanes;
   const uint32_t serve_at = min((uint32_t)a.refill_lanes, lane_cap);
   const unsigned long long use_m = lane_cap == 64u ? ~0ull : (1ull << lane_cap) - 1ull;
 
@@ -600,12 +599,42 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     else
       f(load_uniform<GeomDev>(kernarg));
   };
-  auto finish = [&](unsigned long long m) {
-    if (in(m))
-      with_geom([&](const GeomDev& g) {
-        finish_photon<MULTI, REC, RADIAL>(args(), g, geoms, events, p, gi, lane_ev, lane_k, s_cnt,
-                                          s_tile, run);
-      });
+  // Ended photons wait in HBM until 64 of them are counted at once: about one
+  // lane of a wave ends in two passes, and its tallies are as long as a third
+  // of a pass.
+  auto end_put = [&](unsigned long long m) {
+    if (m == 0ull) return;
+    if (in(m)) {
+      uint32_t* w = wq + kQWords * kQSlots + n_end + rank_below(m);
+      w[0] = (uint32_t)p.fate | (MULTI ? gi << 8 : 0u);
+      w[kEndCap] = __float_as_uint(p.px);
+      w[2 * kEndCap] = __float_as_uint(p.py);
+      w[3 * kEndCap] = lane_ev;
+      if (REC) w[4 * kEndCap] = lane_k;
+    }
+    n_end += count(m);
+  };
+  auto end_count = [&]() {
+    const uint32_t t = min(n_end, 64u);
+    n_end -= t;
+    __threadfence_block();  // the wave's queue stores are complete before its loads
+    if ((uint32_t)lane < t) {
+      const uint32_t* w = wq + kQWords * kQSlots + n_end + lane;
+      Photon q;
+      q.fate = (int)(w[0] & 0xffu);
+      const uint32_t g2 = MULTI ? w[0] >> 8 : 0u;
+      q.px = __uint_as_float(w[kEndCap]);
+      q.py = __uint_as_float(w[2 * kEndCap]);
+      const uint32_t ev = w[3 * kEndCap], k = REC ? w[4 * kEndCap] : 0u;
+      const auto count_one = [&](const GeomDev& g) {
+        finish_photon<MULTI, REC, RADIAL>(args(), g, geoms, events, q, g2, ev, k, s_cnt, s_tile,
+                                          run);
+      };
+      if constexpr (MULTI)
+        count_one(geoms[g2]);
+      else
+        count_one(load_uniform<GeomDev>(kernarg));
+    }
   };
   auto lds_put = [&](uint32_t slot) {
     q_put<MULTI, REC, kWallSlots>(lq + slot, p, rng, lane_ev, gi, lane_k);
@@ -628,17 +657,21 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     step_m |= __ballot(got);
   };
 
+  bool last = false;  // no photon is left; the ended ones are still to be counted
   for (;;) {
+    if (n_end >= 64u || last) {
+      end_count();
+      if (last && n_end == 0u) break;
+      if (last) continue;
+    }
     unsigned long long gap_m = 0;  // lanes whose photon's gap flight is next
     PrptState st = prpt_initial();
     bool drain = pool_done && n_ready == 0u && n_back == 0u;
     // ---- serve
     {
       const unsigned long long waiting = drain || !queued ? wall_m : 0ull;
-      const bool due = !drain || end_m != 0ull || n_wall != 0u || n_gap != 0u;
+      const bool due = !drain || n_wall != 0u || n_gap != 0u;
       if (step_m == 0ull || (due && count(use_m & ~(step_m | waiting)) >= serve_at)) {
-        if (end_m != 0ull) finish(end_m);
-        end_m = 0ull;
         if (queued && !drain && n_wall + count(wall_m) < 64u) {
           while (wall_m != 0ull) {
             const uint32_t k =
@@ -738,7 +771,8 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
           }
         }
         // nothing in a lane: the queues and the work queue are empty
-        if ((step_m | wall_m | gap_m) == 0ull) break;
+        last = (step_m | wall_m | gap_m) == 0ull;
+        if (last) continue;
       }
     }
     // every round steps a photon or runs a phase; a wave that does neither
@@ -763,7 +797,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
           pass(load_column(kernarg));
       }
       const unsigned long long e = __ballot(ended(r)), w = __ballot(r == kWall);
-      end_m |= e;
+      end_put(e);
       wall_m |= w;
       step_m &= ~(e | w);
     }
@@ -777,8 +811,6 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         (n_step == 0u || n_lane >= (park != 0u ? park : n_step));
     if (full || place) {
       progress = true;
-      if (end_m != 0ull) finish(end_m);
-      end_m = 0ull;
       if (full) {
         // every lane without a waiting photon takes one; a photon that was
         // stepping takes a ready slot (all reads come before the writes)
@@ -808,9 +840,10 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
       const bool mine = in(wall_m);
       if (mine)
         with_geom([&](const GeomDev& g) { r = prpt_loop(rng, p, g, st, true, true); });
-      end_m = __ballot(mine && r == kPrEnded);
+      const unsigned long long e = __ballot(mine && r == kPrEnded);
       const unsigned long long flight = __ballot(mine && r == kPrGap);
-      step_m |= wall_m & ~(end_m | flight);
+      end_put(e);
+      step_m |= wall_m & ~(e | flight);
       gap_m |= flight;
       wall_m = 0ull;
     }
@@ -831,8 +864,6 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
           gap_m = 0ull;
         }
         if (n_gap < 64u) break;
-        if (end_m != 0ull) finish(end_m);
-        end_m = 0ull;
         const uint32_t s = count(step_m);
         if (n_back + s > (uint32_t)kBackCap) {  // ruled out by the photons in flight
           failed = true;
@@ -859,7 +890,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         with_geom([&](const GeomDev& g) { r = prpt_loop(rng, p, g, st, false, true); });
       const unsigned long long e = __ballot(mine && r == kPrEnded);
       const unsigned long long again = __ballot(mine && r == kPrGap);
-      end_m |= e;
+      end_put(e);
       step_m |= gap_m & ~(e | again);
       gap_m = again;
     }
