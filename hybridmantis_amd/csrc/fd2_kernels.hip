@@ -657,22 +657,22 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     step_m |= __ballot(got);
   };
 
+  // How waiting photons are served, decided in each serve: 0 through the
+  // queues, 1 in their lanes (no queues, or a small launch), 2 in their lanes
+  // while the wave drains.  A serve is due once at most busy_max lanes step
+  // (or, in place, wait).
+  int mode = queued ? 0 : 1;
+  int busy_max = (int)(lane_cap - serve_at);
   bool last = false;  // no photon is left; the ended ones are still to be counted
   for (;;) {
-    if (n_end >= 64u || last) {
-      end_count();
-      if (last && n_end == 0u) break;
-      if (last) continue;
-    }
     unsigned long long gap_m = 0;  // lanes whose photon's gap flight is next
     PrptState st = prpt_initial();
-    bool drain = pool_done && n_ready == 0u && n_back == 0u;
     // ---- serve
-    {
-      const unsigned long long waiting = drain || !queued ? wall_m : 0ull;
-      const bool due = !drain || n_wall != 0u || n_gap != 0u;
-      if (step_m == 0ull || (due && count(use_m & ~(step_m | waiting)) >= serve_at)) {
-        if (queued && !drain && n_wall + count(wall_m) < 64u) {
+    if (step_m == 0ull || (int)count(mode == 0 ? step_m : step_m | wall_m) <= busy_max) {
+      while (n_end >= 64u || (last && n_end != 0u)) end_count();
+      if (last) break;
+      {
+        if (mode == 0 && n_wall + count(wall_m) < 64u) {
           while (wall_m != 0ull) {
             const uint32_t k =
                 min(count(wall_m), (uint32_t)kWallSlots - n_wall - n_ready);
@@ -745,7 +745,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
           take_ready(need);
           need = use_m & ~(step_m | wall_m);
         }
-        drain = pool_done && n_ready == 0u && n_back == 0u;
+        const bool drain = pool_done && n_ready == 0u && n_back == 0u;
         if (drain && queued && need != 0ull && (n_wall | n_gap) != 0u) {
           // the queues' last photons back into free lanes
           uint32_t t = min(count(need), n_wall);
@@ -771,14 +771,13 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
           }
         }
         // nothing in a lane: the queues and the work queue are empty
+        mode = drain ? 2 : queued ? 0 : 1;
+        busy_max = drain && (n_wall | n_gap) == 0u ? -1 : (int)(lane_cap - serve_at);
         last = (step_m | wall_m | gap_m) == 0ull;
         if (last) continue;
       }
     }
-    // every round steps a photon or runs a phase; a wave that does neither
-    // for many rounds has a broken queue state: it stops and flags the launch
-    // rather than spin
-    bool progress = step_m != 0ull;
+    const bool stepped = step_m != 0ull;
     // ---- pass
     {
       int r = kAlive;
@@ -802,16 +801,22 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
       step_m &= ~(e | w);
     }
     // ---- wall
-    drain = pool_done && n_ready == 0u && n_back == 0u;
-    const bool in_place = drain || !queued;
     const uint32_t n_lane = count(wall_m), n_step = count(step_m);
-    const bool full = !in_place && n_wall + n_lane >= 64u;
-    const bool place =
-        in_place && n_lane != 0u &&
-        (n_step == 0u || n_lane >= (park != 0u ? park : n_step));
-    if (full || place) {
-      progress = true;
-      if (full) {
+    const bool in_place = mode != 0;
+    bool wall = n_wall + n_lane >= 64u;
+    if (in_place) wall = n_lane != 0u && (n_step == 0u || n_lane >= (park != 0u ? park : n_step));
+    // every round steps a photon or runs a phase; a wave that does neither
+    // for many rounds has a broken queue state: it stops and flags the launch
+    // rather than spin
+    if (stepped || wall || gap_m != 0ull) {
+      idle = 0;
+    } else if (++idle > kMaxIdlePasses) {
+      if (lane == 0) atomicOr(args().error_flag, 2u);
+      break;
+    }
+    if (!wall && gap_m == 0ull) continue;
+    if (wall) {
+      if (!in_place) {
         // every lane without a waiting photon takes one; a photon that was
         // stepping takes a ready slot (all reads come before the writes)
         const unsigned long long need = ~wall_m;
@@ -883,7 +888,6 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
       } else if (gap_m == 0ull) {
         break;
       }
-      progress = true;
       int r = kPrAlive;
       const bool mine = in(gap_m);
       if (mine)
@@ -893,11 +897,6 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
       end_put(e);
       step_m |= gap_m & ~(e | again);
       gap_m = again;
-    }
-    if (progress) {
-      idle = 0;
-    } else if (++idle > kMaxIdlePasses) {
-      failed = true;
     }
     if (failed) {
       if (lane == 0) atomicOr(args().error_flag, 2u);
