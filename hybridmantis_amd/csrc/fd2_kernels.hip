@@ -400,6 +400,12 @@ __device__ __forceinline__ bool in(unsigned long long mask) {
   return __builtin_amdgcn_inverse_ballot_w64(mask);
 }
 
+// the lowest `t` lanes of a mask, given their ranks in it
+__device__ __forceinline__ unsigned long long lowest(unsigned long long mask, uint32_t rank,
+                                                     uint32_t t) {
+  return mask & __ballot(rank < t);
+}
+
 // A table entry at a wave-uniform address by scalar loads of the members that
 // are used.  The pointer is opaque: the loads stay where they are asked for,
 // instead of the values being kept in scalar registers over the whole loop
@@ -582,7 +588,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
   // photons [0, n_end)
   uint32_t* wq = a.wave_queue + (size_t)(blockIdx.x * (kTransportThreads / 64) + wave) * kWaveWords;
   uint32_t n_wall = 0, n_ready = 0, n_gap = 0, n_back = 0, n_end = 0, idle = 0;
-  const uint32_t lane_cap = a.plan->lane_cap;
+  const uint32_t lane_cap = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.plan->lane_cap);
   const bool queued = a.queues != 0 && lane_cap == 64u;
   const uint32_t park = a.queues != 0 ? 0u : (uint32_t)a.park_lanes;
   const uint32_t serve_at = min((uint32_t)a.refill_lanes, lane_cap);
@@ -649,12 +655,12 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     const uint32_t t = min(count(want), n_ready);
     if (t == 0u) return;
     const uint32_t rank = rank_below(want);
-    const bool got = in(want) && rank < t;
+    const unsigned long long got = lowest(want, rank, t);
     __builtin_amdgcn_wave_barrier();
-    if (got) lds_get((uint32_t)kWallSlots - n_ready + rank);
+    if (in(got)) lds_get((uint32_t)kWallSlots - n_ready + rank);
     __builtin_amdgcn_wave_barrier();
     n_ready -= t;
-    step_m |= __ballot(got);
+    step_m |= got;
   };
 
   // How waiting photons are served, decided in each serve: 0 through the
@@ -666,7 +672,6 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
   bool last = false;  // no photon is left; the ended ones are still to be counted
   for (;;) {
     unsigned long long gap_m = 0;  // lanes whose photon's gap flight is next
-    PrptState st = prpt_initial();
     // ---- serve
     if (step_m == 0ull || (int)count(mode == 0 ? step_m : step_m | wall_m) <= busy_max) {
       while (n_end >= 64u || (last && n_end != 0u)) end_count();
@@ -677,10 +682,10 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
             const uint32_t k =
                 min(count(wall_m), (uint32_t)kWallSlots - n_wall - n_ready);
             const uint32_t rank = rank_below(wall_m);
-            const bool put = in(wall_m) && rank < k;
-            if (put) lds_put(n_wall + rank);
+            const unsigned long long put = lowest(wall_m, rank, k);
+            if (in(put)) lds_put(n_wall + rank);
             n_wall += k;
-            wall_m &= ~__ballot(put);
+            wall_m &= ~put;
             take_ready(~(step_m | wall_m));
           }
         }
@@ -690,12 +695,12 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
           __threadfence_block();  // the wave's queue stores are complete before its loads
           const uint32_t t = min(count(need), n_back);
           const uint32_t rank = rank_below(need);
-          const bool got = in(need) && rank < t;
-          if (got)
+          const unsigned long long got = lowest(need, rank, t);
+          if (in(got))
             q_get<MULTI, REC, kQBlock>(wq + q_base(kBackBase + n_back - 1u - rank), p, rng,
                                        lane_ev, gi, lane_k);
           n_back -= t;
-          step_m |= __ballot(got);
+          step_m |= got;
           need = use_m & ~(step_m | wall_m);
         }
         while (need != 0ull && !pool_done) {
@@ -749,30 +754,19 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         if (drain && queued && need != 0ull && (n_wall | n_gap) != 0u) {
           // the queues' last photons back into free lanes
           uint32_t t = min(count(need), n_wall);
-          uint32_t rank = rank_below(need);
-          bool got = in(need) && rank < t;
+          const uint32_t rank = rank_below(need);
+          const unsigned long long got = lowest(need, rank, t);
           __builtin_amdgcn_wave_barrier();
-          if (got) lds_get(n_wall - t + rank);
+          if (in(got)) lds_get(n_wall - t + rank);
           n_wall -= t;
-          wall_m |= __ballot(got);
-          need = ~(step_m | wall_m);
+          wall_m |= got;
+          need &= ~got;
           t = min(count(need), n_gap);
-          if (t != 0u) {
-            __threadfence_block();
-            rank = rank_below(need);
-            got = in(need) && rank < t;
-            if (got) {
-              const uint32_t* w = wq + q_base(kGapBase + n_gap - t + rank);
-              q_get<MULTI, REC, kQBlock>(w, p, rng, lane_ev, gi, lane_k);
-              q_get_state(w, st);
-            }
-            n_gap -= t;
-            gap_m = __ballot(got);
-          }
+          if (t != 0u) gap_m = lowest(need, rank_below(need), t);  // loaded in the gap section
         }
-        // nothing in a lane: the queues and the work queue are empty
         mode = drain ? 2 : queued ? 0 : 1;
         busy_max = drain && (n_wall | n_gap) == 0u ? -1 : (int)(lane_cap - serve_at);
+        // nothing in a lane: the queues and the work queue are empty
         last = (step_m | wall_m | gap_m) == 0ull;
         if (last) continue;
       }
@@ -815,6 +809,9 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
       break;
     }
     if (!wall && gap_m == 0ull) continue;
+    PrptState st = prpt_initial();
+    const unsigned long long fetch_m = gap_m;
+    gap_m = 0ull;
     if (wall) {
       if (!in_place) {
         // every lane without a waiting photon takes one; a photon that was
@@ -842,15 +839,24 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         wall_m = ~0ull;
       }
       int r = kPrAlive;
-      const bool mine = in(wall_m);
-      if (mine)
+      if (in(wall_m))
         with_geom([&](const GeomDev& g) { r = prpt_loop(rng, p, g, st, true, true); });
-      const unsigned long long e = __ballot(mine && r == kPrEnded);
-      const unsigned long long flight = __ballot(mine && r == kPrGap);
+      const unsigned long long e = __ballot(r == kPrEnded);
+      gap_m = __ballot(r == kPrGap);
       end_put(e);
-      step_m |= wall_m & ~(e | flight);
-      gap_m |= flight;
+      step_m |= wall_m & ~(e | gap_m);
       wall_m = 0ull;
+    }
+    if (fetch_m != 0ull) {
+      // a draining wave's free lanes take photons of the gap queue
+      n_gap -= count(fetch_m);
+      __threadfence_block();
+      if (in(fetch_m)) {
+        const uint32_t* w = wq + q_base(kGapBase + n_gap + rank_below(fetch_m));
+        q_get<MULTI, REC, kQBlock>(w, p, rng, lane_ev, gi, lane_k);
+        q_get_state(w, st);
+      }
+      gap_m |= fetch_m;
     }
     // ---- gap: one flight per photon and round (to the next column and its
     // Fresnel decision); a photon reflected off the outside of that column
@@ -889,11 +895,10 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         break;
       }
       int r = kPrAlive;
-      const bool mine = in(gap_m);
-      if (mine)
+      if (in(gap_m))
         with_geom([&](const GeomDev& g) { r = prpt_loop(rng, p, g, st, false, true); });
-      const unsigned long long e = __ballot(mine && r == kPrEnded);
-      const unsigned long long again = __ballot(mine && r == kPrGap);
+      const unsigned long long e = __ballot(r == kPrEnded);
+      const unsigned long long again = __ballot(r == kPrGap);
       end_put(e);
       step_m |= gap_m & ~(e | again);
       gap_m = again;
