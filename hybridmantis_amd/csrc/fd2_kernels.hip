@@ -569,13 +569,14 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
   // the wave's index in the block, uniform across the wave: the compiler
   // then keeps the wave's queue and LDS bases in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  // wave-uniform work pool: the launch's photons [pool_next, pool_end), the
-  // first of event pool_ev
-  uint64_t pool_next = 0, pool_end = 0;
-  uint32_t pool_ev = 0;
+  // wave-uniform work pool: pool_left of the launch's photons from
+  // pool_next on, the first of event pool_ev
+  uint64_t pool_next = 0;
+  uint32_t pool_left = 0, pool_ev = 0;
   bool pool_done = false;
 
   Photon p;
+  p.fate = kAlive;
   CounterRng rng;
   unsigned long long step_m = 0, wall_m = 0;
   uint32_t gi = 0;
@@ -705,7 +706,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         }
         while (need != 0ull && !pool_done) {
           const TransportArgs b = args();
-          if (pool_next >= pool_end) {
+          if (pool_left == 0u) {
             uint32_t c = 0;
             if (lane == 0) c = atomicAdd(&b.plan->cursor, 1u);
             c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
@@ -716,13 +717,13 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
               pool_done = true;
               break;
             }
-            pool_end = min(total, pool_next + (1ull << span_log2));
+            pool_left = (uint32_t)min(total - pool_next, (uint64_t)1 << span_log2);
             pool_ev = event_of(photon_off, b.n_events, pool_next, lane);
           }
           // Seeding a stream (Philox) and drawing the first direction are
           // long: every lane starts one of the next photons here, as many as
           // the LDS queue has room for.
-          const uint32_t n = (uint32_t)min((uint64_t)min((uint32_t)kLdsCap - n_wall, 64u), pool_end - pool_next);
+          const uint32_t n = min(min((uint32_t)kLdsCap - n_wall, 64u), pool_left);
           uint32_t e = pool_ev;
           if (photon_off[pool_ev + 1u] - pool_next < n)
             e = events_of(photon_off, b.n_events, pool_ev, pool_next, n, lane);
@@ -746,6 +747,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
           }
           n_ready = n;
           pool_next += n;
+          pool_left -= n;
           pool_ev = (uint32_t)__builtin_amdgcn_readlane((int)e, (int)(n - 1u));
           take_ready(need);
           need = use_m & ~(step_m | wall_m);
@@ -774,12 +776,10 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
     const bool stepped = step_m != 0ull;
     // ---- pass
     {
-      int r = kAlive;
       if (in(step_m)) {
         auto pass = [&](const ColumnGeom& g) {
           hot_step<CounterRng, false>(rng, p, g, &nosink);
-          r = p.fate;
-          if (__builtin_expect(r == kTrapped, 0)) {
+          if (__builtin_expect(p.fate == kTrapped, 0)) {
             atomicAdd(&s_cnt[gi * kCounters + FD2_C_REGEN], 1u);
             restart_trapped(rng, p, g, events[lane_ev]);
           }
@@ -789,7 +789,8 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         else
           pass(load_column(kernarg));
       }
-      const unsigned long long e = __ballot(ended(r)), w = __ballot(r == kWall);
+      const unsigned long long e = step_m & __ballot(ended(p.fate));
+      const unsigned long long w = step_m & __ballot(p.fate == kWall);
       end_put(e);
       wall_m |= w;
       step_m &= ~(e | w);
