@@ -103,27 +103,36 @@ __device__ __forceinline__ void write_offsets(const QueueArgs& q, int64_t base,
 // items than q.max_chunks sets error bit 4 and gets a total of 0, so the
 // transport takes nothing.
 //
-// A large launch uses all its workgroups and takes spans of half a wave's
-// share, at most the tuning's chunk.  A small one lasts as long as its longest
-// photon's chain of passes (up to some hundreds), and a pass takes the longer
-// the more waves share a SIMD (a wave alone waits for its own instructions;
-// six issue 3 times as many as fit meanwhile) and the more lanes take its rare
-// branches.  So the photons go to one wave per SIMD first, evenly, lane_cap
-// to a wave; then to more waves, 64 lanes at kLaneShare photons each.  On
-// MI355X, kernel time before (spans of 128 photons of one event, all waves)
-// and now: one event of 1,375 photons 0.89 -> 0.5 ms, 200 histories at 60 keV
-// (5.3e5 photons) 6.1 -> 3.3 ms; kLaneShare 1, 2, 4, 8, 16 on 500 histories at
-// 25 keV: 3.9, 3.8, 3.1, 3.7, 3.8 ms.
+// A large launch uses all its waves and takes spans of half a wave's share, at
+// most the tuning's chunk.  A small one ends with a long tail: it lasts as long
+// as its longest photon's chain of passes (some hundreds), and a pass takes the
+// longer the more waves share a SIMD (a wave alone waits for its own
+// instructions; six issue 3 times as many as fit meanwhile).  So photons go to
+// one wave per SIMD first, evenly, lane_cap to a wave, and the number of waves
+// per SIMD, k, grows with the square root of the photons: the tail grows with
+// k, the rest falls with the issue slots that k waves fill.  Every SIMD gets
+// the same number of waves, as the launch waits for the fullest one.  On MI355X
+// with k = 1 to 6, 25 keV in 150 um, kernel ms (chosen k marked):
+//   2.7e5 photons   2.49 2.35* 2.40  2.62  2.65  2.63
+//   6.5e5           3.70 3.07* 3.13  3.54  3.93  4.17
+//   1.6e6           6.82 4.81  4.40* 4.57  4.79  5.15
+//   5.5e6          18.83 11.2  9.28  8.74  8.73* 8.99
+//   1.1e7          36.44 20.6  16.5  14.9  14.3  14.2*
+// One wave more per 256 photons, as before: 2.42, 3.16, 5.13, 9.00, 14.2 ms.
+// A single event of 1,375 photons takes 0.46 ms with lane_cap 2 and 0.8 ms in
+// spans of 128 on all waves.
 __device__ __forceinline__ void plan_queue(const QueueArgs& q, unsigned long long photons,
                                            uint64_t chunks) {
   constexpr uint32_t kWaves = kTransportThreads / 64;
-  constexpr unsigned long long kLaneShare = 4;
   const bool over = chunks > q.max_chunks;
   if (over) atomicOr(q.error_flag, 4u);
   q.photon_off[q.n_events] = over ? 0ull : photons;
   const uint32_t alone = min(q.n_simds, q.n_waves);
-  unsigned long long waves = photons / (64u * kLaneShare);
-  if (waves < alone) waves = alone;
+  unsigned long long per_simd = photons < 128ull * alone ? 1u : 2u;
+  while (per_simd >= 2u && per_simd * alone < q.n_waves &&
+         photons >= (2u * per_simd + 1u) * (2u * per_simd + 1u) * 64ull * alone)
+    ++per_simd;
+  unsigned long long waves = per_simd * alone;
   if (waves > q.n_waves) waves = q.n_waves;
   uint32_t span_log2 = 0, lane_cap = 64;
   if (photons >= 64u * waves) {
