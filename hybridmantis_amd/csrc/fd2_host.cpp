@@ -5,6 +5,7 @@
 // errors come back as status codes instead of aborting.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -151,17 +152,6 @@ int grow(fd2_ctx* c, size_t n_events) {
   return FD2_OK;
 }
 
-int grow_stage(fd2_ctx* c, size_t n_events) {
-  if (n_events <= c->cap_stage) return FD2_OK;
-  if (c->h_stage) (void)hipHostFree(c->h_stage);
-  c->h_stage = nullptr;
-  c->cap_stage = 0;
-  const size_t cap = n_events + n_events / 4 + 1024;
-  FD2_HIP(hipHostMalloc(&c->h_stage, cap * sizeof(fd2_event), hipHostMallocDefault));
-  c->cap_stage = cap;
-  return FD2_OK;
-}
-
 int validate_host(const fd2_ctx* c, const fd2_event* ev, int64_t n) {
   for (int64_t i = 0; i < n; ++i) {
     if (ev[i].N > FD2_MAX_PHOTONS_PER_EVENT) return FD2_E_TOO_MANY;
@@ -169,6 +159,31 @@ int validate_host(const fd2_ctx* c, const fd2_event* ev, int64_t n) {
     if (ev[i].geom >= (uint32_t)c->n_geoms) return FD2_E_INVAL;
   }
   return FD2_OK;
+}
+
+// Checks `events`, copies them to c->d_events and counts their work items of
+// one chunk; the caller has waited for the stream.  The first invalid event
+// gives the status, and nothing is launched.
+int stage_events(fd2_ctx* c, const fd2_event* events, int64_t n, uint64_t* items) {
+  const int rc = grow(c, (size_t)n);
+  if (rc) return rc;
+  const uint64_t chunk = (uint64_t)c->tune.chunk;
+  std::atomic<uint64_t> total{0};
+  const int status = c->copy.upload(
+      c->stream, c->device, c->d_events, (size_t)n * sizeof(fd2_event), sizeof(fd2_event),
+      [&](char* dst, size_t off, size_t len) {
+        const fd2_event* ev = events + off / sizeof(fd2_event);
+        const int64_t m = (int64_t)(len / sizeof(fd2_event));
+        const int bad = validate_host(c, ev, m);
+        if (bad) return bad;
+        uint64_t sum = 0;
+        for (int64_t i = 0; i < m; ++i) sum += ((uint64_t)ev[i].N + chunk - 1) / chunk;
+        total.fetch_add(sum);
+        std::memcpy(dst, ev, len);
+        return (int)FD2_OK;
+      });
+  *items = total.load();
+  return status;
 }
 
 // LDS PRF tiles for a tuning value: -1 none, 0 the default side, else the
@@ -271,7 +286,7 @@ hipError_t issue(const Launch& L, hipStream_t s) {
 // queue build rejects a launch above the limit (error bit 4).
 int enqueue(fd2_ctx* c, const fd2_event* d_ev, int64_t n, bool record,
             fd2_photon* d_records, uint32_t* d_radial = nullptr,
-            const fd2_event* h_ev = nullptr) {
+            const fd2_event* h_ev = nullptr, uint64_t items_known = 0) {
   if (n <= 0) return FD2_OK;
   int rc = grow(c, (size_t)n);
   if (rc) return rc;
@@ -282,7 +297,7 @@ int enqueue(fd2_ctx* c, const fd2_event* d_ev, int64_t n, bool record,
   for (int64_t i0 = 0; i0 < n;) {
     int64_t i1 = n;
     uint64_t photons = 0;
-    if (h_ev) {
+    if (h_ev && items_known > limit) {
       uint64_t items = 0;
       for (i1 = i0; i1 < n; ++i1) {
         const uint64_t k = ((uint64_t)h_ev[i1].N + chunk - 1) / chunk;
@@ -369,20 +384,14 @@ namespace fd2 {
 int submit_radial_async(fd2_ctx* c, const fd2_event* events, int64_t n, uint32_t* d_radial) {
   if (!c || n < 0 || (n > 0 && (!events || !d_radial))) return FD2_E_INVAL;
   if (n == 0) return FD2_OK;
-  int rc = validate_host(c, events, n);
-  if (rc) return rc;
   FD2_HIP(hipSetDevice(c->device));
-  // the previous submit may still read the staging buffer
+  // the previous submit may still read the pinned ring
   FD2_HIP(hipStreamSynchronize(c->stream));
-  rc = grow_stage(c, (size_t)n);
+  uint64_t items = 0;
+  const int rc = stage_events(c, events, n, &items);
   if (rc) return rc;
-  rc = grow(c, (size_t)n);
-  if (rc) return rc;
-  std::memcpy(c->h_stage, events, (size_t)n * sizeof(fd2_event));
-  FD2_HIP(hipMemcpyAsync(c->d_events, c->h_stage, (size_t)n * sizeof(fd2_event),
-                         hipMemcpyHostToDevice, c->stream));
   FD2_HIP(launch_fill_u32(d_radial, (size_t)n * FD2_RADIAL_BINS, c->stream));
-  return enqueue(c, c->d_events, n, false, nullptr, d_radial, c->h_stage);
+  return enqueue(c, c->d_events, n, false, nullptr, d_radial, events, items);
 }
 
 }  // namespace fd2
@@ -498,7 +507,7 @@ void fd2_destroy(fd2_ctx* c) {
                   c->d_block_chunks, c->d_block_photons, c->d_plan, c->d_error};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
-  if (c->h_stage) (void)hipHostFree(c->h_stage);
+  c->copy.release();
   if (c->ev_start) (void)hipEventDestroy(c->ev_start);
   if (c->ev_stop) (void)hipEventDestroy(c->ev_stop);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -578,19 +587,13 @@ int fd2_set_next_event(fd2_ctx* c, int64_t first) {
 int fd2_submit(fd2_ctx* c, const fd2_event* events, int64_t n) {
   if (!c || n < 0 || (n > 0 && !events)) return FD2_E_INVAL;
   if (n == 0) return FD2_OK;
-  int rc = validate_host(c, events, n);
-  if (rc) return rc;
   FD2_HIP(hipSetDevice(c->device));
-  // the previous submit may still read the staging buffer
+  // the previous submit may still read the pinned ring
   FD2_HIP(hipStreamSynchronize(c->stream));
-  rc = grow_stage(c, (size_t)n);
+  uint64_t items = 0;
+  const int rc = stage_events(c, events, n, &items);
   if (rc) return rc;
-  rc = grow(c, (size_t)n);
-  if (rc) return rc;
-  std::memcpy(c->h_stage, events, (size_t)n * sizeof(fd2_event));
-  FD2_HIP(hipMemcpyAsync(c->d_events, c->h_stage, (size_t)n * sizeof(fd2_event),
-                         hipMemcpyHostToDevice, c->stream));
-  return enqueue(c, c->d_events, n, false, nullptr, nullptr, c->h_stage);
+  return enqueue(c, c->d_events, n, false, nullptr, nullptr, events, items);
 }
 
 int fd2_submit_device(fd2_ctx* c, const fd2_event* d_events, int64_t n) {
@@ -637,22 +640,19 @@ int fd2_submit_record(fd2_ctx* c, const fd2_event* events, int64_t n,
                       fd2_photon* records) {
   if (!c || n < 0 || (n > 0 && (!events || !records))) return FD2_E_INVAL;
   if (n == 0) return FD2_OK;
-  int rc = validate_host(c, events, n);
-  if (rc) return rc;
   FD2_HIP(hipSetDevice(c->device));
   FD2_HIP(hipStreamSynchronize(c->stream));
+  uint64_t items = 0;
+  int rc = stage_events(c, events, n, &items);
+  if (rc) return rc;
   int64_t total = 0;
   for (int64_t i = 0; i < n; ++i) total += events[i].N;
-  rc = grow(c, (size_t)n);
-  if (rc) return rc;
-  FD2_HIP(hipMemcpyAsync(c->d_events, events, (size_t)n * sizeof(fd2_event),
-                         hipMemcpyHostToDevice, c->stream));
   fd2_photon* d_rec = nullptr;
   if (total > 0) FD2_HIP(hipMalloc(&d_rec, (size_t)total * sizeof(fd2_photon)));
-  rc = enqueue(c, c->d_events, n, true, d_rec, nullptr, events);
+  rc = enqueue(c, c->d_events, n, true, d_rec, nullptr, events, items);
   if (rc == FD2_OK && total > 0)
-    rc = hipMemcpyAsync(records, d_rec, (size_t)total * sizeof(fd2_photon),
-                        hipMemcpyDeviceToHost, c->stream) == hipSuccess ? FD2_OK : FD2_E_DEVICE;
+    rc = c->copy.download(c->stream, c->device, records, d_rec,
+                          (size_t)total * sizeof(fd2_photon));
   if (hipStreamSynchronize(c->stream) != hipSuccess) rc = FD2_E_DEVICE;
   if (d_rec) (void)hipFree(d_rec);
   if (rc) return rc;
@@ -670,9 +670,7 @@ int fd2_submit_radial(fd2_ctx* c, const fd2_event* events, int64_t n,
   uint32_t* d_rad = nullptr;
   FD2_HIP(hipMalloc(&d_rad, nbins * sizeof(uint32_t)));
   rc = submit_radial_async(c, events, n, d_rad);
-  if (!rc && hipMemcpyAsync(radial, d_rad, nbins * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                            c->stream) != hipSuccess)
-    rc = FD2_E_DEVICE;
+  if (!rc) rc = c->copy.download(c->stream, c->device, radial, d_rad, nbins * sizeof(uint32_t));
   if (hipStreamSynchronize(c->stream) != hipSuccess) rc = FD2_E_DEVICE;
   (void)hipFree(d_rad);
   if (rc) return rc;

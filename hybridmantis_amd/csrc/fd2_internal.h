@@ -5,6 +5,7 @@
 
 #include "../../include/fd2.h"
 #include "fd2_device.h"
+#include "fd2_hostcopy.h"
 
 namespace fd2 {
 
@@ -146,8 +147,7 @@ struct fd2_ctx {
   unsigned long long* d_counters = nullptr;
 
   // staging and queue buffers, grown on demand
-  fd2_event* h_stage = nullptr;   // pinned
-  size_t cap_stage = 0;
+  fd2::HostCopy copy;             // to and from the caller's memory
   fd2_event* d_events = nullptr;
   size_t cap_events = 0;
   unsigned long long* d_photon_off = nullptr;

@@ -723,13 +723,15 @@ struct fd2_mlp {
   int64_t n_data = 0;
   int64_t step = 0;
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  // fd2_surrogate_submit's buffers, kept between calls and grown on demand
-  // (a call of the same size allocates nothing): device buffers by SurrBuf
-  // index, and the pinned copy of the audit predictions
-  void* sbuf[9] = {};
-  size_t sbuf_cap[9] = {};
+  // buffers kept between calls and grown on demand (a call of the same size
+  // allocates nothing): device buffers by SurrBuf index (fd2_surrogate_submit,
+  // and the inputs and outputs of a forward or of gradients), and the pinned
+  // copy of the audit predictions
+  void* sbuf[11] = {};
+  size_t sbuf_cap[11] = {};
   float* h_pred = nullptr;
   size_t h_pred_cap = 0;
+  fd2::HostCopy copy;  // results to the caller's memory
 };
 
 namespace {
@@ -749,7 +751,8 @@ bool grow(T** buf, size_t bytes) {
 
 // fd2_surrogate_submit's device buffers (fd2_mlp::sbuf)
 enum SurrBuf : int {
-  kBufAll, kBufEv, kBufIdx, kBufIds, kBufRad, kBufLogits, kBufSpread, kBufFeat, kBufPred, kBufCount
+  kBufAll, kBufEv, kBufIdx, kBufIds, kBufRad, kBufLogits, kBufSpread, kBufFeat, kBufPred, kBufIn,
+  kBufOut, kBufCount
 };
 static_assert(kBufCount == sizeof(fd2_mlp::sbuf) / sizeof(void*), "one slot per buffer");
 
@@ -943,6 +946,7 @@ void fd2_mlp_destroy(fd2_mlp* p) {
     if (b) (void)hipFree(b);
   for (void* b : p->sbuf)
     if (b) (void)hipFree(b);
+  p->copy.release();
   if (p->h_pred) (void)hipHostFree(p->h_pred);
   if (p->e0) (void)hipEventDestroy(p->e0);
   if (p->e1) (void)hipEventDestroy(p->e1);
@@ -982,11 +986,9 @@ int fd2_mlp_forward(fd2_mlp* p, const float* x, int64_t n, float* out) {
   float* dout = nullptr;
   int rc = ensure_batch(p, (int)chunk);
   if (rc) return rc;
-  MLP_HIP(hipMalloc(&dx, (size_t)chunk * kFeat * 4));
-  if (hipMalloc(&dout, (size_t)chunk * kTarget * 4) != hipSuccess) {
-    (void)hipFree(dx);
+  const size_t rows = (size_t)(n < chunk ? n : chunk);
+  if (!reserve(p, kBufIn, rows * kFeat * 4, &dx) || !reserve(p, kBufOut, rows * kTarget * 4, &dout))
     return FD2_E_NOMEM;
-  }
   for (int64_t s = 0; s < n && rc == FD2_OK; s += chunk) {
     const int b = (int)(n - s < chunk ? n - s : chunk);
     if (hipMemcpyAsync(dx, x + s * kFeat, (size_t)b * kFeat * 4, hipMemcpyHostToDevice,
@@ -1000,13 +1002,8 @@ int fd2_mlp_forward(fd2_mlp* p, const float* x, int64_t n, float* out) {
     if (rc) break;
     hipLaunchKernelGGL(k_head_probs, dim3((b * 64 + 255) / 256), dim3(256), 0, p->stream,
                        p->z[3], b, dout);
-    if (hipMemcpyAsync(out + s * kTarget, dout, (size_t)b * kTarget * 4,
-                       hipMemcpyDeviceToHost, p->stream) != hipSuccess ||
-        hipStreamSynchronize(p->stream) != hipSuccess)
-      rc = FD2_E_DEVICE;
+    rc = p->copy.download(p->stream, p->device, out + s * kTarget, dout, (size_t)b * kTarget * 4);
   }
-  (void)hipFree(dx);
-  (void)hipFree(dout);
   return rc;
 }
 
@@ -1068,7 +1065,7 @@ int fd2_mlp_gradients(fd2_mlp* p, const float* x, const float* y, int B, float* 
   // inputs, targets, gradients and loss in one buffer
   const size_t nx = (size_t)B * kFeat, ny = (size_t)B * kTarget;
   float* d = nullptr;
-  MLP_HIP(hipMalloc(&d, (nx + ny + kParams + 1) * 4));
+  if (!reserve(p, kBufIn, (nx + ny + kParams + 1) * 4, &d)) return FD2_E_NOMEM;
   float *dy = d + nx, *dg = dy + ny;
   int slices = 0;
   if (hipMemcpyAsync(d, x, nx * 4, hipMemcpyHostToDevice, p->stream) != hipSuccess ||
@@ -1085,7 +1082,6 @@ int fd2_mlp_gradients(fd2_mlp* p, const float* x, const float* y, int B, float* 
       rc = FD2_E_DEVICE;
   }
   if (hipStreamSynchronize(p->stream) != hipSuccess && !rc) rc = FD2_E_DEVICE;
-  (void)hipFree(d);
   return rc;
 }
 
