@@ -1079,12 +1079,14 @@ __device__ __forceinline__ bool ba_prpt(Rng& rng, Photon& p, const GeomDev& g) {
 // passes out of five) draws the same polar/azimuth pair as a sample's
 // perturbation and shares its code.
 //
-// The pass is bound by vector-ALU issue, and for the last photons of a launch
-// by its latency.  Selects instead of branches of one or two instructions,
-// the short root, reciprocal and quotient, and comparisons of squares instead
-// of roots took the kernel on mono25x50 (100,000 histories at 25 keV, 1.1e8
-// photons) from 972 to 810 vector instructions per photon and from 132 to
-// 118 ms, and a lone event of 1,375 photons from 1.84 to 1.48 ms.
+// The pass is bound by instruction issue, and for the last photons of a launch
+// by its latency.  Selects instead of branches of one or two instructions, the
+// short root, reciprocal and quotient, comparisons of squares instead of roots,
+// one draw for the three decisions, and one outcome code (the fate) instead of
+// flags.  On mono25x50 (100,000 histories at 25 keV, 1.1e8 photons) the first
+// three took the kernel from 972 to 810 vector instructions per photon and from
+// 132 to 118 ms, and the last two, with the column's constants in the kernel's
+// arguments, from 108.1 to 105.5 ms.
 template <class Rng, bool TRACE, class M = MathDevice>
 __device__ __forceinline__ void hot_step(Rng& rng, Photon& p, const ColumnGeom& g,
                                          StepSink* sink) {

@@ -229,8 +229,8 @@ __device__ __forceinline__ void counter_initial_dir(CounterRng& rng, Photon& p,
 
 // Register budget of the transport kernel: 6 waves per SIMD (80 VGPRs, 7
 // values of rare paths in scratch; without a limit the wall branch takes 92).
-// mono25x50 on MI355X at 20 and 24 waves per CU: 117.4 ms with 5 waves per
-// SIMD, 112.1 ms with 6; the LDS (26.5 KB per workgroup) holds no more.
+// mono25x50 on MI355X at 20 and 24 waves per CU: 94.5 ms with 5 waves per
+// SIMD, 89.9 ms with 6; the LDS (26.5 KB per workgroup) holds no more.
 // FD2_WAVES_PER_EU=0 lets the compiler choose.
 #ifndef FD2_WAVES_PER_EU
 #define FD2_WAVES_PER_EU 6
@@ -499,14 +499,15 @@ __device__ __forceinline__ uint32_t events_of(const unsigned long long* __restri
 }
 
 // Persistent transport.  A wave keeps the state of its lanes in wave-uniform
-// masks: step_m (a photon that takes in-column passes), wall_m (a photon that
-// waits for the wall's Fresnel branch), end_m (a photon that has ended and is
-// not tallied yet); the other lanes are free.  Its loop:
+// masks: step_m (a photon that takes in-column passes) and wall_m (a photon
+// that waits for the wall's Fresnel branch); the other lanes are free.  Its
+// loop:
 //
-//   serve   once refill_lanes lanes do not step: tally the ended photons, put
-//           the waiting ones into the wave's LDS queue and fill the free lanes
-//           (LDS queue, HBM backlog, then new photons of the work queue,
-//           which all lanes start together into the LDS queue)
+//   serve   once refill_lanes lanes do not step: count 64 ended photons if as
+//           many wait, put the photons waiting for the wall into the wave's LDS
+//           queue and fill the free lanes (LDS queue, HBM backlog, then new
+//           photons of the work queue, which all lanes start together into the
+//           LDS queue)
 //   pass    one in-column pass of the stepping lanes
 //   wall    once 64 photons wait (in lanes and in the LDS queue): the branch
 //           runs with all 64 lanes, up to a refraction out of the column;
@@ -526,10 +527,17 @@ __device__ __forceinline__ uint32_t events_of(const unsigned long long* __restri
 // refill.
 //
 // Draining (no span, ready photon or backlog left), and throughout when
-// there are no queues (wave_queue null) or a launch has less than 64 photons
-// per wave, waiting photons stay in their lanes: the branch and the flights
+// the queues are not used (tuning) or a launch has less than 64 photons per
+// wave, waiting photons stay in their lanes: the branch and the flights
 // run where they are, with the other lanes masked off, once at least as many
 // wait as step (without queues: park_lanes).
+//
+// The loop's scalar work counts as much as its vector work: six waves share a
+// SIMD's issue slots.  So only a serve decides the mode and when the next serve
+// is due, a round without a phase does nothing else, and a lane mask is made
+// before the branch that uses it (made inside, it becomes a lane flag and a
+// mask again).  mono25x50 on MI355X: 103.7 -> 89.7 ms, 793 -> 719 vector and 365
+// -> 299 scalar instructions per photon, most of it spilled scalar registers.
 //
 // Every photon keeps its own state and random stream, so the results are the
 // same in either mode and in any order.
@@ -617,7 +625,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
   };
   // Ended photons wait in HBM until 64 of them are counted at once: about one
   // lane of a wave ends in two passes, and its tallies are as long as a third
-  // of a pass.
+  // of a pass (mono25x50: 104.5 ms counted in each serve, 103.7 here).
   auto end_put = [&](unsigned long long m) {
     if (m == 0ull) return;
     if (in(m)) {
