@@ -209,11 +209,16 @@ __device__ __forceinline__ void tally_add(T* p, T v) {
 enum Fate : int {
   kNone = 0, kDetect = 1, kDetectOut = 2, kAbsTop = 3, kAbsBulk = 4,
   kLost = 5, kOutOfCol = 6, kTheta1 = 7,
-  // what follows an in-column pass of a photon that has not ended: the next
-  // pass, a restart, the wall's Fresnel branch, a sample of a direction
-  kAlive = 16, kTrapped, kWall, kSample, kSampleTop
+  // what follows an in-column pass of a photon that has not ended: the wall's
+  // Fresnel branch, a restart, the next pass, a sample of a direction.  A hit
+  // of the pass's draw changes kHit of the code: detected or reflected by the
+  // sensor, absorbed or sampled at the top, wall or crosstalk.
+  kHit = 32,
+  kWall = 16, kTrapped = 17, kAlive = kDetectOut ^ kHit, kSampleTop = kAbsTop ^ kHit,
+  kSample = kWall ^ kHit
 };
-__device__ __forceinline__ bool ended(int fate) { return fate < kAlive; }
+static_assert(kAlive < kSampleTop && kSampleTop < kSample, "samples are the highest codes");
+__device__ __forceinline__ bool ended(int fate) { return fate < kWall; }
 static_assert(kDetectOut - 1 == FD2_C_DETECT && kAbsTop - 1 == FD2_C_ABS_TOP &&
               kAbsBulk - 1 == FD2_C_ABS_BULK && kLost - 1 == FD2_C_LOST &&
               kOutOfCol - 1 == FD2_C_OUTOFCOL && kTheta1 - 1 == FD2_C_THETA1,
@@ -1109,14 +1114,13 @@ __device__ __forceinline__ void hot_step(Rng& rng, Photon& p, const ColumnGeom& 
     if (!gone) {
       int fate = kTrapped;
       if (!flat) {
-        const float cct = crosstalk<M>(p.pz, g);
+        float cct = crosstalk<M>(p.pz, g);
+        asm volatile("" : "+v"(cct));  // not in a branch of its own
         const float limit = sensor ? g.sensor_refl : top ? g.top_absfrac : cct;
-        const bool drawn = sensor | !top | (g.top_absfrac > 0.0f);
-        bool hit = false;
-        if (drawn) hit = rng.u() < limit;
-        fate = sensor ? (hit ? kAlive : kDetectOut)
-                      : top ? (hit ? kAbsTop : kSampleTop) : (hit ? kSample : kWall);
-        if (sensor & hit) {
+        int flip = 0;
+        if (sensor | !top | (g.top_absfrac > 0.0f)) flip = rng.u() < limit ? (int)kHit : 0;
+        fate = (sensor ? (int)kDetectOut : top ? (int)kSampleTop : (int)kWall) ^ flip;
+        if (sensor & (flip != 0)) {
           // the reference follows the reflection with another in-column step
           // inside the same pass; here that step is the start of the next
           // pass, so its code exists once
@@ -1130,7 +1134,7 @@ __device__ __forceinline__ void hot_step(Rng& rng, Photon& p, const ColumnGeom& 
       p.fate = fate;
     }
   }
-  if (p.fate >= kSample) {
+  if (__builtin_expect(p.fate >= kSampleTop, 1)) {
     const bool top = p.fate == kSampleTop;
     float qx, qy, w, nx, ny, nz = 0.0f;
     const float mx = -p.ux, my = -p.uy, mz = -p.uz;
