@@ -552,22 +552,24 @@ __global__ void __launch_bounds__(64 * kTrainWaves) k_train_rows(TrainRows a) {
 // gradients and the loss from the rows' sums: partial results of gridDim.y
 // slices of the batch, added in order by k_adam or k_sum_grads (a fixed order:
 // the same step twice gives the same bits).
-// Workgroups [0, kWeightTiles): a 64 x 64 tile of one layer, the slice's row
-// groups (two per 32-k MFMA step) shared by the 4 waves and added in LDS; the
-// others: 64 columns of the sums each.
+// Workgroups [0, kWeightTiles): a 64 x 64 tile of one layer, a 32 x 32 quarter
+// to a wave, the slice's rows (`per` groups of 16) in order through one chain of
+// 16-k MFMA steps; the others: 64 columns of the sums each.  Sixteen slices of
+// whole chains give a partial sum the rounding of the layer-by-layer product
+// over the same rows, and 16 steps hide their loads (four waves sharing a tile's
+// rows read 2.5 times less from L2 and took 10.2 us at batch 4096).
 constexpr int kWeightTiles = 4 + 16 + 16 + 8;
 constexpr int kSumBlocks = (kSums + 63) / 64;
 constexpr size_t kPartial = kParams + 16;  // the loss at kParams
 
 __global__ void __launch_bounds__(256) k_weight_grads(const uint2* __restrict__ frags,
                                                       const float* __restrict__ sums, int groups,
-                                                      float* __restrict__ part) {
-  __shared__ float4_ s_acc[4][16][64];
+                                                      int per, float* __restrict__ part) {
+  __shared__ float s_sum[256];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, lr = lane & 15, lq = lane >> 4;
   const int slices = gridDim.y, slice = blockIdx.y;
   float* const out = part + (size_t)slice * kPartial;
   if ((int)blockIdx.x >= kWeightTiles) {
-    float* s_sum = reinterpret_cast<float*>(s_acc);
     const int c = ((int)blockIdx.x - kWeightTiles) * 64 + lane;
     float v = 0.0f;
     if (c < kSums)
@@ -590,64 +592,46 @@ __global__ void __launch_bounds__(256) k_weight_grads(const uint2* __restrict__ 
   const int mv = l == 0 ? 2 : 4;                       // valid blocks
   const int nv = l == 3 ? (nt == 0 ? 4 : 1) : 4;
   const int N = l == 3 ? kOutPad : kHidden;
-  const uint2* fa = frags + (size_t)(kInBlock[l] + 4 * mt) * 64 + lane;
-  const uint2* fb = frags + (size_t)(kGradBlock[l] + 4 * nt) * 64 + lane;
-  float4_ acc[4][4];
+  const int wm = 2 * (wv >> 1), wn = 2 * (wv & 1);
+  if (wm >= mv || wn >= nv) return;
+  const bool two = wn + 1 < nv;
+  const uint2* fa = frags + (size_t)(kInBlock[l] + 4 * mt + wm) * 64 + lane;
+  const uint2* fb = frags + (size_t)(kGradBlock[l] + 4 * nt + wn) * 64 + lane;
+  float4_ acc[2][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = float4_{0.f, 0.f, 0.f, 0.f};
-  const int pairs = (groups + 1) >> 1;
-  const uint2 none = make_uint2(0u, 0u);
-  for (int p = slice * 4 + wv; p < pairs; p += 4 * slices) {
-    const size_t g0 = (size_t)(2 * p) * kRowBlocks * 64, g1 = g0 + (size_t)kRowBlocks * 64;
-    const bool two = 2 * p + 1 < groups;
-    uint2 va[4][2], vb[4][2];
+    for (int j = 0; j < 2; ++j) acc[i][j] = float4_{0.f, 0.f, 0.f, 0.f};
+  const int end = min(groups, (slice + 1) * per);
+#pragma unroll 8
+  for (int g = slice * per; g < end; ++g) {
+    const size_t at = (size_t)g * kRowBlocks * 64;
+    const uint2 va[2] = {fa[at], fa[at + 64]};
+    const uint2 vb[2] = {fb[at], two ? fb[at + 64] : make_uint2(0u, 0u)};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      va[i][0] = i < mv ? fa[g0 + i * 64] : none;
-      va[i][1] = i < mv && two ? fa[g1 + i * 64] : none;
-      vb[i][0] = i < nv ? fb[g0 + i * 64] : none;
-      vb[i][1] = i < nv && two ? fb[g1 + i * 64] : none;
-    }
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i < mv) {
-        const bf16x8_ x = __builtin_bit_cast(
-            bf16x8_, make_uint4(va[i][0].x, va[i][0].y, va[i][1].x, va[i][1].y));
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              x,
-              __builtin_bit_cast(bf16x8_,
-                                 make_uint4(vb[j][0].x, vb[j][0].y, vb[j][1].x, vb[j][1].y)),
-              acc[i][j], 0, 0, 0);
-      }
+      for (int j = 0; j < 2; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4_, va[i]),
+                                                              __builtin_bit_cast(short4_, vb[j]),
+                                                              acc[i][j], 0, 0, 0);
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) s_acc[wv][i * 4 + j][lane] = acc[i][j];
-  __syncthreads();
-  if (wv < mv) {  // wave w adds and writes the tile's row blocks w
+    for (int j = 0; j < 2; ++j) {
+      if (j == 1 && !two) break;
+      const int row = (4 * mt + wm + i) * 16 + 4 * lq, col = (4 * nt + wn + j) * 16 + lr;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (j >= nv) break;
-      const int k = wv * 4 + j;
-      const float4_ v =
-          (s_acc[0][k][lane] + s_acc[1][k][lane]) + (s_acc[2][k][lane] + s_acc[3][k][lane]);
-      const int row = (4 * mt + wv) * 16 + 4 * lq, col = (4 * nt + j) * 16 + lr;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) out[kWOff[l] + (size_t)(row + r) * N + col] = v[r];
+      for (int r = 0; r < 4; ++r) out[kWOff[l] + (size_t)(row + r) * N + col] = acc[i][j][r];
     }
-  }
 }
 
-// gradient of parameter i: its slices' partial sums in order
+// gradient of parameter i: its slices' partial sums, rounded once
 __device__ __forceinline__ float sum_slices(const float* __restrict__ part, int slices, size_t i) {
-  float g = 0.0f;
-  for (int s = 0; s < slices; ++s) g += part[(size_t)s * kPartial + i];
-  return g;
+  double g = 0.0;
+  for (int s = 0; s < slices; ++s) g += (double)part[(size_t)s * kPartial + i];
+  return (float)g;
 }
 
 // parameters without a gradient: the output padding's biases
@@ -795,13 +779,11 @@ int ensure_layers(fd2_mlp* p, int B) {
   return FD2_OK;
 }
 
-// and for a training step.  The weight gradients' slices (kMaxSlices at most)
-// give every wave of k_weight_grads about 4 pairs of row groups.
+// and for a training step.  The weight gradients' slices (kMaxSlices at most):
+// one below 1,024 rows, else 16 of whole row groups.
 constexpr int kMaxSlices = 16;
-int train_slices(int B) {
-  const int s = B / 16 / 32;
-  return s < 1 ? 1 : s > kMaxSlices ? kMaxSlices : s;
-}
+int slice_groups(int B) { return B >= 1024 ? (B / 16 + kMaxSlices - 1) / kMaxSlices : B / 16; }
+int train_slices(int B) { return (B / 16 + slice_groups(B) - 1) / slice_groups(B); }
 int ensure_train(fd2_mlp* p, int B) {
   if (!p->part && hipMalloc(&p->part, kMaxSlices * kPartial * 4) != hipSuccess)
     return FD2_E_DEVICE;
@@ -867,7 +849,7 @@ int batch_gradients(fd2_mlp* p, const float* xs, const float* ys, const uint32_t
   const int groups = B / 16, slices = train_slices(B);
   hipLaunchKernelGGL(k_train_rows, dim3(groups), dim3(64 * kTrainWaves), 0, p->stream, a);
   hipLaunchKernelGGL(k_weight_grads, dim3(kWeightTiles + kSumBlocks, slices), dim3(256), 0,
-                     p->stream, p->frags, p->sums, groups, p->part);
+                     p->stream, p->frags, p->sums, groups, slice_groups(B), p->part);
   MLP_HIP(hipGetLastError());
   return slices;
 }
