@@ -630,6 +630,7 @@ __global__ void __launch_bounds__(256) k_weight_grads(const uint2* __restrict__ 
 // gradient of parameter i: its slices' partial sums, rounded once
 __device__ __forceinline__ float sum_slices(const float* __restrict__ part, int slices, size_t i) {
   double g = 0.0;
+#pragma unroll 8
   for (int s = 0; s < slices; ++s) g += (double)part[(size_t)s * kPartial + i];
   return (float)g;
 }
