@@ -71,8 +71,8 @@ struct ColumnGeom {
   float top20;           // lower edge of the band of certain crosstalk, H/2 - 0.2 H
   float den_up, inv_up;  // crosstalk slopes' divisors 2*top20 and -H, and their
   float den_dn, inv_dn;  // correctly rounded reciprocals
-  float wall_max;        // dist_to_surface's short form holds up to this wall distance:
-                         // 2^40, or NaN (never) unless R and H/2 are in [2^-8, 2^20]
+  float dist_max;        // dist_to_surface's short form holds up to this distance:
+                         // 2^27, or NaN (never) unless R and H/2 are in [2^-8, 2^20]
 };
 static_assert(sizeof(ColumnGeom) == 64, "one 16-dword scalar load");
 
@@ -469,10 +469,14 @@ struct StepSink {
 //
 // MathDevice: straight-line code for directions and distances of ordinary
 // size, with the correctly rounded root, reciprocal and quotient of
-// fd2_math.h; a lane outside its limits (in about one step of 2^30) takes the
+// fd2_math.h; a lane outside its limits (in about one step of 2^20) takes the
 // IEEE operations in a branch that a wave nearly always skips.  Inside the
 // limits both roots are ordered, so the wall distance is the first, and the
-// direction is not along the axis.  The radii are compared by their squares:
+// direction is not along the axis.  The limit on the plane's distance is one on
+// the quotient itself: a photon far outside the layer (its distance to the plane
+// then overflows or is infinite) would get NaN from the short form.  A numerator
+// other than 0 is at least 2^-33 (H/2 >= 2^-8), so a quotient up to 2^27 also
+// means |uz| >= 2^-60, the short quotient's own limit.  The radii are compared by their squares:
 // rn > r_nudge is s > nudge_sq for the rounded root rn of s, and a candidate's
 // root can only exceed the current one when its square does.
 template <bool TRACE, class M = MathDevice>
@@ -496,7 +500,7 @@ __device__ __forceinline__ float dist_to_surface(Photon& p, const ColumnGeom& g,
     dpl = fd2_div(zpl - p.pz, p.uz);
     plane = !(dpl >= dcyl);
     // dcyl is NaN for a negative, zero or infinite discriminant
-    general = !((qa >= 0x1p-32f) & (dcyl <= g.wall_max) & (fabsf(p.uz) >= 0x1p-60f));
+    general = !((qa >= 0x1p-32f) & (dcyl <= g.dist_max) & (fabsf(dpl) <= g.dist_max));
   }
   if (M::kFaithful || __builtin_expect(general, 0)) {
     float r1, r2;

@@ -94,7 +94,7 @@ void derive(const fd2_params& p, GeomDev& g) {
   g.inv_dn = 1.0f / g.den_dn;
   const bool ordinary =
       g.R >= 0x1p-8f && g.R <= 0x1p20f && g.half_h >= 0x1p-8f && g.half_h <= 0x1p20f;
-  g.wall_max = ordinary ? 0x1p40f : NAN;
+  g.dist_max = ordinary ? 0x1p27f : NAN;
   // out-of-column radius: the largest float whose rounded root is at most the
   // float threshold of R - 1e-5 (none when that is negative)
   const float r_nudge = float_le((double)g.R - 1e-5);
