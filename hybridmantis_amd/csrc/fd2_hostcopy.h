@@ -69,9 +69,11 @@ class HostCopy {
         return FD2_E_DEVICE;
       return FD2_OK;
     }
+    // the stream may still read the ring (an upload of the same call), which
+    // reserve may give back
+    if (hipStreamSynchronize(stream) != hipSuccess) return FD2_E_DEVICE;
     const int rc = reserve(bytes);
     if (rc) return rc;
-    if (hipStreamSynchronize(stream) != hipSuccess) return FD2_E_DEVICE;
     char* out = static_cast<char*>(dst);
     auto empty = [&](Worker& w, int slot) {
       if (!w.used[slot]) return (int)FD2_OK;
