@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -31,7 +32,8 @@ class HostCopy {
       if (e) (void)hipEventDestroy(e);
       e = nullptr;
     }
-    if (ring_) (void)hipHostFree(ring_);
+    if (ring_ && pinned_) (void)hipHostFree(ring_);
+    if (ring_ && !pinned_) std::free(ring_);
     ring_ = nullptr;
     cap_ = 0;
   }
@@ -129,13 +131,20 @@ class HostCopy {
     return ring_ + (size_t)(w.base + slot) * (cap_ / (kWorkers * kSlots));
   }
 
-  // a ring for copies of `bytes`: 64 KB for small ones, else 4 to 16 MB
+  // a ring for copies of `bytes`: 64 KB for small ones, else 4 to 16 MB; of
+  // ordinary memory if no more can be pinned (the runtime then stages its copies).
+  // Freeing that waits for no copy: whoever gets here has waited for the stream.
   int reserve(size_t bytes) {
     const size_t need = bytes <= kSmall ? kSmall : kWorkers * kSlots * slice_of(bytes);
     if (cap_ >= need) return FD2_OK;
     release();
     void* p = nullptr;
-    if (hipHostMalloc(&p, need, hipHostMallocDefault) != hipSuccess) return FD2_E_NOMEM;
+    pinned_ = hipHostMalloc(&p, need, hipHostMallocDefault) == hipSuccess;
+    if (!pinned_) {
+      (void)hipGetLastError();  // answered here
+      p = std::malloc(need);
+      if (!p) return FD2_E_NOMEM;
+    }
     ring_ = static_cast<char*>(p);
     if (need > kSmall)
       for (hipEvent_t& e : ready_)
@@ -199,6 +208,7 @@ class HostCopy {
   }
 
   char* ring_ = nullptr;
+  bool pinned_ = false;
   size_t cap_ = 0;
   hipEvent_t ready_[kWorkers * kSlots] = {};
 };

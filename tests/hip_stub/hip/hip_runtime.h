@@ -28,6 +28,7 @@ struct Op {  // a copy, or the mark of an event
 inline std::mutex mu;
 inline std::deque<Op> queue;  // one stream
 inline int faults = 0, ring_frees = 0;
+inline bool no_pinned = false;  // hipHostMalloc fails
 inline const char* ring = nullptr;
 inline size_t ring_bytes = 0;
 inline void step() {
@@ -45,7 +46,9 @@ typedef int hipStream_t;
 typedef hipstub::Event* hipEvent_t;
 
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (hipstub::no_pinned) return hipErrorUnknown;
   *p = malloc(n);
   hipstub::ring = static_cast<char*>(*p);
   hipstub::ring_bytes = n;

@@ -1,7 +1,8 @@
-// host_copies UP DOWN: one upload of UP bytes and, without a wait between them,
+// host_copies UP DOWN [nopin]: one upload of UP bytes and, without a wait between them,
 // one download of DOWN bytes through the same HostCopy (a submit whose results
 // are read in the same call).  Ends with 0 if both arrived whole and no memory or
-// event was given back while the stream still needed it.
+// event was given back while the stream still needed it.  nopin: there is no
+// pinned memory.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -9,7 +10,8 @@
 #include "../../hybridmantis_amd/csrc/fd2_hostcopy.h"
 
 int main(int argc, char** argv) {
-  if (argc != 3) return 2;
+  if (argc != 3 && argc != 4) return 2;
+  hipstub::no_pinned = argc == 4;
   const size_t up = strtoull(argv[1], nullptr, 10), down = strtoull(argv[2], nullptr, 10);
   std::vector<char> from(up), dev(up), results(down), to(down);
   for (size_t i = 0; i < up; ++i) from[i] = (char)(i * 31 + i / 251);

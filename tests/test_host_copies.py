@@ -28,3 +28,11 @@ def test_download_after_upload(host_copies, up, down):
     r = subprocess.run([host_copies, str(up), str(down)], capture_output=True, text=True,
                        timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("up,down", [(32, 16), (32, MB), (200 * KB, 20 * MB), (40 * MB + 7, 2 * MB)])
+def test_without_pinned_memory(host_copies, up, down):
+    """The same answers, through ordinary memory."""
+    r = subprocess.run([host_copies, str(up), str(down), "nopin"], capture_output=True, text=True,
+                       timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
