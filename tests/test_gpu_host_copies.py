@@ -99,3 +99,13 @@ def test_forward_of_one_call_and_of_many(fd2lib):
     parts = [net.forward(x[a:b]) for a, b in
              ((0, 1), (1, 4033), (4033, 8066), (8066, 20000), (20000, 70001))]
     assert np.array_equal(whole, np.concatenate(parts))
+
+
+def test_radial_histograms_of_one_call_and_of_two(fd2lib):
+    """256 bytes an event: more than the events' own ring holds, on a new context."""
+    ev = events(9001, 1)
+    with fd2lib.Transport(params()) as tr:
+        whole = fd2lib.submit_radial(tr, ev)
+    with fd2lib.Transport(params()) as tr:
+        parts = [fd2lib.submit_radial(tr, ev[a:b]) for a, b in ((0, 3000), (3000, 6001), (6001, 9001))]
+    assert whole.sum() > 0 and np.array_equal(whole, np.concatenate(parts))
