@@ -191,6 +191,14 @@ __device__ __forceinline__ void ranecu_init(RanecuRng& g, int batch,
 
 // ----------------------------------------------------------- tallies
 
+// Orders a wave's LDS accesses of before with those of after, where one lane
+// reads what another wrote: a wave's LDS operations complete in order, so this
+// is only the statement of it to the compiler (no instruction).
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Tally atomics (PRF, history counts, radial bins) through
 // global (address space 1) pointers.  The tally pointers are read from the
 // geometry table, so the compiler cannot tell their address space and would

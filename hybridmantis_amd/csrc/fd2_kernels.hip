@@ -666,17 +666,15 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
   auto lds_get = [&](uint32_t slot) {
     q_get<MULTI, REC, kWallSlots>(lq + slot, p, rng, lane_ev, gi, lane_k);
   };
-  // fills up to n_ready of the lanes in `want` from the ready photons; the
-  // barrier keeps the compiler from moving LDS accesses across (a wave's
-  // complete in order)
+  // fills up to n_ready of the lanes in `want` from the ready photons
   auto take_ready = [&](unsigned long long want) {
     const uint32_t t = min(count(want), n_ready);
     if (t == 0u) return;
     const uint32_t rank = rank_below(want);
     const unsigned long long got = lowest(want, rank, t);
-    __builtin_amdgcn_wave_barrier();
+    lds_order();
     if (in(got)) lds_get((uint32_t)kWallSlots - n_ready + rank);
-    __builtin_amdgcn_wave_barrier();
+    lds_order();
     n_ready -= t;
     step_m |= got;
   };
@@ -775,7 +773,7 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
           uint32_t t = min(count(need), n_wall);
           const uint32_t rank = rank_below(need);
           const unsigned long long got = lowest(need, rank, t);
-          __builtin_amdgcn_wave_barrier();
+          lds_order();
           if (in(got)) lds_get(n_wall - t + rank);
           n_wall -= t;
           wall_m |= got;
@@ -839,10 +837,10 @@ k_transport(TransportArgs a, const GeomDev* __restrict__ geoms_in,
         Photon q;
         CounterRng r;
         uint32_t ev = 0, g2 = 0, k2 = 0;
-        __builtin_amdgcn_wave_barrier();
+        lds_order();
         if (in(need)) {
           q_get<MULTI, REC, kWallSlots>(lq + n_wall - t + rank, q, r, ev, g2, k2);
-          __builtin_amdgcn_wave_barrier();
+          lds_order();
           if (in(step_m))
             lds_put((uint32_t)kWallSlots - n_ready - n_step + rank_below(step_m));
           p = q;

@@ -1307,9 +1307,7 @@ k_surr_sample(SampleArgs a, const fd2_event* __restrict__ events,
       }
       s_guide[w][lane] = gk;
     }
-    // the wave's LDS writes complete in order before its reads below; the
-    // barrier keeps the compiler from moving the reads above them
-    __builtin_amdgcn_wave_barrier();
+    fd2::lds_order();
     const float pdet = 1.0f / (1.0f + expf(-z[0]));
     fd2::CounterRng rng;
     rng.seed(a.seed ^ 0x53555252u, ids[e], (uint32_t)lane);
