@@ -51,8 +51,8 @@ constexpr int kTileDefault = 0;  // no tile: the LDS holds the wall queues
 constexpr int kTileBudget = 64 * 64;   // u32 entries per block (16 KiB)
 // per-wave photon queues of the persistent kernel: photons waiting for the
 // wall branch (at most 63) and photons ready to step in LDS, together at most
-// kLdsCap (so that new photons always start at least 33 at a time), and 8
-// slots to write before reading; the gap queue and the backlog in HBM (slots
+// kLdsCap (so that new photons start at least 33 at a time, the last of a span
+// excepted), and 8 slots to write before reading; the gap queue and the backlog in HBM (slots
 // in that order).  At most 64 + kLdsCap + kGapCap photons are in flight per
 // wave.
 constexpr int kLdsCap = 96;
@@ -71,9 +71,9 @@ constexpr int kWaveWords = kQWords * kQSlots + 5 * kEndCap;
 static_assert(kQSlots % kQBlock == 0 && kGapBase % kQBlock == 0 && kBackBase % kQBlock == 0,
               "queue regions are whole blocks");
 constexpr uint32_t kMaxIdlePasses = 256;  // passes without a step or a wall branch
-// largest LDS tile side: 49 KiB of tile, plus the kernel's static LDS (about
-// 16 KiB with the several-geometry table); fd2_set_tuning checks the sum
-// against the device's LDS per workgroup (160 KiB on gfx950)
+// largest LDS tile side: 49 KiB of tile, plus the kernel's static LDS (26 to 29
+// KiB, transport_lds_bytes) and the table of several geometries; fd2_set_tuning checks
+// the sum against the device's LDS per workgroup (160 KiB on gfx950)
 constexpr int kTileMax = 112;
 
 struct QueueArgs {
@@ -96,6 +96,19 @@ constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanThreads * kScanItems;
 constexpr int kTransportThreads = 256;
+
+// static LDS of the transport: the waves' photon queues, the lanes' history runs
+// and the counters; per CU it leaves room for 6 workgroups (one geometry) and 5
+// (a short table of several, or records)
+constexpr size_t transport_lds_bytes(bool multi, bool record) {
+  return sizeof(uint32_t) * ((size_t)(kTransportThreads / 64) * (14 + multi + record) * kWallSlots +
+                             2 * kTransportThreads + FD2_MAX_GEOMS * kCounters);
+}
+constexpr size_t kLdsPerCu = 160 * 1024;
+static_assert(transport_lds_bytes(false, false) == 26496 && 6 * transport_lds_bytes(false, false) <= kLdsPerCu);
+static_assert(transport_lds_bytes(true, false) == 28160 && transport_lds_bytes(true, true) == 29824 &&
+              5 * (transport_lds_bytes(true, true) + 16 * sizeof(GeomDev)) <= kLdsPerCu);
+static_assert(sizeof(GeomDev) == 168);
 
 // dynamic LDS of the transport: the geometry table (several geometries) and
 // `tile_words` words of PRF tiles

@@ -108,11 +108,15 @@ __device__ __forceinline__ void write_offsets(const QueueArgs& q, int64_t base,
 // as its longest photon's chain of passes (some hundreds), and a pass takes the
 // longer the more waves share a SIMD (a wave alone waits for its own
 // instructions; six issue 3 times as many as fit meanwhile).  So photons go to
-// one wave per SIMD first, evenly, lane_cap to a wave, and the number of waves
-// per SIMD, k, grows with the square root of the photons: the tail grows with
+// one wave per SIMD first, lane_cap to a wave, and the number of waves per SIMD,
+// k, grows with the square root of the photons: the tail grows with
 // k, the rest falls with the issue slots that k waves fill.  Every SIMD gets
-// the same number of waves, as the launch waits for the fullest one.  On MI355X
-// with k = 1 to 6, 25 keV in 150 um, kernel ms (chosen k marked):
+// the same number of waves, as the launch waits for the fullest one.  lane_cap is
+// the power of two with which the planned waves can take all photons, so a wave
+// has up to twice the even share and some have none (33 photons per planned
+// wave: half the waves take 64), and above 32 per planned wave a launch uses all
+// lanes.  On MI355X with k = 1 to 6, 25 keV in 150 um (the only layer measured),
+// kernel ms (chosen k marked):
 //   2.7e5 photons   2.49 2.35* 2.40  2.62  2.65  2.63
 //   6.5e5           3.70 3.07* 3.13  3.54  3.93  4.17
 //   1.6e6           6.82 4.81  4.40* 4.57  4.79  5.15
@@ -236,7 +240,8 @@ __device__ __forceinline__ void counter_initial_dir(CounterRng& rng, Photon& p,
 #define FD2_WAVES_PER_EU 6
 #endif
 // With several geometries per launch (the geometry table in LDS, read per
-// lane, and a geometry index per photon) and with records the LDS holds 5.
+// lane, and a geometry index per photon) and with records the LDS holds 5 (4
+// from some 25 geometries on).
 #if FD2_WAVES_PER_EU > 0
 #define FD2_TRANSPORT_ATTR \
   __attribute__((amdgpu_waves_per_eu(MULTI || REC ? FD2_WAVES_PER_EU - 1 : FD2_WAVES_PER_EU, \
@@ -527,17 +532,17 @@ __device__ __forceinline__ uint32_t events_of(const unsigned long long* __restri
 // refill.
 //
 // Draining (no span, ready photon or backlog left), and throughout when
-// the queues are not used (tuning) or a launch has less than 64 photons per
-// wave, waiting photons stay in their lanes: the branch and the flights
-// run where they are, with the other lanes masked off, once at least as many
+// the queues are not used (tuning) or a launch has at most 32 photons per
+// planned wave (lane_cap < 64), waiting photons stay in their lanes: the branch
+// and the flights run where they are, with the other lanes masked off, once at least as many
 // wait as step (without queues: park_lanes).
 //
 // The loop's scalar work counts as much as its vector work: six waves share a
 // SIMD's issue slots.  So only a serve decides the mode and when the next serve
 // is due, a round without a phase does nothing else, and a lane mask is made
 // before the branch that uses it (made inside, it becomes a lane flag and a
-// mask again).  mono25x50 on MI355X: 103.7 -> 89.7 ms, 793 -> 719 vector and 365
-// -> 299 scalar instructions per photon, most of it spilled scalar registers.
+// mask again).  mono25x50 on MI355X: 103.7 -> 89.7 ms, 793 -> 711 vector and 365
+// -> 276 scalar instructions per photon, most of it spilled scalar registers.
 //
 // Every photon keeps its own state and random stream, so the results are the
 // same in either mode and in any order.

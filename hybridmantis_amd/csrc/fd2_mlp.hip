@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(256) k_forward_fused(const uint16_t* __restric
 // output gradients) and k_adam or k_sum_grads.  The layer-by-layer step
 // they replace took 14 launches of 5 to 19 us, with every layer's FP32
 // pre-activations and bf16 activations through HBM and FP32 atomics for the
-// split weight gradients: 217 us at batch 4096 on MI355X, now 36.6 us.
+// split weight gradients: 217 us at batch 4096 on MI355X, now 35 us.
 //
 // Operands in MFMA fragment order.  Forward weights: forward_slot, in wt.
 // Backward weights (W^T of layers 1..3, in wg at the same offsets): layers 1,
@@ -338,7 +338,8 @@ __device__ __forceinline__ uint2 pack4(uint16_t a, uint16_t b, uint16_t c, uint1
 // (128 KB per workgroup and layer) instead of its latency.  What is left is
 // the GELUs and their derivatives and the chain of 7 layers with their
 // barriers, which 4 waves per SIMD hide best: whole step at batch 4096 with
-// 8 and 16 waves 38.9 and 36.6 us.
+// 8 and 16 waves 38.9 and 36.6 us (35 us since, with the slices' sums loaded
+// eight at a time).
 // Arithmetic, rounding points and k order are the layered forward's and the
 // loss's own, so the rounded gradients are the same bits.
 constexpr int kTrainWaves = 16;
