@@ -34,3 +34,22 @@ def test_trained_equals_set(fd2lib, B, steps):
         assert loss == loss_n and np.array_equal(g, g_n)
         assert np.array_equal(net.logits(x), new.logits(x))
         assert np.array_equal(net.logits(x, layered=True), new.logits(x, layered=True))
+
+
+@pytest.mark.parametrize("B", [48, 1040])
+def test_gradients_leave_training_alone(fd2lib, B):
+    """A call for gradients changes nothing of the training that follows."""
+    rng = np.random.default_rng(B + 1)
+    x = rng.random((B, 5)).astype(np.float32)
+    y = np.zeros((B, 65), np.float32)
+    y[:, 0] = rng.uniform(0.05, 0.95, B)
+    y[:, 1:] = rng.dirichlet(np.ones(64) * 0.5, B)
+    runs = []
+    for ask in (False, True):
+        with fd2lib.Mlp(seed=B) as net:
+            net.set_data(x, y)
+            if ask:
+                net.gradients(x, y)
+            losses, _ = net.train(2, batch=B, lr=1e-3, seed=1)
+            runs.append((losses, net.params()))
+    assert np.array_equal(runs[0][0], runs[1][0]) and np.array_equal(runs[0][1], runs[1][1])
